@@ -232,11 +232,17 @@ void scan_excl_u32(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total,
 
 // ---------------------------------------------------------------------------
 // Stable LSD radix sort of (uint32 key, uint32 value), 8-bit digits.
-// Each workgroup ranks a tile of RS_TILE keys in RS_IPT rounds of RS_BS keys
-// (tile order is preserved: round-major, thread order inside a round),
-// places them in LDS in digit order, then writes each digit's keys as one
-// contiguous run at its global offset (coalesced, instead of one scattered
-// word per key).
+//
+// A workgroup of four waves sorts a tile of RS_BS * IPT keys.  Every wave
+// owns a contiguous IPT * 64 keys of it, held in registers (all loads in
+// flight together), and ranks them round by round against digit counters of
+// its own: the lanes that share a digit find each other with eight ballots,
+// the first of them adds their number to the counter.  No barrier is needed
+// until every key has its rank within its wave; then the waves' counters are
+// scanned, the keys are placed in LDS in digit order and each digit's keys
+// are written as one contiguous run.  (A form with the four waves in step,
+// four barriers and dependent loads in each of the 16 rounds, took 20 us for
+// a few tiles and 58 us for 6.2 M keys; this one 12 and 32 us.)
 // ---------------------------------------------------------------------------
 constexpr int RS_BS = 256, RS_IPT = 16, RS_TILE = RS_BS * RS_IPT, RS_NW = RS_BS / N2M_WAVE;
 
@@ -256,59 +262,80 @@ __device__ __forceinline__ RsTile rs_tile(const RsTile *__restrict__ desc, size_
 	return t;
 }
 
+// h[d] += 1 for every lane in `act`; the lanes that share the first active
+// lane's digit add once.  For leading digits, of which distances and Morton
+// keys have few: 64 lanes on one LDS counter take their turns.
+__device__ __forceinline__ void digit_add(uint32_t *h, uint32_t d, bool act)
+{
+	const unsigned long long m = __ballot(act);
+	if (!m)
+		return;
+	const int first = __ffsll((long long)m) - 1;
+	const uint32_t d0 = __shfl(d, first);
+	const unsigned long long same = __ballot(act && d == d0);
+	if (lane_id() == first)
+		atomicAdd(&h[d0], (uint32_t)__popcll(same));
+	if (act && d != d0)
+		atomicAdd(&h[d], 1u);
+}
+constexpr int RS_LEAD = 16; // shift from which a digit counts as leading
+
 __global__ void __launch_bounds__(RS_BS)
 k_radix_hist(const uint32_t *__restrict__ keys, size_t n, int shift, uint32_t *__restrict__ counts, size_t nblocks,
              const RsTile *__restrict__ desc)
 {
 	__shared__ uint32_t h[256];
-	h[threadIdx.x] = 0;
-	__syncthreads();
 	const RsTile t = rs_tile(desc, n, nblocks);
+	uint32_t key[RS_IPT];
+#pragma unroll
 	for (int k = 0; k < RS_IPT; k++) {
 		const uint32_t i = k * RS_BS + threadIdx.x;
-		if (i < t.len)
-			atomicAdd(&h[(keys[t.start + i] >> shift) & 0xFF], 1u);
+		key[k] = i < t.len ? keys[t.start + i] : 0u;
+	}
+	h[threadIdx.x] = 0;
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < RS_IPT; k++) {
+		const uint32_t d = (key[k] >> shift) & 0xFF;
+		const bool act = k * RS_BS + threadIdx.x < t.len;
+		if (shift >= RS_LEAD)
+			digit_add(h, d, act);
+		else if (act)
+			atomicAdd(&h[d], 1u);
 	}
 	__syncthreads();
 	counts[t.cbase + (size_t)threadIdx.x * t.cstride] = h[threadIdx.x];
 }
 
-__global__ void __launch_bounds__(RS_BS)
-k_radix_scatter(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, uint32_t *__restrict__ kout,
-                uint32_t *__restrict__ vout, size_t n, int shift, const uint32_t *__restrict__ offs, size_t nblocks,
-                const RsTile *__restrict__ desc)
+// The tile [base, base + tn) of one radix pass.  Thread t <-> digit t:
+// start() is called once by every thread while the keys are on their way and
+// returns where the tile's keys of that digit go; it may hold barriers.
+template <int IPT, typename Start>
+__device__ __forceinline__ void radix_tile(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin,
+                                           uint32_t *__restrict__ kout, uint32_t *__restrict__ vout, size_t base,
+                                           int tn, int shift, Start start)
 {
-	__shared__ uint32_t s_k[RS_TILE], s_v[RS_TILE];
-	__shared__ uint32_t run[256];  // keys of each digit placed so far
-	__shared__ uint32_t lofs[256]; // tile-local start of each digit
-	__shared__ uint32_t gbase[256];
-	__shared__ uint32_t wcnt[RS_NW][256];
+	__shared__ uint32_t s_k[RS_BS * IPT], s_v[RS_BS * IPT];
+	__shared__ uint32_t whist[RS_NW][256]; // keys of each digit, per wave; then their starts in the tile
+	__shared__ uint32_t dofs[256];         // output offset of a digit minus its start in the tile
 	__shared__ uint32_t scratch[RS_BS / N2M_WAVE + 1];
-	const RsTile t = rs_tile(desc, n, nblocks);
-	const size_t base = t.start;
-	const int tn = (int)t.len;
-	run[threadIdx.x] = 0;
-	gbase[threadIdx.x] = offs[t.cbase + (size_t)threadIdx.x * t.cstride];
-	for (int w = 0; w < RS_NW; w++)
-		wcnt[w][threadIdx.x] = 0;
-	__syncthreads();
-	for (int k = 0; k < RS_IPT; k++) {
-		const int i = k * RS_BS + threadIdx.x;
-		if (i < tn)
-			atomicAdd(&run[(kin[base + i] >> shift) & 0xFF], 1u);
+	const int lane = lane_id(), wv = wave_id(), w0 = wv * IPT * N2M_WAVE;
+	uint32_t key[IPT], val[IPT], rk[IPT];
+#pragma unroll
+	for (int k = 0; k < IPT; k++) {
+		const int i = w0 + k * N2M_WAVE + lane;
+		key[k] = i < tn ? kin[base + i] : 0u;
+		val[k] = i < tn ? vin[base + i] : 0u;
 	}
+#pragma unroll
+	for (int w = 0; w < RS_NW; w++)
+		whist[w][threadIdx.x] = 0;
+	const uint32_t st = start();
 	__syncthreads();
-	uint32_t tot;
-	lofs[threadIdx.x] = block_excl_scan<RS_BS>(run[threadIdx.x], scratch, &tot); // thread t <-> digit t
-	run[threadIdx.x] = 0;
-	__syncthreads();
-	const int lane = lane_id(), wv = wave_id();
-	const unsigned long long lt = (1ull << lane) - 1ull;
-	for (int k = 0; k < RS_IPT; k++) {
-		const int i = k * RS_BS + threadIdx.x;
-		const bool act = i < tn;
-		const uint32_t key = act ? kin[base + i] : 0u, val = act ? vin[base + i] : 0u;
-		const uint32_t d = (key >> shift) & 0xFF;
+#pragma unroll
+	for (int k = 0; k < IPT; k++) {
+		const bool act = w0 + k * N2M_WAVE + lane < tn;
+		const uint32_t d = (key[k] >> shift) & 0xFF;
 		unsigned long long m = __ballot(act);
 #pragma unroll
 		for (int b = 0; b < 8; b++) {
@@ -316,36 +343,155 @@ k_radix_scatter(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ v
 			const unsigned long long bb = __ballot(bit);
 			m &= bit ? bb : ~bb;
 		}
-		const uint32_t rk = __popcll(m & lt);
-		if (act && rk == 0)
-			wcnt[wv][d] = __popcll(m);
-		__syncthreads();
-		if (act) {
-			uint32_t pos = run[d] + rk;
-			for (int w = 0; w < wv; w++)
-				pos += wcnt[w][d];
-			s_k[lofs[d] + pos] = key;
-			s_v[lofs[d] + pos] = val;
-		}
-		__syncthreads();
-		uint32_t add = 0;
-		for (int w = 0; w < RS_NW; w++) {
-			add += wcnt[w][threadIdx.x];
-			wcnt[w][threadIdx.x] = 0;
-		}
-		run[threadIdx.x] += add;
-		__syncthreads();
+		const uint32_t below = lanes_below(m);
+		uint32_t before = 0;
+		if (act && below == 0)
+			before = atomicAdd(&whist[wv][d], (uint32_t)__popcll(m));
+		// from the first lane of the digit (inactive lanes read any lane)
+		rk[k] = __shfl(before, m ? __ffsll((long long)m) - 1 : 0) + below;
 	}
-	for (int i = threadIdx.x; i < tn; i += RS_BS) {
-		const uint32_t key = s_k[i], d = (key >> shift) & 0xFF;
-		const uint32_t o = gbase[d] + (uint32_t)(i - (int)lofs[d]);
-		kout[o] = key;
-		vout[o] = s_v[i];
+	__syncthreads();
+	uint32_t cnt[RS_NW], total = 0;
+#pragma unroll
+	for (int w = 0; w < RS_NW; w++) {
+		cnt[w] = whist[w][threadIdx.x];
+		total += cnt[w];
+	}
+	uint32_t all;
+	uint32_t run = block_excl_scan<RS_BS>(total, scratch, &all);
+	const uint32_t out = st - run;
+	dofs[threadIdx.x] = out;
+#pragma unroll
+	for (int w = 0; w < RS_NW; w++) {
+		whist[w][threadIdx.x] = run;
+		run += cnt[w];
+	}
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < IPT; k++) {
+		if (w0 + k * N2M_WAVE + lane < tn) {
+			const uint32_t pos = whist[wv][(key[k] >> shift) & 0xFF] + rk[k];
+			s_k[pos] = key[k];
+			s_v[pos] = val[k];
+		}
+	}
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < IPT; k++) {
+		const int i = k * RS_BS + threadIdx.x;
+		if (i < tn) {
+			const uint32_t ky = s_k[i];
+			const uint32_t o = dofs[(ky >> shift) & 0xFF] + (uint32_t)i;
+			kout[o] = ky;
+			vout[o] = s_v[i];
+		}
 	}
 }
 
+__global__ void __launch_bounds__(RS_BS)
+k_radix_scatter(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, uint32_t *__restrict__ kout,
+                uint32_t *__restrict__ vout, size_t n, int shift, const uint32_t *__restrict__ offs, size_t nblocks,
+                const RsTile *__restrict__ desc)
+{
+	const RsTile t = rs_tile(desc, n, nblocks);
+	radix_tile<RS_IPT>(
+	    kin, vin, kout, vout, t.start, (int)t.len, shift,
+	    [&] { return offs[t.cbase + (size_t)threadIdx.x * t.cstride]; });
+}
+
+// ---------------------------------------------------------------------------
+// Short sorts (at most RO_MAX_TILES tiles) are bound by launches and latency:
+// two launches per pass instead of three (the tiles' digit counts, tile by
+// tile; then the scatter, whose workgroups sum the counts themselves while
+// their keys are on their way), and as many tiles as that allows.  One pass
+// over 54 thousand keys went from 31 us to 12, over 240 thousand from 33 to
+// 16.  Measured and dropped: tiles that tell each other their counts inside one launch, as
+// in k_scan_1p (22 us at 118 tiles: the polls cross the XCDs), and counting
+// the next digit by global atomics while writing (33 us).
+// ---------------------------------------------------------------------------
+constexpr int RO_MAX_TILES = 128, RO_SMALL_IPT = 4;
+static_assert(RS_IPT == 4 * RO_SMALL_IPT, "radix_short picks among three tile sizes");
+
+// keys per thread of a short sort: the fewest whose tiles are at most
+// RO_MAX_TILES: more workgroups and fewer ranking rounds in a row outweigh
+// the longer sums of rows (240 thousand keys: 12.0 us with 118 tiles of 2048,
+// 14.5 us with 59 of 4096)
+static int ro_ipt(size_t n)
+{
+	int ipt = RO_SMALL_IPT;
+	while (ipt < RS_IPT && n > (size_t)RO_MAX_TILES * RS_BS * ipt)
+		ipt *= 2;
+	return ipt;
+}
+
+template <int IPT>
+__global__ void __launch_bounds__(RS_BS)
+k_radix_hist_rows(const uint32_t *__restrict__ keys, uint32_t n, int shift, uint32_t *__restrict__ counts)
+{
+	__shared__ uint32_t h[256];
+	const uint32_t base = blockIdx.x * (RS_BS * IPT) + threadIdx.x;
+	uint32_t key[IPT];
+#pragma unroll
+	for (int k = 0; k < IPT; k++)
+		key[k] = base + k * RS_BS < n ? keys[base + k * RS_BS] : 0u;
+	h[threadIdx.x] = 0;
+	__syncthreads();
+#pragma unroll
+	for (int k = 0; k < IPT; k++) {
+		const uint32_t d = (key[k] >> shift) & 0xFF;
+		const bool act = base + k * RS_BS < n;
+		if (shift >= RS_LEAD)
+			digit_add(h, d, act);
+		else if (act)
+			atomicAdd(&h[d], 1u);
+	}
+	__syncthreads();
+	counts[(size_t)blockIdx.x * 256 + threadIdx.x] = h[threadIdx.x];
+}
+
+template <int IPT>
+__global__ void __launch_bounds__(RS_BS)
+k_radix_scatter_rows(const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, uint32_t *__restrict__ kout,
+                     uint32_t *__restrict__ vout, uint32_t n, int shift, const uint4 *__restrict__ counts)
+{
+	constexpr uint32_t TILE = RS_BS * IPT;
+	__shared__ uint4 s_sum[RS_NW][64], s_before[RS_NW][64];
+	__shared__ uint32_t s_scan[RS_BS / N2M_WAVE + 1];
+	const uint32_t tile = blockIdx.x, nt = gridDim.x;
+	radix_tile<IPT>(kin, vin, kout, vout, (size_t)tile * TILE, (int)min(TILE, n - tile * TILE), shift, [&] {
+		// wave w sums every RS_NW-th row, four digits per lane
+		uint4 sum = make_uint4(0, 0, 0, 0), before = sum;
+		const int lane = lane_id(), w = wave_id();
+#pragma unroll 16
+		for (uint32_t j = w; j < nt; j += RS_NW) {
+			const uint4 x = counts[j * 64 + lane];
+			sum.x += x.x;
+			sum.y += x.y;
+			sum.z += x.z;
+			sum.w += x.w;
+			if (j < tile) {
+				before.x += x.x;
+				before.y += x.y;
+				before.z += x.z;
+				before.w += x.w;
+			}
+		}
+		s_sum[w][lane] = sum;
+		s_before[w][lane] = before;
+		__syncthreads();
+		uint32_t t = 0, b = 0;
+#pragma unroll
+		for (int k = 0; k < RS_NW; k++) {
+			t += reinterpret_cast<const uint32_t *>(s_sum[k])[threadIdx.x];
+			b += reinterpret_cast<const uint32_t *>(s_before[k])[threadIdx.x];
+		}
+		uint32_t all;
+		return b + block_excl_scan<RS_BS>(t, s_scan, &all);
+	});
+}
+
 // Sorts (k0,v0) using (k1,v1) as the ping-pong buffers; returns true when
-// the result is in (k1,v1).  counts/offs hold 256*nblocks words each.  With
+// the result is in (k1,v1).  counts holds 256*nblocks words.  With
 // tile descriptors (radix_seg_tiles) every segment is sorted on its own and
 // stays where it is: a segment's tiles count their digits in a region of
 // their own, laid out digit-major after the regions of the earlier segments,
@@ -366,12 +512,36 @@ static bool radix_passes(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1,
 	return flip;
 }
 
+// the short form (at most RO_MAX_TILES tiles of ro_ipt(n) keys per thread)
+template <int IPT>
+static bool radix_short(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, uint32_t n, int bits, uint32_t *counts,
+                        hipStream_t s)
+{
+	const uint32_t nt = (n + RS_BS * IPT - 1) / (RS_BS * IPT);
+	bool flip = false;
+	for (int shift = 0; shift < bits; shift += 8) {
+		const uint32_t *ki = flip ? k1 : k0, *vi = flip ? v1 : v0;
+		uint32_t *ko = flip ? k0 : k1, *vo = flip ? v0 : v1;
+		hipLaunchKernelGGL(k_radix_hist_rows<IPT>, dim3(nt), dim3(RS_BS), 0, s, ki, n, shift, counts);
+		hipLaunchKernelGGL(k_radix_scatter_rows<IPT>, dim3(nt), dim3(RS_BS), 0, s, ki, vi, ko, vo, n, shift,
+		                   (const uint4 *)counts);
+		flip = !flip;
+	}
+	return flip;
+}
+
 bool radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, size_t n, int bits,
                     uint32_t *counts, uint32_t *scan_scratch, hipStream_t s)
 {
 	if (n <= 1)
 		return false;
-	return radix_passes(k0, v0, k1, v1, n, bits, counts, scan_scratch, (n + RS_TILE - 1) / RS_TILE, nullptr, s);
+	const size_t nb = (n + RS_TILE - 1) / RS_TILE;
+	if (nb <= (size_t)RO_MAX_TILES) {
+		const int ipt = ro_ipt(n);
+		const auto f = ipt == 4 ? radix_short<4> : (ipt == 8 ? radix_short<8> : radix_short<16>);
+		return f(k0, v0, k1, v1, (uint32_t)n, bits, counts, s);
+	}
+	return radix_passes(k0, v0, k1, v1, n, bits, counts, scan_scratch, nb, nullptr, s);
 }
 
 std::vector<RsTile> radix_seg_tiles(const std::vector<uint32_t> &sb)
@@ -400,7 +570,13 @@ bool radix_sort_seg_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, 
 	return radix_passes(k0, v0, k1, v1, n, bits, counts, scan_scratch, ntiles, desc, s);
 }
 
-size_t radix_counts_words(size_t n) { return 256 * ((n + RS_TILE - 1) / RS_TILE) + 1; }
+// grows with n, so that a buffer for n keys serves every shorter sort
+size_t radix_counts_words(size_t n)
+{
+	const size_t nb = (n + RS_TILE - 1) / RS_TILE, w = 256 * nb + 1;
+	const size_t o = (size_t)256 * RO_MAX_TILES; // the rows of a short sort
+	return w > o ? w : o;
+}
 
 // ---------------------------------------------------------------------------
 // Vertex welding, src/meshify.c:45-106.  The reference sorts FP32 distances

@@ -122,6 +122,24 @@ def test_unify_scan_tile_boundaries(gpu, oracle, n):
     assert _eq(d1, d2)
 
 
+@pytest.mark.parametrize('n', [2, 64, 1024, 1025, 128 * 1024, 128 * 1024 + 1, 128 * 2048, 128 * 2048 + 1, 128 * 4096,
+                               128 * 4096 + 1])
+def test_unify_sort_tile_boundaries(gpu, oracle, n):
+    """Weld of n points at the sort's size boundaries: one and two 1024-key
+    tiles, 128 and one more of 1024, 2048 and 4096 keys (where the next
+    larger tile, and at last the long sort, takes over).  Class numbers
+    follow the sorted order, ties (equal distances of a 200^3 integer
+    lattice) in input order, so a misplaced key changes the result."""
+    import nii2mesh_amd.abi as abi
+    rng = np.random.default_rng(n)
+    pts = np.ascontiguousarray(rng.integers(0, 200, size=(n, 3)).astype(np.float64))
+    pts[n // 2] = pts[n // 3]  # at least one merge
+    tris = np.ascontiguousarray(rng.integers(0, n, size=(max(n // 4, 1), 3)), np.int32)
+    p1, t1 = abi.bind_unify(gpu.load(), 'n2m_unify_vertices')(pts, tris)
+    p2, t2 = oracle.unify(pts, tris)
+    assert len(p1) < n and _eq(p1, p2) and _eq(t1, t2)
+
+
 @pytest.mark.parametrize('first_nan', [False, True])
 def test_unify_nan_rows(gpu, oracle, first_nan):
     """Weld with vertices at NaN positions: each is a class of its own (its
