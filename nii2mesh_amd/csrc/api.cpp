@@ -18,6 +18,7 @@
 #include <functional>
 #include <limits>
 #include <condition_variable>
+#include <initializer_list>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -228,6 +229,7 @@ enum Slot {
 	S_Q_ERR,
 	S_PIPE_BITS,
 	S_WPOS,
+	S_APPLY,
 	S_COUNT
 };
 
@@ -244,10 +246,10 @@ struct Mesh {
 // small per-context scalars (device + pinned host mirror)
 enum Small {
 	SM_RANGE = 0,  // 2 words: ord min, ord max
-	SM_NROOTS = 2, // 1 word
+	SM_NROOTS = 2, // 1 word: background components (bubble fill)
+	SM_NROOTS2 = 3, // 1 word: foreground components
 	SM_BEST = 4,   // 2 words (u64)
-	SM_BBOX = 6,   // 6 words
-	SM_VMIN = 12,  // 1 word
+	SM_BBOX = 6,   // 9 words, host side only: box, minimum, range (launch_apply)
 	SM_TOTAL = 16, // 4 words of totals
 	SM_HSTAT = 24, // 3 words
 	SM_PBOX = 32,  // 6 words: float box of vertex positions
@@ -397,6 +399,18 @@ struct n2m_ctx {
 		memcpy(p, src, bytes);
 		return p;
 	}
+
+	// words of d_small from `off` set by one launch
+	void put(int off, std::initializer_list<uint32_t> v)
+	{
+		PutWords w;
+		int n = 0;
+		for (uint32_t x : v)
+			w.v[n++] = x;
+		launch_put(d_small + off, w, n, stream);
+	}
+	// the range words (empty), both component counts and the largest cluster
+	void put_volume() { put(SM_RANGE, {0xffffffffu, 0u, 0u, 0u, 0u, 0u}); }
 
 	// read `n` small words at offset `off` back to the host
 	uint32_t *fetch(int off, int n)
@@ -760,29 +774,36 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 	const int NX = dim[0], NY = dim[1], NZ = dim[2];
 	const size_t nvox = (size_t)NX * NY * NZ;
 	hipStream_t s = C->stream;
+	if (!have_range || known_range) // else the caller has, before the range was taken
+		C->put_volume();
 	if (!have_range && !known_range) {
-		uint32_t init[2] = {0xffffffffu, 0u};
-		HIPX(hipMemcpyAsync(C->d_small + SM_RANGE, init, sizeof init, hipMemcpyHostToDevice, s));
 		C->tbegin("minmax", 4.0 * nvox);
 		launch_minmax(in, nvox, C->d_small + SM_RANGE, s);
 		C->tend();
 	}
-	const uint32_t *r = known_range ? known_range : C->fetch(SM_RANGE, 2);
-	float mn = ord2f_host(r[0]), mx = ord2f_host(r[1]);
-	if (mn == mx) {
-		printf("Error: No variability in image intensity.\n");
-		return false;
-	}
-	float isolevel = P.isolevel;
+	// The range stays on the device unless the caller knows it or verbose
+	// prints it: the stages derive the isolevel and edge value from it as the
+	// host does (atlas_iso), and it comes back with the box.
+	const bool defer = !known_range && !P.verbose;
+	const uint32_t *drange = defer ? C->d_small + SM_RANGE : nullptr;
+	float isolevel = P.isolevel, mn = 0.f, edgeMax = 0.f;
 	bool iso_changed = false;
-	if ((isolevel <= mn) || (isolevel > mx)) { // src/meshify.c:316-319
-		isolevel = 0.5 * (mn + mx);
-		iso_changed = true;
-		printf("Suggested isolevel out of range. Intensity range %g..%g, setting isolevel to %g\n", mn, mx,
-		       isolevel);
-	}
-	if (P.verbose)
-		printf("intensity range %g..%g, isolevel %g\n", mn, mx, isolevel);
+	auto settle = [&](const uint32_t *r) { // src/meshify.c:312-319,347
+		mn = ord2f_host(r[0]);
+		const float mx = ord2f_host(r[1]);
+		if (!atlas_iso(P.isolevel, mn, mx, &isolevel, &edgeMax, &iso_changed)) {
+			printf("Error: No variability in image intensity.\n");
+			return false;
+		}
+		if (iso_changed)
+			printf("Suggested isolevel out of range. Intensity range %g..%g, setting isolevel to %g\n", mn, mx,
+			       isolevel);
+		if (P.verbose)
+			printf("intensity range %g..%g, isolevel %g\n", mn, mx, isolevel);
+		return true;
+	};
+	if (!defer && !settle(known_range ? known_range : C->fetch(SM_RANGE, 2)))
+		return false;
 	const int W = (NX + 31) / 32;
 	const size_t nwords = (size_t)W * NY * NZ;
 	uint32_t *keep = nullptr, *dil = nullptr;
@@ -792,9 +813,9 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 	const bool label_ok = NX >= 2 && NY >= 2 && NZ >= 1;
 	if (P.onlyLargest || P.fillBubbles) {
 		uint32_t *bits = spec_bits ? spec_bits : C->buf<uint32_t>(S_BITS, nwords);
-		if (!spec_bits || iso_changed) {
+		if (!spec_bits || iso_changed || defer) {
 			C->tbegin("mask_bits", 4.0 * nvox + nvox / 8.0);
-			launch_mask_bits(in, NX, NY, NZ, isolevel, 0, bits, s);
+			launch_mask_bits(in, NX, NY, NZ, isolevel, 0, bits, s, drange, spec_bits != nullptr);
 			C->tend();
 		}
 		keep = bits;
@@ -805,7 +826,6 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 			uint32_t *scr = scan_scratch(C, nwords + 1);
 			Timer tm(C);
 			if (P.fillBubbles) { // src/bwlabel.c:478-541
-				HIPX(hipMemsetAsync(C->d_small + SM_NROOTS, 0, 4, s));
 				launch_ccl(bits, NX, NY, NZ, 6, 1, L, AUX, 1, C->d_small + SM_NROOTS, nullptr, rbase, scr, s, &tm);
 				C->tbegin("fill_bubbles", 4.0 * nvox);
 				launch_fill_bubbles(bits, NX, NY, NZ, L, AUX, rbase, C->d_small + SM_NROOTS, s);
@@ -813,11 +833,9 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 			}
 			if (P.onlyLargest) { // src/bwlabel.c:453-471
 				uint32_t *roots = C->buf<uint32_t>(S_ROOTS, nvox / 2 + 1024);
-				HIPX(hipMemsetAsync(C->d_small + SM_NROOTS, 0, 4, s));
-				HIPX(hipMemsetAsync(C->d_small + SM_BEST, 0, 8, s));
-				launch_ccl(bits, NX, NY, NZ, 18, 0, L, AUX, 0, C->d_small + SM_NROOTS, roots, rbase, scr, s, &tm);
+				launch_ccl(bits, NX, NY, NZ, 18, 0, L, AUX, 0, C->d_small + SM_NROOTS2, roots, rbase, scr, s, &tm);
 				C->tbegin("ccl_argmax");
-				launch_ccl_argmax(roots, C->d_small + SM_NROOTS, AUX, (unsigned long long *)(C->d_small + SM_BEST), s);
+				launch_ccl_argmax(roots, C->d_small + SM_NROOTS2, AUX, (unsigned long long *)(C->d_small + SM_BEST), s);
 				C->tend();
 				uint32_t *sel = C->buf<uint32_t>(S_BITS2, nwords);
 				C->tbegin("select_root", 4.0 * nvox);
@@ -834,11 +852,6 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 		}
 	}
 	// apply + edge darken + bounding box, src/meshify.c:332-371
-	float edgeMax = 0.75 * (mn + isolevel);
-	int init[7] = {NX, NY, NZ, 0, 0, 0, 0};
-	uint32_t minit = 0xffffffffu;
-	HIPX(hipMemcpyAsync(C->d_small + SM_BBOX, init, 6 * sizeof(int), hipMemcpyHostToDevice, s));
-	HIPX(hipMemcpyAsync(C->d_small + SM_VMIN, &minit, 4, hipMemcpyHostToDevice, s));
 	uint32_t *sgp = nullptr, *sgn = nullptr;
 	if (P.cubes == N2M_CUBES_LEWINER) { // the sign bits the classify pass reads
 		const size_t sw = (size_t)((NX + 31) / 32) * NY * NZ;
@@ -846,13 +859,16 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 		sgn = C->buf<uint32_t>(S_SIGNN, sw);
 	}
 	C->tbegin("apply", 8.0 * nvox);
+	uint32_t *bb = C->h_small + SM_BBOX;
 	const bool signs = launch_apply(in, vol, NX, NY, NZ, isolevel, mn, edgeMax, P.fillBubbles ? keep : nullptr, dil,
-	                                P.fillBubbles ? 1 : 0, (int *)(C->d_small + SM_BBOX), C->d_small + SM_VMIN, s, sgp,
-	                                sgn);
+	                                P.fillBubbles ? 1 : 0, drange,
+	                                C->buf<uint32_t>(S_APPLY, apply_part_words()), bb, s, sgp, sgn);
 	C->tend();
 	out.sgp = signs ? sgp : nullptr;
 	out.sgn = signs ? sgn : nullptr;
-	uint32_t *bb = C->fetch(SM_BBOX, 7);
+	C->sync();
+	if (defer && !settle(bb + 7))
+		return false;
 	if ((P.onlyLargest || P.fillBubbles) && P.verbose)
 		printf("voxel clustering (largest cluster, bubbles): %ld ms\n", (long)round(now_ms() - t0));
 	int lo[3] = {(int)bb[0], (int)bb[1], (int)bb[2]}, hi[3] = {(int)bb[3], (int)bb[4], (int)bb[5]};
@@ -1207,8 +1223,7 @@ bool meshify_device(n2m_ctx *C, const float *src, float *vol, const int dim[3], 
 	uint32_t *spec = nullptr;
 	if (P.preSmooth && NX >= 5 && NY >= 5 && NZ >= 5) { // src/meshify.c:299-304
 		double t0 = now_ms();
-		uint32_t init[2] = {0xffffffffu, 0u};
-		HIPX(hipMemcpyAsync(C->d_small + SM_RANGE, init, sizeof init, hipMemcpyHostToDevice, s));
+		C->put_volume();
 		float *out = vol;
 		if (src == vol) // the stencil cannot run in place
 			out = C->buf<float>(S_VOL2, nvox);
@@ -1595,8 +1610,7 @@ void append_mesh(n2m_ctx *C, Mesh &U, const double *pts, uint32_t np, const int 
 // label count as the CLI finds it: trunc(max), src/nii2mesh.c:494-501
 int atlas_label_count(n2m_ctx *C, const float *labels, size_t nvox)
 {
-	uint32_t init[2] = {0xffffffffu, 0u};
-	HIPX(hipMemcpyAsync(C->d_small + SM_RANGE, init, sizeof init, hipMemcpyHostToDevice, C->stream));
+	C->put_volume();
 	launch_minmax(labels, nvox, C->d_small + SM_RANGE, C->stream);
 	C->check();
 	uint32_t *r = C->fetch(SM_RANGE, 2);
@@ -2831,8 +2845,7 @@ int n2m_ctx_pipeline(n2m_ctx *C, const float *d_img, const int dim[3], const n2m
 		                      : 0;
 		uint32_t *masks = nmask ? C->buf<uint32_t>(S_PIPE_BITS, nmask * nwords) : nullptr;
 		if (smoothed) {
-			uint32_t init[2] = {0xffffffffu, 0u};
-			HIPX(hipMemcpyAsync(C->d_small + SM_RANGE, init, sizeof init, hipMemcpyHostToDevice, s));
+			C->put_volume();
 			C->tbegin("smooth", 8.0 * nvox);
 			launch_smooth(d_img, sm, NX, NY, NZ, C->d_small + SM_RANGE, nullptr, 0, nullptr, s);
 			C->tend();
@@ -3498,8 +3511,7 @@ int marchingCubes(float *img, short dim[3], int lo[3], int hi[3], int originalMC
 		float vmin = 0.f;
 		int cubes = cubes_flavour();
 		if (cubes == N2M_CUBES_LEWINER) {
-			uint32_t init[2] = {0xffffffffu, 0u};
-			HIPX(hipMemcpyAsync(C->d_small + SM_RANGE, init, sizeof init, hipMemcpyHostToDevice, C->stream));
+			C->put_volume();
 			launch_minmax(vol, nvox, C->d_small + SM_RANGE, C->stream);
 			vmin = ord2f_host(C->fetch(SM_RANGE, 1)[0]);
 		}
@@ -3543,23 +3555,21 @@ int bwlabel(float *img, int conn, size_t dim[3], bool onlyLargest, bool fillBubb
 		float *vol = C->buf<float>(S_VOL, nvox);
 		HIPX(hipMemcpyAsync(vol, img, 4 * nvox, hipMemcpyHostToDevice, s));
 		uint32_t *bits = C->buf<uint32_t>(S_BITS, nwords);
+		C->put_volume();
 		launch_mask_bits(vol, NX, NY, NZ, 0.f, 1, bits, s);
 		uint32_t *L = C->buf<uint32_t>(S_L, nvox), *AUX = C->buf<uint32_t>(S_AUX, nvox);
 		uint32_t *roots = C->buf<uint32_t>(S_ROOTS, nvox / 2 + 1024);
 		uint32_t *rbase = C->buf<uint32_t>(S_RBASE, nwords + 1);
 		if (fillBubbles) { // src/bwlabel.c:478-541
-			HIPX(hipMemsetAsync(C->d_small + SM_NROOTS, 0, 4, s));
 			launch_ccl(bits, NX, NY, NZ, 6, 1, L, AUX, 1, C->d_small + SM_NROOTS, nullptr, rbase,
 			           scan_scratch(C, nwords + 1), s, nullptr);
 			launch_fill_bubbles(bits, NX, NY, NZ, L, AUX, rbase, C->d_small + SM_NROOTS, s);
 		}
-		HIPX(hipMemsetAsync(C->d_small + SM_NROOTS, 0, 4, s));
-		launch_ccl(bits, NX, NY, NZ, conn, 0, L, AUX, 0, C->d_small + SM_NROOTS, roots, rbase,
+		launch_ccl(bits, NX, NY, NZ, conn, 0, L, AUX, 0, C->d_small + SM_NROOTS2, roots, rbase,
 		           scan_scratch(C, nwords + 1), s, nullptr);
-		uint32_t nl = C->fetch(SM_NROOTS, 1)[0];
+		uint32_t nl = C->fetch(SM_NROOTS2, 1)[0];
 		if (nl > 0 && onlyLargest) { // src/bwlabel.c:453-471
-			HIPX(hipMemsetAsync(C->d_small + SM_BEST, 0, 8, s));
-			launch_ccl_argmax(roots, C->d_small + SM_NROOTS, AUX, (unsigned long long *)(C->d_small + SM_BEST), s);
+			launch_ccl_argmax(roots, C->d_small + SM_NROOTS2, AUX, (unsigned long long *)(C->d_small + SM_BEST), s);
 			uint32_t *sel = C->buf<uint32_t>(S_BITS2, nwords);
 			launch_select_root(bits, NX, NY, NZ, L, (unsigned long long *)(C->d_small + SM_BEST), sel, rbase, s);
 			launch_bits_to_float(sel, NX, NY, NZ, vol, s);

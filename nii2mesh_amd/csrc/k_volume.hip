@@ -197,12 +197,12 @@ struct ImgSrc {
 };
 
 __global__ void __launch_bounds__(SM_BS)
-k_smooth(const float *__restrict__ in, float *__restrict__ out, int nx, int ny, int nz,
+k_smooth(const float *__restrict__ in, float *__restrict__ out, int nx, int ny, int nz, int zc,
          uint32_t *__restrict__ range /* [0]=ord min, [1]=ord max */, IsoMasks iso,
          uint32_t *__restrict__ bits, int W)
 {
 	const int x0 = blockIdx.x * SM_TX, y0 = blockIdx.y * SM_TY;
-	const int z0 = blockIdx.z * SM_ZC, z1 = min(z0 + SM_ZC, nz);
+	const int z0 = blockIdx.z * zc, z1 = min(z0 + zc, nz);
 	float lmin = __builtin_inff(), lmax = -__builtin_inff();
 	ImgSrc src{in, nx, (size_t)nx * ny};
 	smooth_tile<SM_TX, SM_TY>(src, out, nx, ny, nz, x0, y0, z0, z1, iso, bits, W, lmin, lmax);
@@ -562,17 +562,46 @@ void launch_atlas_apply(float *crops, int gnx, int gny, int gnz, const AtlasTask
 		                   blockTask, nblocks, bbox, vmin);
 }
 
+// Planes per workgroup of the smoothing: SM_ZC, halved (down to SM_ZMIN) until
+// the launch has SM_WGS workgroups.  A workgroup's planes follow one
+// another (about 1.6 us each), so a small volume takes as long as its longest
+// chunk; each chunk reads 4 planes more than it writes, so a launch that
+// fills the chip keeps the long ones.  128^3: 61 us with 32 planes, 23 with
+// 4; 142 x 178 x 142: 69 and 39 (8 planes); 256^3: 92 and 90 (16 planes).
+constexpr int SM_ZMIN = 4;
+constexpr size_t SM_WGS = 2048;
+static int smooth_chunk(size_t columns, int nz)
+{
+	int zc = SM_ZC;
+	while (zc > SM_ZMIN && columns * ((nz + zc - 1) / zc) < SM_WGS)
+		zc /= 2;
+	return zc;
+}
+
 void launch_smooth(const float *in, float *out, int nx, int ny, int nz, uint32_t *range, const float *isos,
                    int nmask, uint32_t *bits, hipStream_t s)
 {
-	dim3 grid((nx + SM_TX - 1) / SM_TX, (ny + SM_TY - 1) / SM_TY, (nz + SM_ZC - 1) / SM_ZC);
+	dim3 grid((nx + SM_TX - 1) / SM_TX, (ny + SM_TY - 1) / SM_TY, 1);
+	const int zc = smooth_chunk((size_t)grid.x * grid.y, nz);
+	grid.z = (nz + zc - 1) / zc;
 	int W = (nx + 31) / 32;
 	IsoMasks m{};
 	m.n = bits ? (nmask < N2M_SMOOTH_MASKS ? nmask : N2M_SMOOTH_MASKS) : 0;
 	for (int k = 0; k < m.n; k++)
 		m.v[k] = isos[k];
 	m.nwords = (size_t)W * ny * nz;
-	hipLaunchKernelGGL(k_smooth, grid, dim3(SM_BS), 0, s, in, out, nx, ny, nz, range, m, bits, W);
+	hipLaunchKernelGGL(k_smooth, grid, dim3(SM_BS), 0, s, in, out, nx, ny, nz, zc, range, m, bits, W);
+}
+
+__global__ void k_put(uint32_t *__restrict__ dst, PutWords w, int n)
+{
+	if ((int)threadIdx.x < n)
+		dst[threadIdx.x] = w.v[threadIdx.x];
+}
+
+void launch_put(uint32_t *dst, const PutWords &w, int n, hipStream_t s)
+{
+	hipLaunchKernelGGL(k_put, dim3(1), dim3(64), 0, s, dst, w, n);
 }
 
 // ---------------------------------------------------------------------------
@@ -628,10 +657,22 @@ void launch_minmax(const float *img, size_t n, uint32_t *range, hipStream_t s)
 // A workgroup walks whole rows (the row index is uniform, so no per-voxel
 // division); one wave covers 64 consecutive x of a row, padded to 64.
 // ---------------------------------------------------------------------------
+// the isolevel of a mask (launch_mask_bits); false: the mask stays
+__device__ __forceinline__ bool mask_iso(const uint32_t *range, int only_moved, float &iso)
+{
+	if (!range)
+		return true;
+	float edgeMax;
+	bool moved = false;
+	return atlas_iso(iso, ord2f(range[0]), ord2f(range[1]), &iso, &edgeMax, &moved) && (moved || !only_moved);
+}
+
 __global__ void __launch_bounds__(256)
 k_mask_bits(const float *__restrict__ img, int nx, int ny, int nz, int W, int xpad, float iso,
-            int nonzero, uint32_t *__restrict__ bits)
+            int nonzero, uint32_t *__restrict__ bits, const uint32_t *__restrict__ range, int only_moved)
 {
+	if (!mask_iso(range, only_moved, iso))
+		return;
 	const size_t rows = (size_t)ny * nz;
 	for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
 		const float *src = img + row * nx;
@@ -661,8 +702,10 @@ k_mask_bits(const float *__restrict__ img, int nx, int ny, int nz, int W, int xp
 // neighbouring lanes OR their nibbles into a word.
 __global__ void __launch_bounds__(256)
 k_mask_bits4(const float *__restrict__ img, int nx, int ny, int nz, int W, float iso, int nonzero,
-             uint32_t *__restrict__ bits)
+             uint32_t *__restrict__ bits, const uint32_t *__restrict__ range, int only_moved)
 {
+	if (!mask_iso(range, only_moved, iso))
+		return;
 	const size_t rows = (size_t)ny * nz;
 	const int lpr = nx >> 2, span = lpr < (int)blockDim.x ? lpr : (int)blockDim.x;
 	const int rpi = (int)blockDim.x / span, sub = threadIdx.x / span, q0 = threadIdx.x % span;
@@ -744,18 +787,18 @@ void launch_mask_bits_multi(const float *img, int nx, int ny, int nz, const floa
 }
 
 void launch_mask_bits(const float *img, int nx, int ny, int nz, float iso, int nonzero, uint32_t *bits,
-                      hipStream_t s)
+                      hipStream_t s, const uint32_t *range, bool only_moved)
 {
 	int W = (nx + 31) / 32, xpad = (nx + 63) / 64 * 64;
 	const int lpr = nx / 4;
 	if (nx % 32 == 0 && (reinterpret_cast<uintptr_t>(img) & 15u) == 0 && (lpr <= 256 || lpr % 256 == 0)) {
 		const size_t rows = (size_t)ny * nz, rpi = lpr < 256 ? 256 / lpr : 1;
 		hipLaunchKernelGGL(k_mask_bits4, dim3(row_blocks((rows + rpi - 1) / rpi)), dim3(256), 0, s, img, nx, ny,
-		                   nz, W, iso, nonzero, bits);
+		                   nz, W, iso, nonzero, bits, range, only_moved ? 1 : 0);
 		return;
 	}
 	hipLaunchKernelGGL(k_mask_bits, dim3(row_blocks((size_t)ny * nz)), dim3(256), 0, s, img, nx, ny, nz, W, xpad,
-	                   iso, nonzero, bits);
+	                   iso, nonzero, bits, range, only_moved ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -821,15 +864,29 @@ void launch_dilate_bits(const uint32_t *in, uint32_t *out, int nx, int ny, int n
 // outside the dilated largest cluster to mn, record the bounding box of
 // voxels >= iso, then clamp the outer faces to edgeMax.
 // keep: mask after bwlabel (fill target); dil: dilated mask (or null).
-// bbox: int[6] = {minx,miny,minz,maxx,maxy,maxz}.
+// The box is {minx,miny,minz,maxx,maxy,maxz}.
 // ---------------------------------------------------------------------------
+// Box and minimum are reduced through one row of partial results per
+// workgroup and a one-workgroup launch, which hands them to the host by
+// itself: with atomics on one line from every workgroup this pass took
+// 40 us on a 128^3 volume (8 MiB) and 97 on a 256^3 one; now 7 and 37, and
+// 5.6 for the small launch, which takes the place of a copy.
+constexpr int AP_WORDS = 7, AP_MAXWG = 1024;
+
 __global__ void __launch_bounds__(256)
 k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, float iso, float mn,
         float edgeMax, const uint32_t *__restrict__ keep, const uint32_t *__restrict__ dil, int fill,
-        int *__restrict__ bbox, uint32_t *__restrict__ vmin, uint32_t *__restrict__ sgp, uint32_t *__restrict__ sgn)
+        const uint32_t *__restrict__ range, uint32_t *__restrict__ part, uint32_t *__restrict__ sgp,
+        uint32_t *__restrict__ sgn)
 {
 	__shared__ int s_red[6][4];
 	__shared__ uint32_t s_min[4];
+	if (range) {
+		bool moved;
+		mn = ord2f(range[0]);
+		if (!atlas_iso(iso, mn, ord2f(range[1]), &iso, &edgeMax, &moved))
+			return;
+	}
 	float lmin = __builtin_inff();
 	int bmin[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff}, bmax[3] = {-1, -1, -1};
 	const size_t rows = (size_t)ny * nz;
@@ -937,21 +994,48 @@ k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, f
 		int r = s_red[k][0];
 		for (int w = 1; w < 4; w++)
 			r = k < 3 ? min(r, s_red[k][w]) : max(r, s_red[k][w]);
-		// a plain read first: most workgroups cannot improve the box
-		const int cur = (int)ld_agent((const uint32_t *)&bbox[k]);
-		if (k < 3) {
-			if (r != 0x7fffffff && r < cur)
-				atomicMin(&bbox[k], r);
-		} else if (r >= 0 && r > cur) {
-			atomicMax(&bbox[k], r);
-		}
+		part[k * AP_MAXWG + blockIdx.x] = (uint32_t)r;
 	}
-	if (threadIdx.x == 6) {
-		uint32_t m = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
-		if (m < ld_agent(vmin))
-			atomicMin(vmin, m);
+	if (threadIdx.x == 6)
+		part[6 * AP_MAXWG + blockIdx.x] = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
+}
+
+// the workgroups' partial boxes and minima to host[0..6], the range to
+// host[7..8]; a box without voxels keeps the reference's start values
+// (src/meshify.c:349-351)
+__global__ void __launch_bounds__(AP_MAXWG)
+k_apply_box(const uint32_t *__restrict__ part, int nwg, int nx, int ny, int nz, const uint32_t *__restrict__ range,
+            uint32_t *__restrict__ host)
+{
+	__shared__ uint32_t s[AP_WORDS][AP_MAXWG / N2M_WAVE];
+	const bool in = (int)threadIdx.x < nwg; // (left over from another call when k_apply found no variability)
+	const int dim[3] = {nx, ny, nz};
+#pragma unroll
+	for (int k = 0; k < AP_WORDS; k++) {
+		const uint32_t v = in ? part[k * AP_MAXWG + threadIdx.x] : (k < 3 ? 0x7fffffffu : 0xffffffffu);
+		const uint32_t r = k < 3 ? (uint32_t)wave_min_i32((int)v) : (k < 6 ? (uint32_t)wave_max_i32((int)v)
+		                                                                  : wave_min_u32(v));
+		if (lane_id() == 0)
+			s[k][wave_id()] = r;
+	}
+	__syncthreads();
+	const int k = threadIdx.x;
+	if (k < AP_WORDS) {
+		uint32_t r = s[k][0];
+		for (int w = 1; w < AP_MAXWG / N2M_WAVE; w++)
+			r = k < 3 ? (uint32_t)min((int)r, (int)s[k][w])
+			          : (k < 6 ? (uint32_t)max((int)r, (int)s[k][w]) : min(r, s[k][w]));
+		if (k < 3)
+			r = (uint32_t)min((int)r, dim[k]);
+		else if (k < 6)
+			r = (uint32_t)max((int)r, 0);
+		host[k] = r;
+	} else if (k < AP_WORDS + 2 && range) {
+		host[k] = range[k - AP_WORDS];
 	}
 }
+
+size_t apply_part_words() { return (size_t)AP_WORDS * AP_MAXWG; }
 
 bool apply_sign_bits_ok(const float *src, const float *img, int nx)
 {
@@ -960,8 +1044,8 @@ bool apply_sign_bits_ok(const float *src, const float *img, int nx)
 }
 
 bool launch_apply(const float *src, float *img, int nx, int ny, int nz, float iso, float mn, float edgeMax,
-                  const uint32_t *keep, const uint32_t *dil, int fill, int *bbox, uint32_t *vmin, hipStream_t s,
-                  uint32_t *sgp, uint32_t *sgn)
+                  const uint32_t *keep, const uint32_t *dil, int fill, const uint32_t *range, uint32_t *part,
+                  uint32_t *host, hipStream_t s, uint32_t *sgp, uint32_t *sgn)
 {
 	const int W = (nx + 31) / 32;
 	const float *in = src ? src : img;
@@ -970,8 +1054,12 @@ bool launch_apply(const float *src, float *img, int nx, int ny, int nz, float is
 		sgp = sgn = nullptr;
 	const size_t rows = (size_t)ny * nz;
 	const size_t rpi = vec4 && nx / 4 < 256 ? 256 / (nx / 4) : 1;
-	hipLaunchKernelGGL(k_apply, dim3(row_blocks((rows + rpi - 1) / rpi)), dim3(256), 0, s, in, img, nx, ny, nz, W,
-	                   vec4 ? 1 : 0, iso, mn, edgeMax, keep, dil, fill, bbox, vmin, sgp, sgn);
+	const size_t items = (rows + rpi - 1) / rpi;
+	const unsigned nwg = (unsigned)(items < (size_t)AP_MAXWG ? (items ? items : 1) : (size_t)AP_MAXWG);
+	hipLaunchKernelGGL(k_apply, dim3(nwg), dim3(256), 0, s, in, img, nx, ny, nz, W, vec4 ? 1 : 0, iso, mn, edgeMax,
+	                   keep, dil, fill, range, part, sgp, sgn);
+	hipLaunchKernelGGL(k_apply_box, dim3(1), dim3(AP_MAXWG), 0, s, (const uint32_t *)part, (int)nwg, nx, ny, nz,
+	                   range, host);
 	return sgp != nullptr;
 }
 

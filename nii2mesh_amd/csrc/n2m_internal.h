@@ -65,6 +65,13 @@ struct AdjGeo {
 	float iso, mnv;
 };
 
+// up to 64 words passed by value: launch_put writes the first n to dst (one
+// launch instead of a pageable copy or a memset per group of words)
+struct PutWords {
+	uint32_t v[64];
+};
+void launch_put(uint32_t *dst, const PutWords &w, int n, hipStream_t s);
+
 struct CclTimer {
 	virtual void begin(const char *name, double bytes) = 0;
 	virtual void end() = 0;
@@ -83,16 +90,25 @@ void launch_mask_bits_multi(const float *img, int nx, int ny, int nz, const floa
 void launch_smooth(const float *in, float *out, int nx, int ny, int nz, uint32_t *range, const float *isos,
                    int nmask, uint32_t *bits, hipStream_t s);
 void launch_minmax(const float *img, size_t n, uint32_t *range, hipStream_t s);
+// range (when given): the ordered min / max words of img on the device; the
+// isolevel is then what meshify() takes for `iso` in that range, and with
+// only_moved the mask is written only when that is another value
 void launch_mask_bits(const float *img, int nx, int ny, int nz, float iso, int nonzero, uint32_t *bits,
-                      hipStream_t s);
+                      hipStream_t s, const uint32_t *range = nullptr, bool only_moved = false);
 void launch_dilate_bits(const uint32_t *in, uint32_t *out, int nx, int ny, int nz, hipStream_t s);
-// img = apply(src) (src null: in place); every voxel of img is written
+// img = apply(src) (src null: in place); every voxel of img is written.
+// range (when given): the ordered min / max words of the input on the device,
+// from which mn, edgeMax and the isolevel meshify() takes for `iso` follow
+// (atlas_iso); without variability nothing is written at all.  part: apply_part_words()
+// words of scratch.  host: 9 words the device can write (pinned): box, ordered
+// minimum of the result, and the range words (when given).
 // sgp / sgn (when given and nx % 32 == 0 with 16-byte aligned volumes):
 // the Lewiner sign bits of the result, lw_clamp(v - iso) > 0 / < 0, ceil(nx
 // / 32) words per row; returns whether they were written
 bool launch_apply(const float *src, float *img, int nx, int ny, int nz, float iso, float mn, float edgeMax,
-                  const uint32_t *keep, const uint32_t *dil, int fill, int *bbox, uint32_t *vmin, hipStream_t s,
-                  uint32_t *sgp = nullptr, uint32_t *sgn = nullptr);
+                  const uint32_t *keep, const uint32_t *dil, int fill, const uint32_t *range, uint32_t *part,
+                  uint32_t *host, hipStream_t s, uint32_t *sgp = nullptr, uint32_t *sgn = nullptr);
+size_t apply_part_words();
 void launch_hist_range(const float *img, size_t n, uint32_t *stats, hipStream_t s);
 // mesh output encoding (k_encode.hip)
 void launch_f64_to_f32(const double *in, size_t n, float *out, hipStream_t s);

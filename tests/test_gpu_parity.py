@@ -32,6 +32,17 @@ def test_quick_smooth(gpu, oracle, shape, seed):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
+@pytest.mark.parametrize('shape', [(33, 1024, 250), (64, 1024, 250), (70, 2048, 250)])
+def test_quick_smooth_chunks(gpu, oracle, shape):
+    """The smoothing with 8, 16 and 32 planes per workgroup (the smaller
+    volumes above take 4)."""
+    rng = np.random.default_rng(shape[0])
+    a = rng.standard_normal(shape, dtype=np.float32)
+    b = a.copy()
+    assert gpu.load().n2m_quick_smooth(a, shape[2], shape[1], shape[0]) == oracle.quick_smooth(b)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 @pytest.mark.parametrize('shape', [(13, 17, 19), (40, 33, 70), (1, 9, 9), (3, 2, 40)])
 @pytest.mark.parametrize('p', [0.3, 0.55, 0.75])
 @pytest.mark.parametrize('conn', [6, 18, 26])
