@@ -7,8 +7,8 @@
 // order and the largest-cluster tie rule (lowest label wins,
 // src/bwlabel.c:463) is "smallest root wins".
 //
-//  1. k_ccl_local: a workgroup labels the runs of a 512x4x4 tile in LDS
-//     (16 bit words per tile row) and writes each run's tile-local root to
+//  1. k_ccl_local: a workgroup labels the runs of a tile of 256 words (128x8x8
+//     voxels) in LDS and writes each run's tile-local root to
 //     L; it also clears AUX at every tile-local root (every global root is
 //     one of them).
 //  2. k_ccl_merge: tile-boundary voxels union with their backward neighbours
@@ -24,7 +24,14 @@
 
 namespace n2m {
 
-constexpr int CC_KW = 16, CC_TY = 4, CC_TZ = 4, CC_BS = CC_KW * CC_TY * CC_TZ; // 256
+// A tile of CC_BS words: CC_KW words of CC_TY rows and CC_TZ slices (template
+// parameters of the passes below).  Few of a compact tile's rows face another
+// tile, and short rows leave no thread without a word (a 512 x 4 x 4 tile on
+// rows of 128 voxels left three in four).  The four passes on a solid mask:
+// 128^3 68 us with 512 x 4 x 4, 46 with 128 x 8 x 8; 256^3 165 us, 128 x 8 x 8
+// 148 (its two tiles per row lengthen the chains of the merge), 256 x 8 x 4
+// 110; 512^3 within 2 % (noisy masks).
+constexpr int CC_BS = 256;
 constexpr uint32_t NONE = 0xffffffffu;
 
 // Run-based labelling.  A row word is split into maximal runs of set bits
@@ -121,11 +128,26 @@ __device__ __forceinline__ uint32_t lds_find(const uint32_t *lab, uint32_t x)
 	return x;
 }
 
+// the same while unions are in flight, every node on the way pointed at its
+// grandparent (an ancestor; only roots are hooked, as in uf_find_live)
+__device__ __forceinline__ uint32_t lds_find_live(uint32_t *lab, uint32_t x)
+{
+	uint32_t p = __hip_atomic_load(&lab[x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+	while (p != x) {
+		const uint32_t gp = __hip_atomic_load(&lab[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+		if (gp != p)
+			__hip_atomic_store(&lab[x], gp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+		x = p;
+		p = gp;
+	}
+	return x;
+}
+
 __device__ __forceinline__ void lds_union(uint32_t *lab, uint32_t a, uint32_t b)
 {
 	for (;;) {
-		a = lds_find(lab, a);
-		b = lds_find(lab, b);
+		a = lds_find_live(lab, a);
+		b = lds_find_live(lab, b);
 		if (a == b)
 			return;
 		if (a < b) {
@@ -140,28 +162,22 @@ __device__ __forceinline__ void lds_union(uint32_t *lab, uint32_t a, uint32_t b)
 	}
 }
 
-// Visit every (run of w, run of u) pair connected by the x shift dx
-// (u is the neighbour row word at the same word index; up / un are the
-// neighbour row words at word index -1 / +1, used for the bit that crosses
-// the word boundary).  f(bit_in_w, word_offset_of_u, bit_in_u).
+// Visit every run of a neighbour row that the run rm (a mask of its word's
+// bits) is connected to, once each: u is the neighbour row's word at the same
+// word index, up / un those before and after it, and the x shifts go from
+// nb.dxlo to nb.dxhi.  f(word_offset, bit of the neighbour's run).  (One visit
+// per shift instead of per run had up to three links for one.)
 template <typename F>
-__device__ __forceinline__ void for_links(uint32_t w, uint32_t u, uint32_t up, uint32_t un, int dx, F f)
+__device__ __forceinline__ void run_links(uint32_t rm, uint32_t u, uint32_t up, uint32_t un, const NbrRow &nb, F f)
 {
-	uint32_t m;
-	if (dx == 0)
-		m = w & u;
-	else if (dx < 0)
-		m = w & (u << 1); // bit b of w touches bit b-1 of u
-	else
-		m = w & (u >> 1); // bit b of w touches bit b+1 of u
-	for (uint32_t sg = m & ~(m << 1); sg; sg &= sg - 1) {
-		int b = __ffs(sg) - 1;
-		f(b, 0, b + dx);
-	}
-	if (dx < 0 && (w & 1u) && (up >> 31))
-		f(0, -1, 31);
-	if (dx > 0 && (w >> 31) && (un & 1u))
-		f(31, 1, 0);
+	const bool lo = nb.dxlo < 0, hi = nb.dxhi > 0;
+	const uint32_t m = (rm | (lo ? rm >> 1 : 0u) | (hi ? rm << 1 : 0u)) & u;
+	for (uint32_t sg = m & ~(m << 1); sg; sg &= sg - 1)
+		f(0, __ffs(sg) - 1);
+	if (lo && (rm & 1u) && (up >> 31))
+		f(-1, 31);
+	if (hi && (rm >> 31) && (un & 1u))
+		f(1, 0);
 }
 
 // per word: the number of runs (starts) of the predicate; cnt[nw] = 0, so
@@ -181,7 +197,7 @@ k_run_count(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__re
 	cnt[t] = c;
 }
 
-// Pass 1: label runs inside a tile of 16 words x 4 rows x 4 slices in LDS.
+// Pass 1: label runs inside a tile in LDS.
 // A run's tile-local node is its rank among the tile's runs in (slice, row,
 // word, bit) order -- the order of their global ids -- so the smallest node
 // of a tile component is its smallest run id.  A tile holds at most
@@ -192,9 +208,9 @@ k_run_count(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__re
 constexpr int CC_RUNS = CC_BS * 16;
 constexpr uint32_t TILE_ROOT = 0x80000000u;
 static_assert((uint32_t)CC_RUNS <= (1u << LAB_BITS), "node ids fit the label bits");
-static_assert((uint64_t)CC_KW * 32 * CC_TY * CC_TZ < (1ull << (31 - LAB_BITS)), "tile counts fit above them");
+static_assert((uint64_t)CC_BS * 32 < (1ull << (31 - LAB_BITS)), "tile counts fit above them");
 
-// word of the tile (flat index r * CC_KW + k) holding tile-local run `node`:
+// word of the tile (flat index, thread order) holding tile-local run `node`:
 // the last word whose first run is at or before it
 __device__ __forceinline__ int tile_word_of(const uint32_t *pre, uint32_t node)
 {
@@ -209,6 +225,7 @@ __device__ __forceinline__ int tile_word_of(const uint32_t *pre, uint32_t node)
 	return lo;
 }
 
+template <int CC_KW, int CC_TY, int CC_TZ>
 __global__ void __launch_bounds__(CC_BS)
 k_ccl_local(const uint32_t *__restrict__ bits, Geo g, int conn, int invert, uint32_t *__restrict__ L,
             uint32_t *__restrict__ AUX, int mode)
@@ -228,26 +245,48 @@ k_ccl_local(const uint32_t *__restrict__ bits, Geo g, int conn, int invert, uint
 	uint32_t tot;
 	const uint32_t pre = block_excl_scan<CC_BS>(__popc(st), scratch, &tot); // thread order = (r, k)
 	s_pre[r][k] = pre;
-	for (uint32_t j = 0, n = __popc(st); j < n; j++)
-		lab[pre + j] = pre + j;
 	__syncthreads();
-	// x-1 across the word boundary inside the tile
-	if (k > 0 && (w & 1u) && (s_w[r][k - 1] >> 31))
-		lds_union(lab, pre, s_pre[r][k - 1] + run_index(run_starts(s_w[r][k - 1]), 31));
 	int nn;
 	const NbrRow *nb = nbr_rows(conn, &nn);
-	for (int i = 0; i < nn; i++) {
-		const int ny2 = ry + nb[i].dy, nz2 = rz + nb[i].dz;
-		if (ny2 < 0 || ny2 >= CC_TY || nz2 < 0 || nz2 >= CC_TZ)
-			continue; // another tile: merge pass
-		const int r2 = ny2 + CC_TY * nz2;
-		const uint32_t u = s_w[r2][k];
-		const uint32_t up = k > 0 ? s_w[r2][k - 1] : 0u, un = k + 1 < CC_KW ? s_w[r2][k + 1] : 0u;
-		for (int dx = nb[i].dxlo; dx <= nb[i].dxhi; dx++)
-			for_links(w, u, up, un, dx, [&](int bw, int wo, int bu) {
-				uint32_t uw = wo == 0 ? u : (wo < 0 ? up : un);
-				lds_union(lab, pre + run_index(st, bw), s_pre[r2][k + wo] + run_index(run_starts(uw), bu));
+	// Every run of the tile's own rows next to this one, in a fixed order:
+	// f(node) for each link of the run rm.
+	auto links = [&](uint32_t rm, auto f) {
+		if (k > 0 && (rm & 1u) && (s_w[r][k - 1] >> 31)) // x-1 across the word boundary
+			f(pre - 1u); // the last run of the word before
+		for (int i = 0; i < nn; i++) {
+			const int ny2 = ry + nb[i].dy, nz2 = rz + nb[i].dz;
+			if (ny2 < 0 || ny2 >= CC_TY || nz2 < 0 || nz2 >= CC_TZ)
+				continue; // another tile: merge pass
+			const int r2 = ny2 + CC_TY * nz2;
+			const uint32_t u = s_w[r2][k];
+			const uint32_t up = k > 0 ? s_w[r2][k - 1] : 0u, un = k + 1 < CC_KW ? s_w[r2][k + 1] : 0u;
+			run_links(rm, u, up, un, nb[i], [&](int wo, int bu) {
+				const uint32_t uw = wo == 0 ? u : (wo < 0 ? up : un);
+				f(s_pre[r2][k + wo] + run_index(run_starts(uw), bu));
 			});
+		}
+	};
+	// Each run starts under its first neighbour (a smaller node: every link
+	// goes backwards), by plain stores; only the links after it are unions.
+	{
+		uint32_t j = 0;
+		for (uint32_t t = st; t; t &= t - 1, j++) {
+			uint32_t first = NONE;
+			links(run_mask(w, __ffs(t) - 1), [&](uint32_t node) { first = first == NONE ? node : first; });
+			lab[pre + j] = first == NONE ? pre + j : first;
+		}
+	}
+	__syncthreads();
+	{
+		uint32_t j = 0;
+		for (uint32_t t = st; t; t &= t - 1, j++) {
+			bool first = true;
+			links(run_mask(w, __ffs(t) - 1), [&](uint32_t node) {
+				if (!first)
+					lds_union(lab, pre + j, node);
+				first = false;
+			});
+		}
 	}
 	__syncthreads();
 	if (mode == 0) { // voxel count of each tile component, at its root
@@ -276,9 +315,15 @@ k_ccl_local(const uint32_t *__restrict__ bits, Geo g, int conn, int invert, uint
 // hash set; a pair already there is skipped.
 constexpr int CC_SEEN = 512;
 
+__device__ __forceinline__ uint32_t ld_group(const uint32_t *p)
+{
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 __device__ __forceinline__ void ccl_link(uint32_t *L, unsigned long long *seen, uint32_t a, uint32_t b)
 {
-	uint32_t pa = ld_agent(&L[a]), pb = ld_agent(&L[b]);
+	// plain loads: a parent seen late is an ancestor all the same
+	uint32_t pa = ld_group(&L[a]), pb = ld_group(&L[b]);
 	if (pa == pb)
 		return;
 	if (pa > pb) {
@@ -299,6 +344,7 @@ __device__ __forceinline__ void ccl_link(uint32_t *L, unsigned long long *seen, 
 	uf_union(L, pa, pb);
 }
 
+template <int CC_KW, int CC_TY, int CC_TZ>
 __global__ void __launch_bounds__(CC_BS)
 k_ccl_merge(const uint32_t *__restrict__ bits, Geo g, int conn, int invert, uint32_t *__restrict__ L)
 {
@@ -333,17 +379,17 @@ k_ccl_merge(const uint32_t *__restrict__ bits, Geo g, int conn, int invert, uint
 		// neighbouring words of the tile's first and last word
 		if (!other_tile_row && k != 0 && k != CC_KW - 1)
 			continue;
-		const uint32_t u = g.word(bits, wx, y2, z2, invert);
-		const uint32_t up = g.word(bits, wx - 1, y2, z2, invert), un = g.word(bits, wx + 1, y2, z2, invert);
-		for (int dx = nb[i].dxlo; dx <= nb[i].dxhi; dx++)
-			for_links(w, u, up, un, dx, [&](int bw, int wo, int bu) {
-				// same tile unless the row or the word lies outside it
-				bool other = other_tile_row || (wo < 0 && k == 0) || (wo > 0 && k == CC_KW - 1);
-				if (!other)
-					return;
-				uint32_t uw = wo == 0 ? u : (wo < 0 ? up : un);
-				ccl_link(L, s_seen, rb0 + run_index(st, bw),
-				         g.rb[g.widx(wx + wo, y2, z2)] + run_index(run_starts(uw), bu));
+		const uint32_t u = other_tile_row ? g.word(bits, wx, y2, z2, invert) : 0u;
+		const uint32_t up = other_tile_row || k == 0 ? g.word(bits, wx - 1, y2, z2, invert) : 0u,
+		               un = other_tile_row || k == CC_KW - 1 ? g.word(bits, wx + 1, y2, z2, invert) : 0u;
+		if (!(u | (up >> 31) | (un & 1u)))
+			continue;
+		const size_t wu = g.widx(wx, y2, z2);
+		uint32_t id = rb0;
+		for (uint32_t t = st; t; t &= t - 1, id++)
+			run_links(run_mask(w, __ffs(t) - 1), u, up, un, nb[i], [&](int wo, int bu) {
+				const uint32_t uw = wo == 0 ? u : (wo < 0 ? up : un);
+				ccl_link(L, s_seen, id, g.rb[wu + wo] + run_index(run_starts(uw), bu));
 			});
 	}
 }
@@ -402,6 +448,7 @@ __device__ __forceinline__ uint32_t ccl_root(uint32_t *L, uint32_t x0)
 // instead of walked in full by each of them; the flatten pass then finds
 // every root in a few steps.  No value here needs to be final, which is what
 // makes splitting safe (the flatten pass writes only roots).
+template <int CC_KW, int CC_TY, int CC_TZ>
 __global__ void __launch_bounds__(CC_BS)
 k_ccl_jump(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__restrict__ L)
 {
@@ -413,7 +460,7 @@ k_ccl_jump(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__res
 	__syncthreads();
 	uint32_t gi = w ? g.rb[g.widx(wx, y, z)] : 0u;
 	for (uint32_t t = run_starts(w); t; t &= t - 1, gi++) {
-		const uint32_t p = ld_agent(&L[gi]);
+		const uint32_t p = ld_group(&L[gi]);
 		if (p == gi)
 			continue;
 		uint32_t h = memo_hash(p);
@@ -436,6 +483,7 @@ k_ccl_jump(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__res
 // thousands of tiles serialise (they took about 0.8 ms on a 512^3 mask).
 constexpr unsigned CC_FLAT_WG = 1024;
 
+template <int CC_KW, int CC_TY, int CC_TZ>
 __global__ void __launch_bounds__(CC_BS)
 k_ccl_flatten(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__restrict__ L,
               uint32_t *__restrict__ AUX, int mode, uint32_t *__restrict__ nroots,
@@ -598,9 +646,25 @@ k_ccl_flatten(const uint32_t *__restrict__ bits, Geo g, int invert, uint32_t *__
 	}
 }
 
-static dim3 cc_grid(const Geo &g)
+template <int KW, int TY, int TZ>
+static void ccl_passes(const uint32_t *bits, const Geo &g, int conn, int invert, uint32_t *L, uint32_t *AUX, int mode,
+                       uint32_t *nroots, uint32_t *rootlist, hipStream_t s, CclTimer *timer)
 {
-	return dim3((g.W + CC_KW - 1) / CC_KW, (g.ny + CC_TY - 1) / CC_TY, (g.nz + CC_TZ - 1) / CC_TZ);
+	static_assert(KW * TY * TZ == CC_BS, "one word per thread");
+	const dim3 grid((g.W + KW - 1) / KW, (g.ny + TY - 1) / TY, (g.nz + TZ - 1) / TZ);
+	const double nb = (double)g.nx * g.ny * g.nz / 8;
+	if (timer) timer->begin("ccl_local", nb);
+	hipLaunchKernelGGL((k_ccl_local<KW, TY, TZ>), grid, dim3(CC_BS), 0, s, bits, g, conn, invert, L, AUX, mode);
+	if (timer) timer->end();
+	if (timer) timer->begin("ccl_merge", nb);
+	hipLaunchKernelGGL((k_ccl_merge<KW, TY, TZ>), grid, dim3(CC_BS), 0, s, bits, g, conn, invert, L);
+	if (timer) timer->end();
+	if (timer) timer->begin("ccl_flatten", nb);
+	hipLaunchKernelGGL((k_ccl_jump<KW, TY, TZ>), grid, dim3(CC_BS), 0, s, bits, g, invert, L);
+	const uint32_t ntiles = grid.x * grid.y * grid.z;
+	hipLaunchKernelGGL((k_ccl_flatten<KW, TY, TZ>), dim3(ntiles < CC_FLAT_WG ? ntiles : CC_FLAT_WG), dim3(CC_BS), 0, s,
+	                   bits, g, invert, L, AUX, mode, nroots, rootlist, (int)grid.x, (int)grid.y, ntiles);
+	if (timer) timer->end();
 }
 
 void launch_ccl(const uint32_t *bits, int nx, int ny, int nz, int conn, int invert, uint32_t *L,
@@ -608,7 +672,6 @@ void launch_ccl(const uint32_t *bits, int nx, int ny, int nz, int conn, int inve
                 uint32_t *scan_scratch, hipStream_t s, CclTimer *timer)
 {
 	Geo g{nx, ny, nz, (nx + 31) / 32, rbase};
-	dim3 grid = cc_grid(g);
 	const double nb = (double)nx * ny * nz / 8;
 	const size_t nw = (size_t)g.W * ny * nz;
 	// algorithmic bytes: mask bits in per pass; run labels are not counted
@@ -616,18 +679,9 @@ void launch_ccl(const uint32_t *bits, int nx, int ny, int nz, int conn, int inve
 	hipLaunchKernelGGL(k_run_count, dim3((unsigned)((nw + 1 + 255) / 256)), dim3(256), 0, s, bits, g, invert, rbase);
 	scan_excl_u32(rbase, rbase, nw + 1, nullptr, scan_scratch, s);
 	if (timer) timer->end();
-	if (timer) timer->begin("ccl_local", nb);
-	hipLaunchKernelGGL(k_ccl_local, grid, dim3(CC_BS), 0, s, bits, g, conn, invert, L, AUX, mode);
-	if (timer) timer->end();
-	if (timer) timer->begin("ccl_merge", nb);
-	hipLaunchKernelGGL(k_ccl_merge, grid, dim3(CC_BS), 0, s, bits, g, conn, invert, L);
-	if (timer) timer->end();
-	if (timer) timer->begin("ccl_flatten", nb);
-	hipLaunchKernelGGL(k_ccl_jump, grid, dim3(CC_BS), 0, s, bits, g, invert, L);
-	const uint32_t ntiles = grid.x * grid.y * grid.z;
-	hipLaunchKernelGGL(k_ccl_flatten, dim3(ntiles < CC_FLAT_WG ? ntiles : CC_FLAT_WG), dim3(CC_BS), 0, s, bits, g,
-	                   invert, L, AUX, mode, nroots, rootlist, (int)grid.x, (int)grid.y, ntiles);
-	if (timer) timer->end();
+	// tile shape by the words of a row, see CC_BS
+	const auto passes = g.W == 1 ? ccl_passes<1, 16, 16> : (g.W == 2 ? ccl_passes<2, 16, 8> : (g.W <= 4 ? ccl_passes<4, 8, 8> : ccl_passes<8, 8, 4>));
+	passes(bits, g, conn, invert, L, AUX, mode, nroots, rootlist, s, timer);
 }
 
 // largest root: max count, ties -> smallest root.  best = (count<<32)|~root;

@@ -58,6 +58,19 @@ def test_bwlabel(gpu, oracle, shape, p, conn, largest, fill):
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize('shape', [(17, 17, 32), (9, 17, 64), (9, 9, 65), (17, 9, 128), (5, 9, 129), (9, 17, 257)])
+@pytest.mark.parametrize('p', [0.5, 0.97])
+@pytest.mark.parametrize('conn', [6, 18, 26])
+def test_bwlabel_tile_shapes(gpu, oracle, shape, p, conn):
+    """Labelling with each tile shape (rows of one, two, up to four and more
+    words), one row and slice past a whole tile."""
+    m = support.random_mask(shape, conn + shape[2], p)
+    for largest, fill in [(False, False), (True, True)]:
+        a, b = m.copy(), m.copy()
+        assert gpu.lib().bwlabel(a, conn, largest, fill) == oracle.bwlabel(b, conn, largest, fill)
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize('shape', SHAPES)
 @pytest.mark.parametrize('seed', [3, 4])
 @pytest.mark.parametrize('flavour', ['classic', 'lewiner', 'lewiner_o1'])
