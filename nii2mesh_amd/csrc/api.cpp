@@ -3714,12 +3714,11 @@ int set_thresholds_device(n2m_ctx *C, const float *d_img, int64_t nvox, int n, c
 	bool need5 = false;
 	for (int i = 0; i < n; i++)
 		need5 = need5 || modes[i] == 1 || modes[i] == 3;
-	constexpr size_t REC = (sizeof(ThrRecord) + 255) / 256 * 256, H1001 = 4096;
-	char *b = C->buf<char>(S_OTSU, REC + H1001 + (size_t)256 * 256 * 8);
+	constexpr size_t REC = (sizeof(ThrRecord) + 255) / 256 * 256;
+	char *b = C->buf<char>(S_OTSU, REC + N2M_THR_WORK);
 	ThrRecord *rec = (ThrRecord *)b;
 	C->tbegin("set_threshold", 12.0 * nvox);
-	launch_threshold_chain(d_img, (size_t)nvox, rec, (uint32_t *)(b + REC), (double *)(b + REC + H1001), need5,
-	                       C->stream);
+	launch_threshold_chain(d_img, (size_t)nvox, rec, b + REC, need5, C->stream);
 	C->tend();
 	if (!C->h_thr)
 		HIPX(hipHostMalloc((void **)&C->h_thr, sizeof(ThrRecord), hipHostMallocDefault));

@@ -1091,9 +1091,23 @@ template <typename F> __device__ __forceinline__ void each_voxel(const float *__
 		f(img[i]);
 }
 
-__global__ void __launch_bounds__(256) k_hist_range(const float *__restrict__ img, size_t n, uint32_t *stats)
+// The range and histogram passes run in at most TH_ROWS workgroups of 1024
+// threads, each leaving one row of results that the next launch (one
+// workgroup) sums: thousands of workgroups adding to the same range words
+// and bins spent most of these passes in atomics (7.1 M voxels, 28 MB: range
+// 50 us, each histogram 43; now 11 and 16).
+constexpr int TH_BS = 1024, TH_ROWS = 256, TH_BINS = 1001;
+
+static unsigned thr_rows(size_t n)
 {
-	__shared__ uint32_t s_red[3][4];
+	const size_t b = (n + 65535) / 65536; // below that the rows to sum weigh more
+	return (unsigned)(b < 1 ? 1 : (b > (size_t)TH_ROWS ? (size_t)TH_ROWS : b));
+}
+
+// rows[3 * workgroup]: ordered min, ordered max over non-NaN, NaN count
+__global__ void __launch_bounds__(TH_BS) k_hist_range(const float *__restrict__ img, size_t n, uint32_t *rows)
+{
+	__shared__ uint32_t s_red[3][TH_BS / N2M_WAVE];
 	float lmin = __builtin_inff(), lmax = -__builtin_inff();
 	uint32_t nan = 0;
 	each_voxel(img, n, [&](float v) {
@@ -1113,37 +1127,45 @@ __global__ void __launch_bounds__(256) k_hist_range(const float *__restrict__ im
 	}
 	__syncthreads();
 	if (threadIdx.x == 0) {
-		for (int w = 1; w < 4; w++) {
+		for (int w = 1; w < TH_BS / N2M_WAVE; w++) {
 			omin = min(omin, s_red[0][w]);
 			omax = max(omax, s_red[1][w]);
 			nan += s_red[2][w];
 		}
-		atomicMin(&stats[0], omin);
-		atomicMax(&stats[1], omax);
-		if (nan)
-			atomicAdd(&stats[2], nan);
+		rows[3 * blockIdx.x] = omin;
+		rows[3 * blockIdx.x + 1] = omax;
+		rows[3 * blockIdx.x + 2] = nan;
 	}
 }
 
-// bin = round((v - mn) * scl) in float, clamped to [0, nbins-1] (the
-// 1001-bin pass never leaves that range for finite data).
-__device__ __forceinline__ void hist_bins_body(const float *__restrict__ img, size_t n, float mn, float scl, int nbins,
-                                               uint32_t *hist)
+// rows[nbins * workgroup + bin]; bin = round((v - mn) * scl) in float, clamped
+// to [0, nbins-1] (the 1001-bin pass never leaves that range for finite
+// data), with mn = par[0], scl = par[1]; nothing when *enable is 0.
+__global__ void __launch_bounds__(TH_BS)
+k_hist_bins(const float *__restrict__ img, size_t n, const float *__restrict__ par,
+            const int32_t *__restrict__ enable, int nbins, uint32_t *__restrict__ rows)
 {
-	extern __shared__ uint32_t s_h[];
-	for (int i = threadIdx.x; i < nbins; i += blockDim.x)
+	__shared__ uint32_t s_h[TH_BINS];
+	if (enable && *enable == 0)
+		return;
+	const float mn = par[0], scl = par[1];
+	for (int i = threadIdx.x; i < nbins; i += TH_BS)
 		s_h[i] = 0;
 	__syncthreads();
-	// a run of voxels in the same bin (most of a background) is added with
-	// one LDS atomic
+	// bin 0 (most of a background) is counted in a register, a run of voxels in
+	// another bin is added with one LDS atomic
 	int cb = 0;
-	uint32_t cc = 0;
+	uint32_t cc = 0, c0 = 0;
 	each_voxel(img, n, [&](float v) {
 		if (v != v)
 			return;
 		float f = (v - mn) * scl;
 		int b = (int)roundf(f);
 		b = b < 0 ? 0 : (b > nbins - 1 ? nbins - 1 : b);
+		if (b == 0) {
+			c0++;
+			return;
+		}
 		if (b == cb) {
 			cc++;
 			return;
@@ -1155,45 +1177,12 @@ __device__ __forceinline__ void hist_bins_body(const float *__restrict__ img, si
 	});
 	if (cc)
 		atomicAdd(&s_h[cb], cc);
+	c0 = wave_sum(c0);
+	if (lane_id() == 0 && c0)
+		atomicAdd(&s_h[0], c0);
 	__syncthreads();
-	for (int i = threadIdx.x; i < nbins; i += blockDim.x)
-		if (s_h[i])
-			atomicAdd(&hist[i], s_h[i]);
-}
-
-__global__ void __launch_bounds__(256)
-k_hist_bins(const float *__restrict__ img, size_t n, float mn, float scl, int nbins, uint32_t *hist)
-{
-	hist_bins_body(img, n, mn, scl, nbins, hist);
-}
-
-// the same with mn = par[0], scl = par[1] from the device; nothing when
-// *enable is 0
-__global__ void __launch_bounds__(256)
-k_hist_bins_dev(const float *__restrict__ img, size_t n, const float *__restrict__ par,
-                const int32_t *__restrict__ enable, int nbins, uint32_t *hist)
-{
-	if (enable && *enable == 0)
-		return;
-	hist_bins_body(img, n, par[0], par[1], nbins, hist);
-}
-
-static unsigned hist_blocks(size_t n)
-{
-	size_t b = (n + 255) / 256;
-	return (unsigned)(b < 1 ? 1 : (b > 2048 ? 2048 : b));
-}
-
-void launch_hist_range(const float *img, size_t n, uint32_t *stats, hipStream_t s)
-{
-	hipLaunchKernelGGL(k_hist_range, dim3(hist_blocks(n)), dim3(256), 0, s, img, n, stats);
-}
-
-void launch_hist_bins(const float *img, size_t n, float mn, float scl, int nbins, uint32_t *hist,
-                      hipStream_t s)
-{
-	hipLaunchKernelGGL(k_hist_bins, dim3(hist_blocks(n)), dim3(256), nbins * sizeof(uint32_t), s, img, n,
-	                   mn, scl, nbins, hist);
+	for (int i = threadIdx.x; i < nbins; i += TH_BS)
+		rows[(size_t)nbins * blockIdx.x + i] = s_h[i];
 }
 
 unsigned atlas_smooth_blocks(int nx, int ny, int nz, int smooth, int tile)
@@ -1241,143 +1230,220 @@ void launch_binarize(const float *labels, size_t n, float lo, float hi, float *o
 
 // ---------------------------------------------------------------------------
 // Three-threshold Otsu search of nii_otsu() mode 5 (src/isolevel.c:176-197)
-// over the Liao table P (nBin x nBin doubles, built on the host exactly as
-// the reference builds it).  Workgroup l scans every (m, h) for that l;
-// each lane keeps the first strict maximum in h order, the workgroup the
-// first in m order, and the host the first in l order -- the reference's
-// first occurrence of the maximum in (l, m, h) order.
+// over the Liao table, P[u][v] at P[u * su + v * sv].  Workgroup l scans every
+// (m, h) for that l; each lane keeps the first strict maximum in h order, the
+// workgroup the first in m order, and the host the first in l order -- the
+// reference's first occurrence of the maximum in (l, m, h) order.
+// The lanes of a wave read consecutive m for one h, so the device chain
+// keeps the table column by column (su = 1): row by row every lane reads a
+// line of its own.  OT_Q threads share an m, each with every OT_Q-th run of h.
+// 81 us -> 14.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
-k_otsu3(const double *__restrict__ P, int nBin, double *__restrict__ bv, int *__restrict__ bm, int *__restrict__ bh)
+constexpr int OT_Q = 4, OT_RUN = 8;
+__global__ void __launch_bounds__(256 * OT_Q)
+k_otsu3(const double *__restrict__ P, int su, int sv, int nBin, double *__restrict__ bv, int *__restrict__ bm,
+        int *__restrict__ bh)
 {
-	__shared__ double s_v[256];
-	__shared__ int s_h[256];
-	const int l = blockIdx.x, m = l + 1 + threadIdx.x;
+	constexpr int NW = 256 * OT_Q / N2M_WAVE;
+	__shared__ double s_col[256 + OT_Q * OT_RUN], s_v[NW];
+	__shared__ int s_m[NW], s_h[NW];
+	const int tm = threadIdx.x & 255, q = threadIdx.x >> 8;
+	const int l = blockIdx.x, m = l + 1 + tm;
+	if (threadIdx.x < 256 + OT_Q * OT_RUN)
+		s_col[threadIdx.x] =
+		    (int)threadIdx.x < nBin - 1 ? P[(size_t)(threadIdx.x + 1) * su + (size_t)255 * sv] : 0.0;
+	__syncthreads();
 	double best = 0.0;
-	int bestH = -1;
-	if (m < nBin - 2) {
-		const double a = P[l] + P[(size_t)(l + 1) * nBin + m];
-		const double *row = P + (size_t)(m + 1) * nBin;
-		for (int h = m + 1; h < nBin - 1; h++) {
-			const double v = a + row[h] + P[(size_t)(h + 1) * nBin + 255];
-			if (bestH < 0 || v > best) {
+	int bestH = -1, bestM = m;
+	const bool live = m < nBin - 2;
+	const double a = live ? P[(size_t)l * sv] + P[(size_t)(l + 1) * su + (size_t)m * sv] : 0.0;
+	const double *row = P + (size_t)(live ? m + 1 : 0) * su;
+	for (int h0 = m - lane_id() + 1 + q * OT_RUN; h0 < nBin - 1; h0 += OT_Q * OT_RUN) { // from the wave's first m
+		double t[OT_RUN];
+#pragma unroll
+		for (int k = 0; k < OT_RUN; k++)
+			t[k] = h0 + k < nBin ? row[(size_t)(h0 + k) * sv] : 0.0;
+#pragma unroll
+		for (int k = 0; k < OT_RUN; k++) {
+			const int h = h0 + k;
+			const double v = a + t[k] + s_col[h];
+			if (live && h > m && h < nBin - 1 && (bestH < 0 || v > best)) {
 				best = v;
 				bestH = h;
 			}
 		}
 	}
-	s_v[threadIdx.x] = best;
-	s_h[threadIdx.x] = bestH;
+	// the first maximum in (m, h) order: larger value, then smaller m, then h
+	auto take = [&](double v, int vm, int vh) {
+		if (vh >= 0 && (bestH < 0 || v > best || (v == best && (vm < bestM || (vm == bestM && vh < bestH))))) {
+			best = v;
+			bestM = vm;
+			bestH = vh;
+		}
+	};
+#pragma unroll
+	for (int d = N2M_WAVE / 2; d > 0; d >>= 1) {
+		const double v = __shfl_xor(best, d);
+		const int vm = __shfl_xor(bestM, d), vh = __shfl_xor(bestH, d);
+		take(v, vm, vh);
+	}
+	if (lane_id() == 0) {
+		s_v[wave_id()] = best;
+		s_m[wave_id()] = bestM;
+		s_h[wave_id()] = bestH;
+	}
 	__syncthreads();
 	if (threadIdx.x == 0) {
-		double b = 0.0;
-		int bt = -1;
-		for (int t = 0; t < 256; t++) {
-			if (s_h[t] < 0)
-				continue;
-			if (bt < 0 || s_v[t] > b) {
-				b = s_v[t];
-				bt = t;
-			}
-		}
-		bv[l] = b;
-		bm[l] = bt < 0 ? -1 : l + 1 + bt;
-		bh[l] = bt < 0 ? -1 : s_h[bt];
+		for (int w = 1; w < NW; w++)
+			take(s_v[w], s_m[w], s_h[w]);
+		bv[l] = bestH < 0 ? 0.0 : best;
+		bm[l] = bestH < 0 ? -1 : bestM;
+		bh[l] = bestH;
 	}
 }
 
 void launch_otsu3(const double *P, int nBin, double *bv, int *bm, int *bh, hipStream_t s)
 {
 	if (nBin > 3)
-		hipLaunchKernelGGL(k_otsu3, dim3(nBin - 3), dim3(256), 0, s, P, nBin, bv, bm, bh);
+		hipLaunchKernelGGL(k_otsu3, dim3(nBin - 3), dim3(256 * OT_Q), 0, s, P, nBin, 1, nBin, bv, bm, bh);
 }
 
-// The Liao table of nii_otsu (src/isolevel.c:147-175) for a 256-bin
-// histogram, built on the device, one workgroup per row u.  Each workgroup
-// forms the running sums in the reference's order (the bin probabilities in
-// parallel, the sums by one thread; P[0] is the raw count H[0], a quirk the
-// thresholds depend on), then thread v writes P[u][v] = (S*S)/P of the bin
-// range [u, v] (left as is when P is 0); entries with v < u are never read
-// and are set to 0.
-__global__ void __launch_bounds__(256) k_otsu_table(const uint32_t *__restrict__ H, double *__restrict__ P)
+// The 256-bin histogram summed from its rows, and the running sums of
+// nii_otsu's Liao table (src/isolevel.c:147-165) in the reference's order: the
+// bin probabilities in parallel, the sums by one thread (P[0] is the raw
+// count H[0], a quirk the thresholds depend on); sums[0..255] = P,
+// sums[256..511] = S.
+__global__ void __launch_bounds__(TH_BS)
+k_otsu_sums(const uint32_t *__restrict__ rows, int nrows, uint32_t *__restrict__ H, double *__restrict__ sums)
 {
 	constexpr int n = 256;
-	__shared__ double s_p[n], s_s[n], s_prob[n];
-	__shared__ double s_sum;
-	if (threadIdx.x == 0) {
-		double Sum = 0.0;
-		for (int v = 0; v < n; v++)
-			Sum = Sum + (double)(int)H[v];
-		s_sum = Sum;
+	__shared__ uint32_t s_part[TH_BS];
+	__shared__ double s_prob[n], s_w[n], s_red[n / N2M_WAVE];
+	const int v = threadIdx.x % n, q = threadIdx.x / n; // four threads per bin
+	uint32_t c = 0;
+#pragma unroll 32
+	for (int r = q; r < nrows; r += TH_BS / n)
+		c += rows[(size_t)n * r + v];
+	s_part[threadIdx.x] = c;
+	__syncthreads();
+	double h = 0.0;
+	if (threadIdx.x < n) {
+		c = s_part[v] + s_part[n + v] + s_part[2 * n + v] + s_part[3 * n + v];
+		H[v] = c;
+		h = (double)(int)c;
+		const double t = wave_sum(h); // whole numbers: exact in any order
+		if (lane_id() == 0)
+			s_red[wave_id()] = t;
 	}
 	__syncthreads();
-	s_prob[threadIdx.x] = (double)(int)H[threadIdx.x] / s_sum;
+	if (threadIdx.x < n) {
+		const double Sum = s_red[0] + s_red[1] + s_red[2] + s_red[3];
+		const double prob = h / Sum;
+		s_prob[v] = v ? prob : h;
+		s_w[v] = v ? (v + 1) * prob : h;
+	}
 	__syncthreads();
 	if (threadIdx.x == 0) {
-		s_p[0] = (double)(int)H[0];
-		s_s[0] = (double)(int)H[0];
-		for (int v = 1; v < n; v++) {
-			const double prob = s_prob[v];
-			s_p[v] = s_p[v - 1] + prob;
-			s_s[v] = s_s[v - 1] + (v + 1) * prob;
+		double p = s_prob[0], w = s_w[0];
+		sums[0] = p;
+		sums[n] = w;
+#pragma unroll 16
+		for (int i = 1; i < n; i++) {
+			p = p + s_prob[i];
+			w = w + s_w[i];
+			sums[i] = p;
+			sums[n + i] = w;
 		}
 	}
-	__syncthreads();
-	const int u = blockIdx.x, v = threadIdx.x;
-	double val = 0.0;
-	if (v >= u) {
-		const double p = u == 0 ? s_p[v] : s_p[v] - s_p[u - 1];
-		const double q = u == 0 ? s_s[v] : s_s[v] - s_s[u - 1];
-		val = p != 0 ? (q * q) / p : p;
-	}
-	P[(size_t)u * n + v] = val;
 }
 
-// the table entries the host-side searches read: row 0 (P[i]), column 255
-// shifted by one row (P[i+1][255]) and the four terms of the mode-5 start
-// value (lo, mi, hi = 64, 128, 192)
-__global__ void __launch_bounds__(256) k_otsu_probe(const double *__restrict__ P, double *__restrict__ probe)
+// The Liao table (src/isolevel.c:166-175), column by column: entry (u, v) at
+// PT[v * 256 + u] = (S*S)/P of the bin range [u, v] (left as is when P is 0);
+// entries with v < u are never read and are set to 0.  probe: the entries the
+// host-side searches read: row 0, column 255 shifted by one row and the four
+// terms of the mode-5 start value (lo, mi, hi = 64, 128, 192).
+__global__ void __launch_bounds__(256)
+k_otsu_table(const double *__restrict__ sums, double *__restrict__ PT, double *__restrict__ probe)
 {
 	constexpr int n = 256;
-	const int i = threadIdx.x;
-	probe[i] = P[i];
-	probe[n + i] = i < n - 1 ? P[(size_t)(i + 1) * n + (n - 1)] : 0.0;
-	if (i == 0) {
-		probe[2 * n + 0] = P[64];
-		probe[2 * n + 1] = P[(size_t)65 * n + 128];
-		probe[2 * n + 2] = P[(size_t)129 * n + 192];
-		probe[2 * n + 3] = P[(size_t)193 * n + 255];
+	const int v = blockIdx.x, u = threadIdx.x;
+	double val = 0.0;
+	if (v >= u) {
+		const double p = u == 0 ? sums[v] : sums[v] - sums[u - 1];
+		const double q = u == 0 ? sums[n + v] : sums[n + v] - sums[n + u - 1];
+		val = p != 0 ? (q * q) / p : p;
 	}
+	PT[(size_t)v * n + u] = val;
+	if (u == 0)
+		probe[v] = val;
+	if (v == n - 1) {
+		if (u > 0)
+			probe[n + u - 1] = val;
+		else
+			probe[2 * n - 1] = 0.0;
+	}
+	if (u == 0 && v == 64)
+		probe[2 * n] = val;
+	else if (u == 65 && v == 128)
+		probe[2 * n + 1] = val;
+	else if (u == 129 && v == 192)
+		probe[2 * n + 2] = val;
+	else if (u == 193 && v == 255)
+		probe[2 * n + 3] = val;
 }
 
 // ---------------------------------------------------------------------------
 // setThreshold() as one chain of launches (src/isolevel.c:35-277), results
 // in a ThrRecord.
 // ---------------------------------------------------------------------------
-// range statistics {ordered min, ordered max, NaN count}, the parameters and
-// both histograms cleared in one launch (no memset nodes)
-__global__ void __launch_bounds__(256) k_thr_init(ThrRecord *__restrict__ r, uint32_t *__restrict__ h1001)
+// The cases of the robust range (src/isolevel.c:59-139).  First launch
+// (final = 0): the range from its rows, and whether the 1001-bin pass runs,
+// with its mn and scl.  Second launch: the percentiles (the walk over that
+// histogram, summed from its rows, when it ran) and the 256-bin pass's mn and
+// scl (src/isolevel.c:245-250).  All float and double arithmetic in the host
+// code's order.
+__global__ void __launch_bounds__(TH_BS)
+k_thr_range(ThrRecord *__restrict__ r, const uint32_t *__restrict__ rows, int nrows, size_t nvox, int final)
 {
-	for (int i = threadIdx.x; i < 1024; i += blockDim.x)
-		h1001[i] = 0u;
-	r->h256[threadIdx.x] = 0u;
-	if (threadIdx.x < 4) {
-		r->stats[threadIdx.x] = threadIdx.x == 0 ? 0xffffffffu : 0u;
-		r->par[threadIdx.x] = 0.0f;
+	constexpr int kBins = TH_BINS;
+	__shared__ uint32_t s_st[3];
+	const int t = threadIdx.x;
+	if (!final) {
+		__shared__ uint32_t s_red[3][TH_BS / N2M_WAVE];
+		uint32_t omin = 0xffffffffu, omax = 0u, nan = 0u;
+		if (t < nrows) {
+			omin = rows[3 * t];
+			omax = rows[3 * t + 1];
+			nan = rows[3 * t + 2];
+		}
+		omin = wave_min_u32(omin);
+		omax = wave_max_u32(omax);
+		nan = wave_sum(nan);
+		if (lane_id() == 0) {
+			s_red[0][wave_id()] = omin;
+			s_red[1][wave_id()] = omax;
+			s_red[2][wave_id()] = nan;
+		}
+		__syncthreads();
+		if (t == 0) {
+			for (int w = 1; w < TH_BS / N2M_WAVE; w++) {
+				omin = min(omin, s_red[0][w]);
+				omax = max(omax, s_red[1][w]);
+				nan += s_red[2][w];
+			}
+			r->stats[0] = s_st[0] = omin;
+			r->stats[1] = s_st[1] = omax;
+			r->stats[2] = s_st[2] = nan;
+			r->stats[3] = 0u;
+			r->par[0] = r->par[1] = 0.0f;
+			r->do1001 = 0;
+		}
+	} else if (t < 3) {
+		s_st[t] = r->stats[t];
 	}
-	if (threadIdx.x == 0)
-		r->do1001 = 0;
-}
-
-// One thread: the cases of the robust range (src/isolevel.c:59-139).  First
-// call (final = 0): whether the 1001-bin pass runs, with its mn and scl.
-// Second call: the percentiles (the walk over that histogram when it ran)
-// and the 256-bin pass's mn and scl (src/isolevel.c:245-250).  All float
-// and double arithmetic in the host code's order.
-__global__ void k_thr_range(ThrRecord *__restrict__ r, const uint32_t *__restrict__ h1001, size_t nvox, int final)
-{
-	const size_t nNan = r->stats[2];
-	const float mn = ord2f(r->stats[0]), mx = ord2f(r->stats[1]);
+	__syncthreads();
+	const size_t nNan = s_st[2];
+	const float mn = ord2f(s_st[0]), mx = ord2f(s_st[1]);
 	float pct2 = 0.0f, pct98 = 1.0f;
 	if (nvox == nNan) {
 		// all NaN: the range keeps its 0..1 defaults
@@ -1390,88 +1456,159 @@ __global__ void k_thr_range(ThrRecord *__restrict__ r, const uint32_t *__restric
 		if (n2pct < 1 || valid < 100) {
 			pct2 = mn;
 			pct98 = mx;
-		} else {
-			const int kBins = 1001;
+		} else { // the same for every thread
 			const float scl = (kBins - 1) / (mx - mn);
 			if (!final) {
-				r->do1001 = 1;
-				r->par[0] = mn;
-				r->par[1] = scl;
+				if (t == 0) {
+					r->do1001 = 1;
+					r->par[0] = mn;
+					r->par[1] = scl;
+				}
 				return;
 			}
-			int lo, hi;
-			robust_walk(h1001, kBins, n2pct, &lo, &hi);
-			pct2 = (lo) / scl + mn;
-			pct98 = (hi) / scl + mn;
+			// robust_walk() over the summed bins: lo is the first bin whose
+			// count from below reaches n2pct, hi the last from above
+			__shared__ uint32_t s_h[TH_BS];
+			__shared__ unsigned long long s_wave[TH_BS / N2M_WAVE];
+			__shared__ int s_lo, s_hi;
+			uint32_t c = 0;
+			if (t < kBins)
+#pragma unroll 32
+				for (int i = 0; i < nrows; i++)
+					c += rows[(size_t)kBins * i + t];
+			s_h[t] = c;
+			if (t == 0) {
+				s_lo = 0;
+				s_hi = kBins - 1;
+			}
+			unsigned long long upto = c; // 64-bit: volumes of 2^32 voxels and more
+#pragma unroll
+			for (int d = 1; d < N2M_WAVE; d <<= 1) {
+				const unsigned long long o = __shfl_up(upto, d);
+				upto += lane_id() >= d ? o : 0ull;
+			}
+			if (lane_id() == N2M_WAVE - 1)
+				s_wave[wave_id()] = upto;
+			__syncthreads();
+			unsigned long long all = 0;
+			for (int w = 0; w < TH_BS / N2M_WAVE; w++) {
+				upto += w < wave_id() ? s_wave[w] : 0ull;
+				all += s_wave[w];
+			}
+			const unsigned long long before = upto - c;
+			if (upto >= n2pct && before < n2pct)
+				s_lo = t;
+			if (t < kBins && all - before >= n2pct && all - upto < n2pct)
+				s_hi = t;
+			__syncthreads();
+			if (t == 0) {
+				int lo = s_lo, hi = s_hi;
+				if (lo == hi) // both move outwards to the next bins in use
+					robust_walk(s_h, kBins, n2pct, &lo, &hi);
+				pct2 = (lo) / scl + mn;
+				pct98 = (hi) / scl + mn;
+			}
 		}
 	}
-	if (final) {
+	if (final && t == 0) {
 		const int nBin = 256;
 		r->par[2] = pct2;
 		r->par[3] = (nBin - 1) / (pct98 - pct2);
 	}
 }
 
-void launch_threshold_chain(const float *img, size_t nvox, ThrRecord *rec, uint32_t *h1001, double *P, bool need5,
-                            hipStream_t s)
+// work: the rows of a pass, then (once the last histogram is summed) the
+// Liao table and, after it, its running sums
+static_assert(N2M_THR_WORK >= (size_t)TH_ROWS * TH_BINS * sizeof(uint32_t), "the rows of the longest pass fit");
+static_assert((size_t)256 * 256 * 8 >= (size_t)TH_ROWS * 256 * 4, "the sums are not among the rows they come from");
+static_assert((size_t)(256 + 2) * 256 * 8 <= N2M_THR_WORK, "table and sums fit");
+
+void launch_threshold_chain(const float *img, size_t nvox, ThrRecord *rec, void *work, bool need5, hipStream_t s)
 {
-	const unsigned hb = hist_blocks(nvox);
-	hipLaunchKernelGGL(k_thr_init, dim3(1), dim3(256), 0, s, rec, h1001);
-	hipLaunchKernelGGL(k_hist_range, dim3(hb), dim3(256), 0, s, img, nvox, rec->stats);
-	hipLaunchKernelGGL(k_thr_range, dim3(1), dim3(1), 0, s, rec, (const uint32_t *)h1001, nvox, 0);
-	hipLaunchKernelGGL(k_hist_bins_dev, dim3(hb), dim3(256), 1001 * sizeof(uint32_t), s, img, nvox,
-	                   (const float *)rec->par, (const int32_t *)&rec->do1001, 1001, h1001);
-	hipLaunchKernelGGL(k_thr_range, dim3(1), dim3(1), 0, s, rec, (const uint32_t *)h1001, nvox, 1);
-	hipLaunchKernelGGL(k_hist_bins_dev, dim3(hb), dim3(256), 256 * sizeof(uint32_t), s, img, nvox,
-	                   (const float *)(rec->par + 2), (const int32_t *)nullptr, 256, rec->h256);
-	hipLaunchKernelGGL(k_otsu_table, dim3(256), dim3(256), 0, s, (const uint32_t *)rec->h256, P);
-	hipLaunchKernelGGL(k_otsu_probe, dim3(1), dim3(256), 0, s, (const double *)P, rec->probe);
+	const unsigned nr = thr_rows(nvox);
+	uint32_t *rows = (uint32_t *)work;
+	double *PT = (double *)work, *sums = PT + 256 * 256;
+	hipLaunchKernelGGL(k_hist_range, dim3(nr), dim3(TH_BS), 0, s, img, nvox, rows);
+	hipLaunchKernelGGL(k_thr_range, dim3(1), dim3(TH_BS), 0, s, rec, (const uint32_t *)rows, (int)nr, nvox, 0);
+	hipLaunchKernelGGL(k_hist_bins, dim3(nr), dim3(TH_BS), 0, s, img, nvox, (const float *)rec->par,
+	                   (const int32_t *)&rec->do1001, TH_BINS, rows);
+	hipLaunchKernelGGL(k_thr_range, dim3(1), dim3(TH_BS), 0, s, rec, (const uint32_t *)rows, (int)nr, nvox, 1);
+	hipLaunchKernelGGL(k_hist_bins, dim3(nr), dim3(TH_BS), 0, s, img, nvox, (const float *)(rec->par + 2),
+	                   (const int32_t *)nullptr, 256, rows);
+	hipLaunchKernelGGL(k_otsu_sums, dim3(1), dim3(TH_BS), 0, s, (const uint32_t *)rows, (int)nr, rec->h256, sums);
+	hipLaunchKernelGGL(k_otsu_table, dim3(256), dim3(256), 0, s, (const double *)sums, PT, rec->probe);
 	if (need5)
-		launch_otsu3(P, 256, rec->bv, rec->bm, rec->bh, s);
+		hipLaunchKernelGGL(k_otsu3, dim3(256 - 3), dim3(256 * OT_Q), 0, s, (const double *)PT, 1, 256, 256, rec->bv, rec->bm,
+		                   rec->bh);
 }
 
 
 // ---------------------------------------------------------------------------
 // Raw NIfTI voxels to the FP32 working volume, src/nii2mesh.c:155-172:
 // out = (raw * slope) + inter in float (two roundings), for uint8, int16,
-// uint16 and float32 data.  Four voxels per thread.
+// uint16 and float32 data.
 // ---------------------------------------------------------------------------
-template <typename T>
+// Bound by memory.  VEC: 16-byte stores and loads of DEC_VPT raw voxels at a time (raw and out
+// aligned to that); the last n % DEC_VPT voxels one by one.
+constexpr int DEC_VPT = 8;
+template <typename T, bool VEC>
 __global__ void __launch_bounds__(256)
 k_decode(const T *__restrict__ raw, size_t n, float slope, float inter, float *__restrict__ out)
 {
-	const size_t stride = (size_t)gridDim.x * blockDim.x * 4;
-	for (size_t i = (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * 4; i < n; i += stride) {
+	const size_t tid = blockIdx.x * (size_t)blockDim.x + threadIdx.x, stride = (size_t)gridDim.x * blockDim.x;
+	size_t done = 0;
+	if (VEC) {
+		struct alignas(DEC_VPT * sizeof(T) < 16 ? DEC_VPT * sizeof(T) : 16) Pack {
+			T v[DEC_VPT];
+		};
+		const size_t np = n / DEC_VPT;
+		for (size_t i = tid; i < np; i += stride) {
+			const Pack p = reinterpret_cast<const Pack *>(raw)[i];
+			float f[DEC_VPT];
 #pragma unroll
-		for (int k = 0; k < 4; k++) {
-			if (i + k < n) {
-				const float v = (float)raw[i + k] * slope;
-				out[i + k] = v + inter;
+			for (int k = 0; k < DEC_VPT; k++) {
+				const float v = (float)p.v[k] * slope;
+				f[k] = v + inter;
 			}
+			float4 *o = reinterpret_cast<float4 *>(out) + i * (DEC_VPT / 4);
+#pragma unroll
+			for (int k = 0; k < DEC_VPT / 4; k++)
+				o[k] = make_float4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
 		}
+		done = np * DEC_VPT;
 	}
+	for (size_t i = done + tid; i < n; i += stride) {
+		const float v = (float)raw[i] * slope;
+		out[i] = v + inter;
+	}
+}
+
+template <typename T>
+static void decode_launch(const void *raw, size_t n, float slope, float inter, float *out, hipStream_t s)
+{
+	const uintptr_t at = DEC_VPT * sizeof(T) < 16 ? DEC_VPT * sizeof(T) : 16;
+	const bool vec = ((uintptr_t)raw % at) == 0 && ((uintptr_t)out & 15u) == 0;
+	const size_t per = 256 * (size_t)(vec ? DEC_VPT : 4);
+	size_t b = (n + per - 1) / per;
+	b = b > 8192 ? 8192 : (b < 1 ? 1 : b);
+	const auto k = vec ? k_decode<T, true> : k_decode<T, false>;
+	hipLaunchKernelGGL(k, dim3((unsigned)b), dim3(256), 0, s, (const T *)raw, n, slope, inter, out);
 }
 
 int launch_decode(const void *raw, int datatype, size_t n, float slope, float inter, float *out, hipStream_t s)
 {
-	size_t b = (n + 1023) / 1024;
-	b = b > 8192 ? 8192 : (b < 1 ? 1 : b);
 	switch (datatype) {
 	case 2: // DT_UINT8
-		hipLaunchKernelGGL(k_decode<uint8_t>, dim3((unsigned)b), dim3(256), 0, s, (const uint8_t *)raw, n, slope,
-		                   inter, out);
+		decode_launch<uint8_t>(raw, n, slope, inter, out, s);
 		return 0;
 	case 4: // DT_INT16
-		hipLaunchKernelGGL(k_decode<int16_t>, dim3((unsigned)b), dim3(256), 0, s, (const int16_t *)raw, n, slope,
-		                   inter, out);
+		decode_launch<int16_t>(raw, n, slope, inter, out, s);
 		return 0;
 	case 512: // DT_UINT16
-		hipLaunchKernelGGL(k_decode<uint16_t>, dim3((unsigned)b), dim3(256), 0, s, (const uint16_t *)raw, n, slope,
-		                   inter, out);
+		decode_launch<uint16_t>(raw, n, slope, inter, out, s);
 		return 0;
 	case 16: // DT_FLOAT32
-		hipLaunchKernelGGL(k_decode<float>, dim3((unsigned)b), dim3(256), 0, s, (const float *)raw, n, slope, inter,
-		                   out);
+		decode_launch<float>(raw, n, slope, inter, out, s);
 		return 0;
 	}
 	return -1;

@@ -109,7 +109,6 @@ bool launch_apply(const float *src, float *img, int nx, int ny, int nz, float is
                   const uint32_t *keep, const uint32_t *dil, int fill, const uint32_t *range, uint32_t *part,
                   uint32_t *host, hipStream_t s, uint32_t *sgp = nullptr, uint32_t *sgn = nullptr);
 size_t apply_part_words();
-void launch_hist_range(const float *img, size_t n, uint32_t *stats, hipStream_t s);
 // mesh output encoding (k_encode.hip)
 void launch_f64_to_f32(const double *in, size_t n, float *out, hipStream_t s);
 void launch_ply_faces(const int *tris, size_t nt, uint8_t *out, hipStream_t s);
@@ -124,7 +123,6 @@ void launch_vtk_polys(const int *tris, size_t nt, uint32_t *out, hipStream_t s);
 int launch_decode(const void *raw, int datatype, size_t n, float slope, float inter, float *out, hipStream_t s);
 // mode-5 Otsu search, one workgroup per first threshold l (nBin <= 258)
 void launch_otsu3(const double *P, int nBin, double *bv, int *bm, int *bh, hipStream_t s);
-void launch_hist_bins(const float *img, size_t n, float mn, float scl, int nbins, uint32_t *hist, hipStream_t s);
 
 // atlas volume stages (k_volume.hip)
 void launch_atlas_stats(const float *labels, int nx, int ny, int nz, int nlabel, uint32_t *stats, hipStream_t s);
@@ -365,10 +363,10 @@ struct ThrRecord {
 	double bv[256];            // mode-5 search: best value, m and h per first threshold l
 	int32_t bm[256], bh[256];
 };
-// rec: device record; h1001: 1024 words; P: 256 x 256 doubles.  need5: run
+// rec: device record; work: N2M_THR_WORK bytes, 8-byte aligned.  need5: run
 // the three-threshold search (modes 1 and 3).  Uses no host round trip.
-void launch_threshold_chain(const float *img, size_t nvox, ThrRecord *rec, uint32_t *h1001, double *P, bool need5,
-                            hipStream_t s);
+void launch_threshold_chain(const float *img, size_t nvox, ThrRecord *rec, void *work, bool need5, hipStream_t s);
+constexpr size_t N2M_THR_WORK = 256 * 1001 * 4;
 // the isolevels of setThreshold(img, nvox, modes[i]) from the chain's record
 // (src/isolevel.c:141-277): mode 1 dark, 3 bright, anything else medium
 void thresholds_from_record(const ThrRecord &r, int n, const int *modes, float *out);

@@ -7,7 +7,7 @@
 // (`scratch` below, 1 MiB per device, held until the process ends); host
 // side it uses only a fixed-size stack record.  Every call on a device
 // shares that device's array: calls that overlap on one device race.
-// Whatever the previous call left there is cleared by a kernel before use.
+// Whatever the previous call left there is overwritten before it is read.
 #include <hip/hip_runtime.h>
 
 #include <math.h>
@@ -27,9 +27,8 @@ namespace {
 constexpr size_t SCRATCH_BYTES = (size_t)1 << 20;
 // byte offsets inside scratch
 constexpr size_t OFF_REC = 0;                                           // the chain's record
-constexpr size_t OFF_H1001 = (sizeof(ThrRecord) + 255) / 256 * 256;    // 1024 words (1001 bins used)
-constexpr size_t OFF_P = OFF_H1001 + 4096;                              // 256 x 256 doubles: the Otsu table
-static_assert(OFF_P + 256 * 256 * 8 <= SCRATCH_BYTES, "scratch size");
+constexpr size_t OFF_WORK = (sizeof(ThrRecord) + 255) / 256 * 256;     // the chain's work area
+static_assert(OFF_WORK + N2M_THR_WORK <= SCRATCH_BYTES, "scratch size");
 
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
@@ -94,8 +93,7 @@ int thresholds(const float *d_img, int64_t nvox, int n, const int *modes, float 
 		need5 = need5 || modes[i] != 2;
 	// the whole of setThreshold() on the device (src/isolevel.c:35-277), one
 	// copy of the record back
-	launch_threshold_chain(d_img, (size_t)nvox, (ThrRecord *)(base + OFF_REC), (uint32_t *)(base + OFF_H1001),
-	                       (double *)(base + OFF_P), need5, s);
+	launch_threshold_chain(d_img, (size_t)nvox, (ThrRecord *)(base + OFF_REC), base + OFF_WORK, need5, s);
 	NAX(hipGetLastError());
 	ThrRecord rec;
 	NAX(hipMemcpyAsync(&rec, base + OFF_REC, sizeof rec, hipMemcpyDeviceToHost, s));

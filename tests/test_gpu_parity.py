@@ -146,6 +146,26 @@ def test_unify_scan_tile_boundaries(gpu, oracle, n):
     assert _eq(d1, d2)
 
 
+@pytest.mark.parametrize('n', [99, 100, 65536, 65537, 5 * 65536 + 3, 257 * 65536 + 1])
+@pytest.mark.parametrize('kind', ['clipped', 'nan', 'two', 'spike'])
+def test_set_threshold_rows(gpu, oracle, n, kind):
+    """Thresholds with one, two and the most workgroups (each sums a row of
+    its own), a clipped background in the first bin, NaN voxels, two values
+    only and one value far from the rest (both percentiles in one bin: they
+    move outwards)."""
+    rng = np.random.default_rng(n)
+    img = np.clip(rng.standard_normal(n, dtype=np.float32) * 20 + 30 * (np.arange(n) % 3), 0, 255).astype(np.float32)
+    if kind == 'nan':
+        img[::7] = np.nan
+    elif kind == 'two':
+        img = (img > 40).astype(np.float32)
+    elif kind == 'spike':
+        img[:] = 5.0
+        img[0], img[1] = 1e6, -3.0
+    for mode in (1, 2, 3):
+        assert gpu.lib().setThreshold(img, mode) == oracle.setThreshold(img, mode)
+
+
 @pytest.mark.parametrize('n', [2, 64, 1024, 1025, 128 * 1024, 128 * 1024 + 1, 128 * 2048, 128 * 2048 + 1, 128 * 4096,
                                128 * 4096 + 1])
 def test_unify_sort_tile_boundaries(gpu, oracle, n):
