@@ -1712,26 +1712,39 @@ k_laplace_h(const uint32_t *__restrict__ start, const uint32_t *__restrict__ slo
 // those of the two-launch form.  Ring-1 pair lists are kept per block as LDS
 // slots (roff: 16-bit offsets, rslots: slot pairs).
 // ---------------------------------------------------------------------------
-// RB (vertices per block) is a template parameter: 512, 640 or 768.
-constexpr int RT = 1024;
-constexpr int R1CAP = 1024;      // ring-1 vertices per block (RB + R1CAP <= 2 * RT)
-constexpr int RROWS = 2304;      // LDS rows: RB + ring 1 + ring 2 (ring words per block: RROWS - RB)
-constexpr int RPCAP = 4096;      // ring-1 pair words per block
-constexpr int ROFFW = R1CAP + 2; // 16-bit ring-1 offsets per block
+constexpr int HE = 6; // a vertex's pairs kept pair by pair, see k_ring_build
+// RB (vertices per block) is a template parameter: 512 to 896 with 1024
+// threads, or 256 with 512 (ring_rb chooses).  An iteration of a small mesh
+// takes as long as one of its blocks does, and a smaller block has fewer rows
+// to read and leaves no CU without one.
+template <int RB_> struct RingCfg {
+	static constexpr bool LARGE = RB_ >= 512;
+	static constexpr int T = LARGE ? 1024 : 2 * RB_;                       // threads
+	static constexpr int R1CAP = LARGE ? 1024 : 2 * RB_;                   // ring-1 vertices per block
+	static constexpr int ROWS = LARGE ? 2304 : 1152;                       // LDS rows: RB + ring 1 + ring 2
+	static constexpr int CAP = ROWS - RB_;                                 // ring words per block
+	static constexpr int RP = LARGE ? 6144 : HE * R1CAP + R1CAP;            // ring-1 pair words per block
+	static constexpr int OP = 2 * RB_;                                     // own pairs beyond HE per block
+	static constexpr int PCAP = RP + OP;                                   // pair words of a block
+	static constexpr int HBITS = LARGE ? 12 : 11;                          // hash slots of the build, log2
+	static_assert(RB_ + R1CAP <= 2 * T, "two passes take block and ring 1");
+	static_assert(R1CAP <= T, "one ring-1 vertex per thread in the build");
+	static_assert((1 << HBITS) > CAP + CAP / 4, "hash slots for the rings");
+};
 constexpr int RK = 6;            // pairs per vertex held in registers by k_ring_build
 
-// LDS hash set of vertex ids (open addressing, RHS slots) used by
+// LDS hash set of vertex ids (open addressing, 2^BITS slots) used by
 // k_ring_build: key RH_EMPTY marks a free slot, val the id's LDS row.
-constexpr int RHS = 4096;
 constexpr uint32_t RH_EMPTY = 0xffffffffu;
-__device__ __forceinline__ uint32_t rh_hash(uint32_t x) { return (x * 2654435761u) >> 20; } // 12 bits
+template <int BITS> __device__ __forceinline__ uint32_t rh_hash(uint32_t x) { return (x * 2654435761u) >> (32 - BITS); }
 
 // insert x; a new id is appended (as its slot) to list[*count] when *count <
 // cap.  Returns false when the table is full or the list overflows.
+template <int BITS>
 __device__ __forceinline__ bool rh_insert(uint32_t *key, uint32_t x, uint32_t *list, uint32_t *count, uint32_t cap)
 {
-	uint32_t h = rh_hash(x);
-	for (int p = 0; p < RHS; p++, h = (h + 1) & (RHS - 1)) {
+	uint32_t h = rh_hash<BITS>(x);
+	for (int p = 0; p < (1 << BITS); p++, h = (h + 1) & ((1 << BITS) - 1)) {
 		const uint32_t prev = atomicCAS(&key[h], RH_EMPTY, x);
 		if (prev == RH_EMPTY) {
 			const uint32_t i = atomicAdd(count, 1u);
@@ -1747,17 +1760,19 @@ __device__ __forceinline__ bool rh_insert(uint32_t *key, uint32_t x, uint32_t *l
 }
 
 // slot of x, which is present
+template <int BITS>
 __device__ __forceinline__ uint32_t rh_find(const uint32_t *key, uint32_t x)
 {
-	uint32_t h = rh_hash(x);
-	for (int p = 0; p < RHS && key[h] != x; p++)
-		h = (h + 1) & (RHS - 1);
+	uint32_t h = rh_hash<BITS>(x);
+	for (int p = 0; p < (1 << BITS) && key[h] != x; p++)
+		h = (h + 1) & ((1 << BITS) - 1);
 	return h;
 }
 
 // The n ids at key[list[0, n)] in ascending order into out[0, n), and each
 // id's row (row0 + its rank) into val.  Rank = number of smaller ids (the
 // ids are distinct); O(n^2 / RT) LDS reads, broadcast across the wave.
+template <int RT>
 __device__ __forceinline__ void rh_rank(const uint32_t *key, const uint32_t *list, uint32_t n, uint32_t *ids,
                                         uint32_t *out, uint32_t *val, uint32_t row0)
 {
@@ -1775,19 +1790,29 @@ __device__ __forceinline__ void rh_rank(const uint32_t *key, const uint32_t *lis
 	__syncthreads();
 }
 
-// Per block: ring 1, ring 2, the block's pairs as row slots (slots, indexed
-// like pairs) and ring 1's pairs (roff / rslots).  The rings are collected in
-// an LDS hash set (an id already present -- block, ring 1 or ring 2 -- is
-// skipped) and then ordered by id.  A block whose rings exceed the caps
-// raises *overflow and the caller keeps the two-launch form.
+// Per block: ring 1, ring 2, the block's pairs as row slots and ring 1's.  The
+// first HE pairs of every vertex are kept pair by pair (pair k of all the
+// block's vertices, then pair k + 1), so that a wave reads them in whole lines
+// and without knowing where the vertex's list starts: ell, HE * RB words per
+// block, and rslots, HE * (ring-1 stride) words.  The pairs after them follow
+// densely in rslots: ring 1's, and from Cfg::RP on the block's own.  deg and
+// rdeg: a vertex's degree | its first such pair << 16.  The rings are
+// collected in an LDS hash set (an id already present -- block, ring 1 or ring
+// 2 -- is skipped) and then ordered by id.  A small block's unused ring words
+// name a vertex too, so that the iteration can read them before it knows the
+// rings' sizes.  A block whose rings or lists exceed the caps raises *overflow
+// and the caller keeps another form.
 template <int RB>
-__global__ void __launch_bounds__(RT, 8)
+__global__ void __launch_bounds__(RingCfg<RB>::T, 8)
 k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs, uint32_t nv,
              const d3 *__restrict__ o, uint32_t *__restrict__ ring, uint2 *__restrict__ rcnt,
-             uint32_t *__restrict__ slots, uint16_t *__restrict__ roff, uint32_t *__restrict__ rslots,
+             uint32_t *__restrict__ deg, uint32_t *__restrict__ ell, uint32_t *__restrict__ rdeg,
+             uint32_t *__restrict__ rslots,
              d3 *__restrict__ o1, uint32_t *__restrict__ overflow)
 {
-	constexpr int RCAP = RROWS - RB;
+	using Cfg = RingCfg<RB>;
+	constexpr int RT = Cfg::T, RCAP = Cfg::CAP, R1CAP = Cfg::R1CAP;
+	constexpr int HB_ = Cfg::HBITS, RHS = 1 << HB_;
 	__shared__ uint32_t hkey[RHS], hval[RHS];
 	__shared__ uint32_t lst[RCAP], ids[RCAP], srt[RCAP]; // hash slots, ids, sorted ids (ring 1, then ring 2)
 	__shared__ uint32_t scratch[RT / N2M_WAVE + 1];
@@ -1817,7 +1842,7 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 #pragma unroll
 		for (int c = 0; c < 2; c++) {
 			const uint32_t x = (uint32_t)(c ? q.y : q.x);
-			if (x - base >= (uint32_t)RB && !rh_insert(hkey, x, lst, &s_n1, R1CAP))
+			if (x - base >= (uint32_t)RB && !rh_insert<HB_>(hkey, x, lst, &s_n1, R1CAP))
 				s_bad = 1;
 		}
 	};
@@ -1838,7 +1863,7 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 		return;
 	}
 	const uint32_t n1 = s_n1;
-	rh_rank(hkey, lst, n1, ids, srt, hval, RB);
+	rh_rank<RT>(hkey, lst, n1, ids, srt, hval, RB);
 	// ring 2: ring 1's references to vertices outside block and ring 1
 	// (ring-1 vertex i = tid, n1 <= RT)
 	uint32_t hb = 0, he = 0;
@@ -1853,7 +1878,7 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 #pragma unroll
 		for (int c = 0; c < 2; c++) {
 			const uint32_t x = (uint32_t)(c ? q.y : q.x);
-			if (x - base >= (uint32_t)RB && !rh_insert(hkey, x, lst + n1, &s_n2, RCAP - n1))
+			if (x - base >= (uint32_t)RB && !rh_insert<HB_>(hkey, x, lst + n1, &s_n2, RCAP - n1))
 				s_bad = 1;
 		}
 	};
@@ -1873,137 +1898,202 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 		return;
 	}
 	const uint32_t n2 = s_n2;
-	rh_rank(hkey, lst + n1, n2, ids + n1, srt + n1, hval, RB + n1);
-	// ring-1 pair offsets (one ring-1 vertex per thread)
-	uint32_t ptot;
-	const uint32_t poff = block_excl_scan<RT>(he - hb, scratch, &ptot);
-	if (ptot > (uint32_t)RPCAP) { // uniform
+	rh_rank<RT>(hkey, lst + n1, n2, ids + n1, srt + n1, hval, RB + n1);
+	// the pairs beyond HE, of ring 1 (one vertex per thread) and the block's own
+	const uint32_t rd = he - hb, od = e - b, S1 = Cfg::LARGE ? n1 : (uint32_t)R1CAP;
+	uint32_t ptot, otot;
+	const uint32_t poff = block_excl_scan<RT>(rd > (uint32_t)HE ? rd - HE : 0u, scratch, &ptot);
+	const uint32_t ooff = block_excl_scan<RT>(od > (uint32_t)HE ? od - HE : 0u, scratch, &otot);
+	if (HE * S1 + ptot > (uint32_t)Cfg::RP || otot > (uint32_t)Cfg::OP) { // uniform
 		if (tid == 0)
 			atomicOr(overflow, 1u);
 		return;
 	}
 	uint32_t *rg = ring + (size_t)blk * RCAP;
-	for (uint32_t i = tid; i < n1 + n2; i += RT)
-		rg[i] = srt[i];
-	if (tid < n1)
+	for (uint32_t i = tid; i < (Cfg::LARGE ? n1 + n2 : (uint32_t)RCAP); i += RT)
+		rg[i] = i < n1 + n2 ? srt[i] : base;
+	if (tid < n1) {
 		o1[(size_t)blk * R1CAP + tid] = ov1;
+		// a degree of 2^16 has more pairs beyond HE than any block takes
+		rdeg[(size_t)blk * R1CAP + tid] = rd | (poff << 16);
+	}
 	if (tid == 0)
 		rcnt[blk] = make_uint2(n1, n2);
-	uint16_t *ro = roff + (size_t)blk * ROFFW;
-	if (tid < n1)
-		ro[tid] = (uint16_t)poff;
-	if (tid == 0)
-		ro[n1] = (uint16_t)ptot;
 	// row slot of a vertex of block, ring 1 or ring 2
-	auto row = [&](uint32_t x) -> uint32_t { return x - base < (uint32_t)RB ? x - base : hval[rh_find(hkey, x)]; };
+	auto row = [&](uint32_t x) -> uint32_t { return x - base < (uint32_t)RB ? x - base : hval[rh_find<HB_>(hkey, x)]; };
 	auto slot = [&](const int2 q) { return row((uint32_t)q.x) | (row((uint32_t)q.y) << 16); };
+	static_assert(RK == HE, "the pairs held in registers are the first HE");
+	uint32_t *el = ell + (size_t)blk * HE * RB + tid, *rs = rslots + (size_t)blk * Cfg::PCAP;
+	if (tid < RB && base + tid < nv)
+		deg[base + tid] = od | (ooff << 16);
 	{
 		int2 qa[RK];
 		load_pairs(qa, b, e);
 #pragma unroll
 		for (int k = 0; k < RK; k++)
 			if (b + k < e)
-				slots[b + k] = slot(qa[k]);
+				el[k * RB] = slot(qa[k]);
 	}
-	for (uint32_t k = b + RK; k < e; k++)
-		slots[k] = slot(pairs[k]);
-	uint32_t *rs = rslots + (size_t)blk * RPCAP + poff;
+	for (uint32_t k = HE; b + k < e; k++)
+		rs[Cfg::RP + ooff + (k - HE)] = slot(pairs[b + k]);
 	{
 		int2 qr[RK];
 		load_pairs(qr, hb, he);
 #pragma unroll
 		for (int k = 0; k < RK; k++)
 			if (hb + k < he)
-				rs[k] = slot(qr[k]);
+				rs[k * S1 + tid] = slot(qr[k]);
 	}
-	for (uint32_t k = hb + RK; k < he; k++)
-		rs[k - hb] = slot(pairs[k]);
+	for (uint32_t k = HE; hb + k < he; k++)
+		rs[HE * S1 + poff + (k - HE)] = slot(pairs[hb + k]);
+}
+
+// A vertex's list in the two-ring form: its first HK pairs, its degree | first
+// pair beyond HE << 16.
+struct EllRefs {
+	uint32_t q[HK], d;
+};
+
+// laplace_at() over it; the pairs beyond HE start at m
+template <int NR>
+__device__ __forceinline__ d3 laplace_ell(const EllRefs &r, const lds_double *L, const d3 self,
+                                          const uint32_t *__restrict__ rs, uint32_t m)
+{
+	const uint32_t n = r.d & 0xffffu;
+	if (n == 0)
+		return self;
+	double sx = 0.0, sy = 0.0, sz = 0.0;
+	auto add = [&](uint32_t w) {
+		const d3 P = lds_row_w<2, NR>(L, w & 0xffffu), Q = lds_row_w<2, NR>(L, w >> 16);
+		sx = sx + (P.x + Q.x);
+		sy = sy + (P.y + Q.y);
+		sz = sz + (P.z + Q.z);
+	};
+#pragma unroll
+	for (int k = 0; k < HK; k++)
+		if ((uint32_t)k < n)
+			add(r.q[k]);
+#pragma unroll 1
+	for (uint32_t k = HK; k < n; k++)
+		add(rs[m + (k - HE)]);
+	const double num = (double)(2 * n);
+	d3 out;
+	out.x = sx / num;
+	out.y = sy / num;
+	out.z = sz / num;
+	return out;
 }
 
 // one HC iteration (hc_a then hc_b) in two-ring form; pout != p.  LDS rows
 // in split form (an (x, y) array and a z array, read as 16 + 8 bytes).
 template <int RB>
-__global__ void __launch_bounds__(RT)
-k_hc_ring(const uint32_t *__restrict__ start, const uint32_t *__restrict__ slots, const uint16_t *__restrict__ roff,
-          const uint32_t *__restrict__ rslots, const uint32_t *__restrict__ ring, const uint2 *__restrict__ rcnt,
-          const d3 *__restrict__ o, const d3 *__restrict__ o1, const d3 *__restrict__ p, d3 *__restrict__ pout,
-          uint32_t nv, double alpha, double alpha1, double beta, double beta1)
+__global__ void __launch_bounds__(RingCfg<RB>::T, RingCfg<RB>::LARGE ? 8 : 4)
+k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, const uint32_t *__restrict__ rdeg,
+          const uint32_t *__restrict__ rslots, const uint32_t *__restrict__ ring,
+          const uint2 *__restrict__ rcnt, const d3 *__restrict__ o, const d3 *__restrict__ o1,
+          const d3 *__restrict__ p, d3 *__restrict__ pout, uint32_t nv, double alpha, double alpha1, double beta,
+          double beta1)
 {
-	constexpr int W = 2;
+	using Cfg = RingCfg<RB>;
+	constexpr int RT = Cfg::T, RROWS = Cfg::ROWS, RCAP = Cfg::CAP, R1CAP = Cfg::R1CAP;
 	__shared__ double lds[4 * RROWS];
-	constexpr int RCAP = RROWS - RB;
 	const uint32_t blk = blockIdx.x, base = blk * RB, tid = threadIdx.x;
 	const uint2 nn = rcnt[blk];
 	const uint32_t n1 = nn.x, n2 = nn.y;
 	const uint32_t *rg = ring + (size_t)blk * RCAP;
-	const uint16_t *ro = roff + (size_t)blk * ROFFW;
-	const uint32_t *rs = rslots + (size_t)blk * RPCAP;
+	const uint32_t *rd = rdeg + (size_t)blk * R1CAP;
+	const uint32_t *rs = rslots + (size_t)blk * Cfg::PCAP;
 	const d3 *ob = o1 + (size_t)blk * R1CAP; // original positions of ring 1
-	// row tid: a block vertex (tid < RB) or ring-1 vertex tid - RB
+	const uint32_t S1 = Cfg::LARGE ? n1 : (uint32_t)R1CAP;
+	// row tid: a block vertex (tid < RB) or ring-1 vertex tid - RB.  Small
+	// blocks read ring 1's words whatever its size is (they are there).
 	const bool own = tid < RB && base + tid < nv;
-	const bool r1a = tid >= RB && tid - RB < n1;
-	SlotRefs<HK> r;
-	const uint32_t *sl = own ? slots : rs;
-	d3 ov = {0.0, 0.0, 0.0}, pv = {0.0, 0.0, 0.0};
-	{
-		uint32_t gid = 0, b = 0, e = 0;
-		if (own) {
-			gid = base + tid;
-			b = start[gid];
-			e = start[gid + 1];
-		} else if (r1a) {
-			gid = rg[tid - RB];
-			b = ro[tid - RB];
-			e = ro[tid - RB + 1];
-		}
-		r.b = b;
-		r.e = e;
+	const bool r1a = tid >= RB && tid - RB < (Cfg::LARGE ? n1 : (uint32_t)R1CAP);
+	constexpr int NR = Cfg::LARGE ? 1 : (RCAP + RT - 1) / RT;
+	const uint32_t nr = n1 + n2;
+	uint32_t id[NR];
 #pragma unroll
-		for (int k = 0; k < HK; k++)
-			r.q[k] = b + k < e ? sl[b + k] : 0u;
-		if (own)
-			ov = o[gid];
-		else if (r1a)
-			ov = ob[tid - RB];
-		if (own)
-			pv = p[gid];
+	for (int k = 0; k < NR; k++)
+		id[k] = k * RT + tid < (Cfg::LARGE ? nr : (uint32_t)RCAP) ? rg[k * RT + tid] : base;
+	EllRefs r;
+	r.d = 0;
+#pragma unroll
+	for (int k = 0; k < HK; k++)
+		r.q[k] = 0;
+	d3 ov = {0.0, 0.0, 0.0}, pv = {0.0, 0.0, 0.0};
+	// the list of ring-1 vertex i, up to HE; where a list goes on; its pairs
+	// from HE to HK
+	auto ring1 = [&](EllRefs &q, uint32_t i) {
+		q.d = rd[i];
+#pragma unroll
+		for (int k = 0; k < HE; k++)
+			q.q[k] = rs[k * S1 + i];
+	};
+	auto more = [&](const EllRefs &q, bool mine) { return (mine ? (uint32_t)Cfg::RP : HE * S1) + (q.d >> 16); };
+	auto beyond = [&](EllRefs &q, bool mine) {
+		const uint32_t n = q.d & 0xffffu, m = more(q, mine);
+#pragma unroll
+		for (int k = HE; k < HK; k++)
+			q.q[k] = n > (uint32_t)k ? rs[m + (k - HE)] : 0u;
+	};
+	if (own) {
+		const uint32_t *el = ell + (size_t)blk * HE * RB + tid;
+		r.d = deg[base + tid];
+#pragma unroll
+		for (int k = 0; k < HE; k++)
+			r.q[k] = el[k * RB];
+		ov = o[base + tid];
+		pv = p[base + tid];
+	} else if (r1a) {
+		ring1(r, tid - RB);
+		ov = ob[tid - RB];
 	}
-	// stage block (the own rows, already in registers), ring-1 and ring-2
-	// positions
+	// stage ring-1 and ring-2 positions and the block's (the own rows): the
+	// ids were asked for before everything above and the gathers go out before
+	// the own rows are waited for, so that the three latencies overlap
+	d3 v[NR];
+#pragma unroll
+	for (int k = 0; k < NR; k++)
+		if ((k == 0 && !Cfg::LARGE) || k * RT + tid < nr)
+			v[k] = p[id[k]];
+	const bool r1 = r1a && tid - RB < n1;
+	if (own || r1)
+		beyond(r, own);
 	if (tid < RB)
 		lds_put_split<RROWS>(lds, tid, pv);
-	for (uint32_t i = tid; i < n1 + n2; i += RT)
+#pragma unroll
+	for (int k = 0; k < NR; k++)
+		if (k * RT + tid < nr)
+			lds_put_split<RROWS>(lds, RB + k * RT + tid, v[k]);
+	for (uint32_t i = NR * RT + tid; i < nr; i += RT)
 		lds_put_split<RROWS>(lds, RB + i, p[rg[i]]);
 	__syncthreads();
 	const lds_double *L = (const lds_double *)lds;
 	// hc_a on row tid and, for rings longer than RT - RB, on row tid + RT
 	d3 Lp = {0.0, 0.0, 0.0}, bb = {0.0, 0.0, 0.0}, bb2 = {0.0, 0.0, 0.0};
-	if (own || r1a) {
+	if (own || r1) {
 		if (!own)
-			pv = lds_row_w<W, RROWS>(L, tid);
-		Lp = laplace_slots<HK, W, RROWS>(r, sl, L, pv);
+			pv = lds_row_w<2, RROWS>(L, tid);
+		Lp = laplace_ell<RROWS>(r, L, pv, rs, more(r, own));
 		bb.x = Lp.x - (ov.x * alpha + pv.x * alpha1);
 		bb.y = Lp.y - (ov.y * alpha + pv.y * alpha1);
 		bb.z = Lp.z - (ov.z * alpha + pv.z * alpha1);
 	}
 	const uint32_t u2 = tid + RT; // always a ring-1 row (RT >= RB)
 	const bool r2a = u2 - RB < n1;
-	if (r2a) { // its first HK slots are loaded at once
-		SlotRefs<HK> r2;
-		r2.b = ro[u2 - RB];
-		r2.e = ro[u2 - RB + 1];
-#pragma unroll
-		for (int k = 0; k < HK; k++)
-			r2.q[k] = r2.b + k < r2.e ? rs[r2.b + k] : 0u;
+	if (r2a) {
+		EllRefs r2;
+		ring1(r2, u2 - RB);
+		beyond(r2, false);
 		const d3 o2 = ob[u2 - RB];
-		const d3 pv2 = lds_row_w<W, RROWS>(L, u2);
-		const d3 L2 = laplace_slots<HK, W, RROWS>(r2, rs, L, pv2);
+		const d3 pv2 = lds_row_w<2, RROWS>(L, u2);
+		const d3 L2 = laplace_ell<RROWS>(r2, L, pv2, rs, more(r2, false));
 		bb2.x = L2.x - (o2.x * alpha + pv2.x * alpha1);
 		bb2.y = L2.y - (o2.y * alpha + pv2.y * alpha1);
 		bb2.z = L2.z - (o2.z * alpha + pv2.z * alpha1);
 	}
 	__syncthreads(); // every position row has been read
-	if (own || r1a)
+	if (own || r1)
 		lds_put_split<RROWS>(lds, tid, bb);
 	if (r2a)
 		lds_put_split<RROWS>(lds, u2, bb2);
@@ -2011,7 +2101,7 @@ k_hc_ring(const uint32_t *__restrict__ start, const uint32_t *__restrict__ slots
 	if (!own)
 		return;
 	// hc_b on the block's vertices: their pairs reach block and ring 1 only
-	const d3 Lb = laplace_slots<HK, W, RROWS>(r, sl, L, bb);
+	const d3 Lb = laplace_ell<RROWS>(r, L, bb, rs, more(r, true));
 	d3 out;
 	out.x = Lp.x - (bb.x * beta + Lb.x * beta1);
 	out.y = Lp.y - (bb.y * beta + Lb.y * beta1);
@@ -2415,24 +2505,50 @@ void launch_laplace_halo(const uint32_t *start, const uint32_t *slots, const uin
 		hipLaunchKernelGGL(k_laplace_h, dim3(halo_blocks(nv)), dim3(HB), 0, s, start, slots, halo, hcount,
 		                   (const d3 *)p, (d3 *)pout, nv);
 }
-// vertices per two-ring block: N2M_HC_RB = 512, 640 (default) or 768, read
-// by each smoothing call
-int ring_rb()
+// Vertices per two-ring block: N2M_HC_RB (256, 512, 640, 768 or 896), read by
+// each smoothing call, or by the mesh's size.  One iteration, us:
+//
+//   vertices    3.5 k   58 k   92 k  151 k  181 k  369 k  606 k
+//   256          4.9    5.4    7.2    9.0    9.3   15.5   22.5
+//   640          6.7    7.4    7.7    8.5   11.8   17.9   23.3
+//
+// A block of 640 on its own CU is the better one as long as the chip takes all
+// of them at once (256 CUs); small blocks pack it more evenly up to some
+// 700 k; beyond, larger blocks read less ring: the 512^3 pipeline, whose
+// largest mesh has 9.6 M vertices, took 52.9 ms with 256, 49.9 with 640, 49.1
+// with 768 and 48.7 with 896.
+int ring_rb(uint32_t nv)
 {
 	const char *e = getenv("N2M_HC_RB");
-	const int v = e ? atoi(e) : 640;
-	return v == 512 || v == 768 ? v : 640;
+	const int v = e ? atoi(e) : 0;
+	for (int rb : {256, 512, 640, 768, 896})
+		if (v == rb)
+			return rb;
+	if (nv > 650000)
+		return 896;
+	return nv > 120000 && nv <= 256 * 640 ? 640 : 256;
+}
+#define N2M_RING_RBS(X) X(256) X(512) X(640) X(768) X(896)
+struct RingDims {
+	size_t cap, pcap, r1cap;
+};
+static RingDims ring_dims(int rb)
+{
+	switch (rb) {
+#define X(n)                                                                                                       	case n:                                                                                                        		return {(size_t)RingCfg<n>::CAP, (size_t)RingCfg<n>::PCAP, (size_t)RingCfg<n>::R1CAP};
+		N2M_RING_RBS(X)
+#undef X
+	}
+	return {0, 0, 0};
 }
 uint32_t ring_blocks(uint32_t nv, int rb) { return (nv + rb - 1) / rb; }
-size_t ring_words(uint32_t nv, int rb) { return (size_t)ring_blocks(nv, rb) * (RROWS - rb); }
-size_t ring_pair_words(uint32_t nv, int rb) { return (size_t)ring_blocks(nv, rb) * RPCAP; }
-size_t ring_off_words(uint32_t nv, int rb) { return (size_t)ring_blocks(nv, rb) * ROFFW; }
-size_t ring_o_rows(uint32_t nv, int rb) { return (size_t)ring_blocks(nv, rb) * R1CAP; }
-
-#define N2M_RING_RBS(X) X(512) X(640) X(768)
+size_t ring_words(uint32_t nv, int rb) { return ring_blocks(nv, rb) * ring_dims(rb).cap; }
+size_t ring_pair_words(uint32_t nv, int rb) { return ring_blocks(nv, rb) * ring_dims(rb).pcap; }
+size_t ring_ell_words(uint32_t nv, int rb) { return (size_t)ring_blocks(nv, rb) * HE * rb; }
+size_t ring_o_rows(uint32_t nv, int rb) { return ring_blocks(nv, rb) * ring_dims(rb).r1cap; }
 
 void launch_ring_build(const uint32_t *start, const int2 *pairs, uint32_t nv, const double *o, uint32_t *ring,
-                       uint32_t *rcnt, uint32_t *slots, uint16_t *roff, uint32_t *rslots, double *o1,
+                       uint32_t *rcnt, uint32_t *deg, uint32_t *ell, uint32_t *rdeg, uint32_t *rslots, double *o1,
                        uint32_t *overflow, int rbv, hipStream_t s)
 {
 	if (!nv)
@@ -2440,14 +2556,15 @@ void launch_ring_build(const uint32_t *start, const int2 *pairs, uint32_t nv, co
 	switch (rbv) {
 #define X(rb)                                                                                                      \
 	case rb:                                                                                                     \
-		hipLaunchKernelGGL(k_ring_build<rb>, dim3(ring_blocks(nv, rb)), dim3(RT), 0, s, start, pairs, nv,           \
-		                   (const d3 *)o, ring, (uint2 *)rcnt, slots, roff, rslots, (d3 *)o1, overflow);           \
+		hipLaunchKernelGGL(k_ring_build<rb>, dim3(ring_blocks(nv, rb)), dim3(RingCfg<rb>::T), 0, s, start, pairs,  \
+		                   nv, \
+		                   (const d3 *)o, ring, (uint2 *)rcnt, deg, ell, rdeg, rslots, (d3 *)o1, overflow);        \
 		break;
 		N2M_RING_RBS(X)
 #undef X
 	}
 }
-void launch_hc_ring(const uint32_t *start, const uint32_t *slots, const uint16_t *roff, const uint32_t *rslots,
+void launch_hc_ring(const uint32_t *deg, const uint32_t *ell, const uint32_t *rdeg, const uint32_t *rslots,
                     const uint32_t *ring, const uint32_t *rcnt, const double *o, const double *o1, const double *p,
                     double *pout, uint32_t nv, double alpha, double beta, int rbv, hipStream_t s)
 {
@@ -2456,7 +2573,7 @@ void launch_hc_ring(const uint32_t *start, const uint32_t *slots, const uint16_t
 	switch (rbv) {
 #define X(rb)                                                                                                      \
 	case rb:                                                                                                     \
-		hipLaunchKernelGGL(k_hc_ring<rb>, dim3(ring_blocks(nv, rb)), dim3(RT), 0, s, start, slots, roff, rslots, \
+		hipLaunchKernelGGL(k_hc_ring<rb>, dim3(ring_blocks(nv, rb)), dim3(RingCfg<rb>::T), 0, s, deg, ell, rdeg, rslots, \
 		                   ring, (const uint2 *)rcnt, (const d3 *)o, (const d3 *)o1, (const d3 *)p, (d3 *)pout, nv, \
 		                   alpha, 1.0 - alpha, beta, 1.0 - beta);                                                  \
 		break;
@@ -2524,7 +2641,7 @@ __device__ __forceinline__ uint32_t spread10(uint32_t v)
 }
 
 __global__ void k_morton(const double *__restrict__ pts, uint32_t n, const uint32_t *__restrict__ bb,
-                         uint32_t *__restrict__ keys, uint32_t *__restrict__ vals)
+                         int bits, uint32_t *__restrict__ keys, uint32_t *__restrict__ vals)
 {
 	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n)
@@ -2537,7 +2654,7 @@ __global__ void k_morton(const double *__restrict__ pts, uint32_t n, const uint3
 		uint32_t q = f > 0.f ? (f < 1023.f ? (uint32_t)f : 1023u) : 0u; // NaN -> 0
 		key |= spread10(q) << k;
 	}
-	keys[i] = key >> 6; // 8 bits per axis: 24-bit keys, three radix passes
+	keys[i] = key >> (30 - 3 * bits); // `bits` per axis
 	vals[i] = i;
 }
 
@@ -2615,9 +2732,10 @@ void launch_pts_bbox(const double *pts, uint32_t n, uint32_t *bb, hipStream_t s)
 	b = b > 1024 ? 1024 : (b < 1 ? 1 : b);
 	hipLaunchKernelGGL(k_pts_bbox, dim3(b), dim3(256), 0, s, pts, n, bb);
 }
-void launch_morton(const double *pts, uint32_t n, const uint32_t *bb, uint32_t *keys, uint32_t *vals, hipStream_t s)
+void launch_morton(const double *pts, uint32_t n, const uint32_t *bb, int bits, uint32_t *keys, uint32_t *vals,
+                   hipStream_t s)
 {
-	hipLaunchKernelGGL(k_morton, dim3(g1(n)), dim3(256), 0, s, pts, n, bb, keys, vals);
+	hipLaunchKernelGGL(k_morton, dim3(g1(n)), dim3(256), 0, s, pts, n, bb, bits, keys, vals);
 }
 void launch_invert_perm(const uint32_t *perm, uint32_t n, uint32_t *inv, hipStream_t s)
 {

@@ -298,20 +298,20 @@ void launch_hc_b_halo(const uint32_t *start, const uint32_t *slots, const uint32
 void launch_laplace_halo(const uint32_t *start, const uint32_t *slots, const uint32_t *halo,
                          const uint32_t *hcount, const double *p, double *pout, uint32_t nv, hipStream_t s);
 // two-ring form of an HC iteration: per block of rb vertices, ring 1 and ring 2
-// (ring_words, stride 2304 - rb; counts as uint2 in rcnt, 2 words per block), the
-// block's pairs as 16-bit LDS row slots (slots, 3*nt words) and ring 1's pairs
-// (roff: ring_off_words 16-bit offsets, rslots: ring_pair_words words), and
-// ring 1's original positions (o1)
-int ring_rb(); // vertices per block (N2M_HC_RB: 512, 640 or 768)
+// (ring_words; counts as uint2 in rcnt, 2 words per block), the pairs of the
+// block and of ring 1 as 16-bit LDS row slots (ell: ring_ell_words, rslots:
+// ring_pair_words; degrees and list starts in deg, nv words, and rdeg,
+// ring_o_rows words), and ring 1's original positions (o1: ring_o_rows rows)
+int ring_rb(uint32_t nv); // vertices per block for a mesh of nv (N2M_HC_RB: 256, 512, 640, 768 or 896)
 uint32_t ring_blocks(uint32_t nv, int rb);
 size_t ring_words(uint32_t nv, int rb);
 size_t ring_pair_words(uint32_t nv, int rb);
-size_t ring_off_words(uint32_t nv, int rb);
-size_t ring_o_rows(uint32_t nv, int rb); // ring 1's original positions, stride 1024 rows
+size_t ring_ell_words(uint32_t nv, int rb);
+size_t ring_o_rows(uint32_t nv, int rb); // ring 1's original positions
 void launch_ring_build(const uint32_t *start, const int2 *pairs, uint32_t nv, const double *o, uint32_t *ring,
-                       uint32_t *rcnt, uint32_t *slots, uint16_t *roff, uint32_t *rslots, double *o1,
+                       uint32_t *rcnt, uint32_t *deg, uint32_t *ell, uint32_t *rdeg, uint32_t *rslots, double *o1,
                        uint32_t *overflow, int rb, hipStream_t s);
-void launch_hc_ring(const uint32_t *start, const uint32_t *slots, const uint16_t *roff, const uint32_t *rslots,
+void launch_hc_ring(const uint32_t *deg, const uint32_t *ell, const uint32_t *rdeg, const uint32_t *rslots,
                     const uint32_t *ring, const uint32_t *rcnt, const double *o, const double *o1, const double *p,
                     double *pout, uint32_t nv, double alpha, double beta, int rb, hipStream_t s);
 // smoothing state: 3 doubles per vertex, optionally gathered / scattered
@@ -320,7 +320,8 @@ void launch_hc_load(const double *src, const uint32_t *perm, uint32_t n, double 
 void launch_hc_store(const double *p, const double *o, const uint8_t *border, const uint32_t *perm, uint32_t n,
                   double *dst, hipStream_t s);
 void launch_pts_bbox(const double *pts, uint32_t n, uint32_t *bb, hipStream_t s);
-void launch_morton(const double *pts, uint32_t n, const uint32_t *bb, uint32_t *keys, uint32_t *vals,
+// keys of `bits` (at most 10) bits per axis
+void launch_morton(const double *pts, uint32_t n, const uint32_t *bb, int bits, uint32_t *keys, uint32_t *vals,
                    hipStream_t s);
 void launch_invert_perm(const uint32_t *perm, uint32_t n, uint32_t *inv, hipStream_t s);
 void launch_tris_repeat(const int *tris, uint32_t nt, uint32_t *flag, hipStream_t s);

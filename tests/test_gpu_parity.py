@@ -290,7 +290,7 @@ def test_hc_gather_forms(gpu, oracle, monkeypatch, form, iters, lock):
     assert ('hc_a' in stats) == (form != 'ring')
 
 
-@pytest.mark.parametrize('rb', ['512', '640', '768'])
+@pytest.mark.parametrize('rb', ['256', '512', '640', '768', '896'])
 @pytest.mark.parametrize('lock', [True, False])
 def test_hc_ring_block_sizes(gpu, oracle, monkeypatch, rb, lock):
     """The one-launch HC iteration at each block size (N2M_HC_RB) on a noisy
@@ -317,6 +317,36 @@ def test_hc_ring_block_sizes(gpu, oracle, monkeypatch, rb, lock):
     oracle.laplacian_smoothHC(po, to, 0.1, 0.5, 9, lock)
     assert _eq(t, to) and np.array_equal(p, po)
     assert 'hc_ring' in stats and 'hc_a' not in stats
+
+
+@pytest.mark.parametrize('nv', [4095, 4096, 32767, 32768, 120000, 120001, 163841])
+@pytest.mark.parametrize('iters', [2, 24])
+@pytest.mark.parametrize('shuffled', [False, True])
+def test_hc_sizes(gpu, oracle, nv, iters, shuffled):
+    """HC smoothing around the sizes where the renumbering starts (with many
+    and with few iterations) and where the small blocks end, on a torus strip
+    with vertices of degree 3 to 12; shuffled, its blocks' rings overflow
+    wherever it is not renumbered, and the larger forms take over."""
+    rng = np.random.default_rng(nv + iters)
+    w = 61
+    h = nv // w
+    v = np.arange(w * h).reshape(h, w)
+    th, ph = np.meshgrid(np.arange(h) * (2 * np.pi / h), np.arange(w) * (2 * np.pi / w), indexing='ij')
+    pts = np.stack([(40 + 9 * np.cos(ph)) * np.cos(th), (40 + 9 * np.cos(ph)) * np.sin(th), 9 * np.sin(ph)], -1)
+    pts = np.concatenate([pts.reshape(-1, 3), rng.normal(size=(nv - w * h, 3)) * 50])
+    pts += rng.normal(size=pts.shape) * 0.05
+    a, b, c, d = v, np.roll(v, -1, 1), np.roll(v, -1, 0), np.roll(np.roll(v, -1, 0), -1, 1)
+    flip = rng.random(v.shape) < 0.5
+    t1 = np.where(flip[..., None], np.stack([a, b, c], -1), np.stack([a, b, d], -1))
+    t2 = np.where(flip[..., None], np.stack([b, d, c], -1), np.stack([a, d, c], -1))
+    tris = np.concatenate([t1.reshape(-1, 3), t2.reshape(-1, 3)])[w:].astype(np.int32)
+    if shuffled:
+        perm = rng.permutation(nv)
+        pts, tris = pts[np.argsort(perm)], perm[tris].astype(np.int32)
+    p, q = np.ascontiguousarray(pts), np.ascontiguousarray(pts).copy()
+    gpu.lib().laplacian_smoothHC(p, tris, 0.1, 0.5, iters, True)
+    oracle.laplacian_smoothHC(q, np.ascontiguousarray(tris), 0.1, 0.5, iters, True)
+    assert np.array_equal(p, q)
 
 
 @pytest.mark.parametrize('threads,hc_in_worker', [('1', '1'), ('1', '0'), ('0', '0')])
