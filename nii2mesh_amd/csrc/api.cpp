@@ -180,6 +180,7 @@ enum Slot {
 	S_HC_PAIRS,
 	S_HC_BORDER,
 	S_HC_O,
+	S_HC_O32,
 	S_HC_P,
 	S_HC_PN,
 	S_HC_B,
@@ -256,6 +257,7 @@ enum Small {
 	SM_HSTAT = 24, // 3 words
 	SM_PBOX = 32,  // 6 words: float box of vertex positions
 	SM_FLAG = 40,  // 1 word
+	SM_WIDE = 41,  // 1 word: a smoothed coordinate is not a float
 	SM_HALO = 44,  // 1 word: a smoothing block overflowed its halo
 	SM_RING = 45,  // 1 word: a smoothing block overflowed its two rings
 	SM_WNSEG = 48, // 1 word: weld segment count (left on the device)
@@ -1415,7 +1417,7 @@ Ring build_ring(n2m_ctx *C, const Csr &c, uint32_t nv, uint32_t nt, const double
 	r.o1 = C->buf<double>(S_HC_RO, 3 * ring_o_rows(nv, rb));
 	C->tbegin("hc_rings", 8.0 * nv + 12.0 * 3 * nt);
 	launch_ring_build(c.start, c.pairs, nv, o, r.ring, r.rcnt, r.deg, r.ell, r.rdeg, r.rslots, r.o1,
-	                  C->d_small + SM_RING, rb, s);
+	                  C->d_small + SM_RING, C->d_small + SM_WIDE, rb, s);
 	C->tend();
 	return r;
 }
@@ -1439,22 +1441,24 @@ void smooth_hc_device(n2m_ctx *C, double *pts, const int *tris, uint32_t nv, uin
 	const size_t n3 = 3 * (size_t)nv;
 	double *o = C->buf<double>(S_HC_O, n3), *p = C->buf<double>(S_HC_P, n3);
 	double *pn = C->buf<double>(S_HC_PN, n3);
-	launch_hc_load(pts, R.on ? R.perm : nullptr, nv, o, s);
+	float *o32 = iter > 0 ? C->buf<float>(S_HC_O32, n3) : nullptr;
+	C->put(SM_FLAG, {0u, 0u, 0u, 0u, 0u, 0u}); // SM_FLAG .. SM_RING
+	launch_hc_load(pts, R.on ? R.perm : nullptr, nv, o, s, o32, C->d_small + SM_WIDE);
 	// the rings and whether a triangle repeats a vertex (for the border flags)
 	// come back in one round trip; rings that overflowed at another size are
 	// built again with 640 vertices per block, which leaves them the most room
 	const char *er = getenv("N2M_HC_RING");
 	const bool want_ring = iter > 0 && !(er && *er == '0');
 	Ring G;
-	bool repeats = false;
+	bool repeats = false, f32 = false;
 	if (want_ring || lockEdges) {
-		C->put(SM_FLAG, {0u, 0u, 0u, 0u, 0u, 0u});
 		if (want_ring)
 			G = build_ring(C, c, nv, nt, o, ring_rb(nv));
 		if (lockEdges)
 			launch_tris_repeat(tris, nt, C->d_small + SM_FLAG, s);
 		const uint32_t *f = C->fetch(SM_FLAG, SM_RING + 1 - SM_FLAG);
 		repeats = f[0] != 0;
+		f32 = f[SM_WIDE - SM_FLAG] == 0;
 		G.on = want_ring && f[SM_RING - SM_FLAG] == 0;
 		if (want_ring && !G.on && G.rb != 640) {
 			C->put(SM_RING, {0u});
@@ -1471,14 +1475,14 @@ void smooth_hc_device(n2m_ctx *C, double *pts, const int *tris, uint32_t nv, uin
 		(*before_iter)();
 	const double *res = o;
 	if (G.on) {
-		// algorithmic bytes: CSR offsets, one 4-byte slot pair per reference,
-		// the original and current positions in, the new positions out.  The
+		// algorithmic bytes: degrees, one 4-byte slot pair per reference, the
+		// original (12 bytes as floats) and current positions in, the new ones out.  The
 		// iterations are back-to-back launches, timed with one event pair.
-		C->tbegin(stat, (4.0 * nv + 12.0 * nt + 72.0 * nv) * iter);
+		C->tbegin(stat, (4.0 * nv + 12.0 * nt + (f32 ? 60.0 : 72.0) * nv) * iter);
 		for (int it = 0; it < iter; it++) {
 			double *nxt = it % 2 == 0 ? p : pn;
-			launch_hc_ring(G.deg, G.ell, G.rdeg, G.rslots, G.ring, G.rcnt, o, G.o1, res, nxt, nv, alpha,
-			               beta, G.rb, s);
+			launch_hc_ring(G.deg, G.ell, G.rdeg, G.rslots, G.ring, G.rcnt, f32 ? (const void *)o32 : o, G.o1, f32,
+			               res, nxt, nv, alpha, beta, G.rb, s);
 			res = nxt;
 		}
 		C->tend(iter);

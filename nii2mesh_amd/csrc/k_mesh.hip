@@ -6,6 +6,8 @@
 #include <float.h>
 #include <stdlib.h>
 
+#include <type_traits>
+
 #include "n2m_device.cuh"
 #include "n2m_internal.h"
 
@@ -1243,6 +1245,9 @@ __global__ void k_border(const int *__restrict__ tris, uint32_t nv, const uint32
 struct d3 {
 	double x, y, z;
 };
+struct f3 {
+	float x, y, z;
+};
 
 // Neighbour gathers of the smoothers.  Vertices are in Morton order (see
 // the relabelling below), so a workgroup of B consecutive vertices finds
@@ -1808,7 +1813,7 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
              const d3 *__restrict__ o, uint32_t *__restrict__ ring, uint2 *__restrict__ rcnt,
              uint32_t *__restrict__ deg, uint32_t *__restrict__ ell, uint32_t *__restrict__ rdeg,
              uint32_t *__restrict__ rslots,
-             d3 *__restrict__ o1, uint32_t *__restrict__ overflow)
+             void *__restrict__ o1, uint32_t *__restrict__ overflow, const uint32_t *__restrict__ wide)
 {
 	using Cfg = RingCfg<RB>;
 	constexpr int RT = Cfg::T, RCAP = Cfg::CAP, R1CAP = Cfg::R1CAP;
@@ -1913,7 +1918,11 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 	for (uint32_t i = tid; i < (Cfg::LARGE ? n1 + n2 : (uint32_t)RCAP); i += RT)
 		rg[i] = i < n1 + n2 ? srt[i] : base;
 	if (tid < n1) {
-		o1[(size_t)blk * R1CAP + tid] = ov1;
+		const size_t at = (size_t)blk * R1CAP + tid;
+		if (*wide)
+			reinterpret_cast<d3 *>(o1)[at] = ov1;
+		else
+			reinterpret_cast<f3 *>(o1)[at] = {(float)ov1.x, (float)ov1.y, (float)ov1.z};
 		// a degree of 2^16 has more pairs beyond HE than any block takes
 		rdeg[(size_t)blk * R1CAP + tid] = rd | (poff << 16);
 	}
@@ -1948,6 +1957,12 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 		rs[HE * S1 + poff + (k - HE)] = slot(pairs[hb + k]);
 }
 
+// The originals o and o1 of the iteration are doubles, or, when every coordinate
+// is a float (F32, see k_hc_load), floats.  Marching cubes computes Lewiner
+// vertices in floats, so their meshes take the second form as long as no
+// transform came between: 17 of some 153 bytes per vertex less for an
+// iteration that runs at the rate of a copy (9.6 M vertices:
+// 322 -> 311 us).
 // A vertex's list in the two-ring form: its first HK pairs, its degree | first
 // pair beyond HE << 16.
 struct EllRefs {
@@ -1986,11 +2001,11 @@ __device__ __forceinline__ d3 laplace_ell(const EllRefs &r, const lds_double *L,
 
 // one HC iteration (hc_a then hc_b) in two-ring form; pout != p.  LDS rows
 // in split form (an (x, y) array and a z array, read as 16 + 8 bytes).
-template <int RB>
+template <int RB, bool F32>
 __global__ void __launch_bounds__(RingCfg<RB>::T, RingCfg<RB>::LARGE ? 8 : 4)
 k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, const uint32_t *__restrict__ rdeg,
           const uint32_t *__restrict__ rslots, const uint32_t *__restrict__ ring,
-          const uint2 *__restrict__ rcnt, const d3 *__restrict__ o, const d3 *__restrict__ o1,
+          const uint2 *__restrict__ rcnt, const void *__restrict__ o, const void *__restrict__ o1,
           const d3 *__restrict__ p, d3 *__restrict__ pout, uint32_t nv, double alpha, double alpha1, double beta,
           double beta1)
 {
@@ -2003,7 +2018,7 @@ k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, co
 	const uint32_t *rg = ring + (size_t)blk * RCAP;
 	const uint32_t *rd = rdeg + (size_t)blk * R1CAP;
 	const uint32_t *rs = rslots + (size_t)blk * Cfg::PCAP;
-	const d3 *ob = o1 + (size_t)blk * R1CAP; // original positions of ring 1
+	const size_t ob = (size_t)blk * R1CAP; // first of ring 1's original positions
 	const uint32_t S1 = Cfg::LARGE ? n1 : (uint32_t)R1CAP;
 	// row tid: a block vertex (tid < RB) or ring-1 vertex tid - RB.  Small
 	// blocks read ring 1's words whatever its size is (they are there).
@@ -2020,7 +2035,9 @@ k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, co
 #pragma unroll
 	for (int k = 0; k < HK; k++)
 		r.q[k] = 0;
-	d3 ov = {0.0, 0.0, 0.0}, pv = {0.0, 0.0, 0.0};
+	using orig = typename std::conditional<F32, f3, d3>::type;
+	orig ov = {};
+	d3 pv = {0.0, 0.0, 0.0};
 	// the list of ring-1 vertex i, up to HE; where a list goes on; its pairs
 	// from HE to HK
 	auto ring1 = [&](EllRefs &q, uint32_t i) {
@@ -2042,11 +2059,11 @@ k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, co
 #pragma unroll
 		for (int k = 0; k < HE; k++)
 			r.q[k] = el[k * RB];
-		ov = o[base + tid];
+		ov = ((const orig *)o)[base + tid];
 		pv = p[base + tid];
 	} else if (r1a) {
 		ring1(r, tid - RB);
-		ov = ob[tid - RB];
+		ov = ((const orig *)o1)[ob + tid - RB];
 	}
 	// stage ring-1 and ring-2 positions and the block's (the own rows): the
 	// ids were asked for before everything above and the gathers go out before
@@ -2075,9 +2092,9 @@ k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, co
 		if (!own)
 			pv = lds_row_w<2, RROWS>(L, tid);
 		Lp = laplace_ell<RROWS>(r, L, pv, rs, more(r, own));
-		bb.x = Lp.x - (ov.x * alpha + pv.x * alpha1);
-		bb.y = Lp.y - (ov.y * alpha + pv.y * alpha1);
-		bb.z = Lp.z - (ov.z * alpha + pv.z * alpha1);
+		bb.x = Lp.x - ((double)ov.x * alpha + pv.x * alpha1);
+		bb.y = Lp.y - ((double)ov.y * alpha + pv.y * alpha1);
+		bb.z = Lp.z - ((double)ov.z * alpha + pv.z * alpha1);
 	}
 	const uint32_t u2 = tid + RT; // always a ring-1 row (RT >= RB)
 	const bool r2a = u2 - RB < n1;
@@ -2085,12 +2102,12 @@ k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, co
 		EllRefs r2;
 		ring1(r2, u2 - RB);
 		beyond(r2, false);
-		const d3 o2 = ob[u2 - RB];
+		const orig o2 = ((const orig *)o1)[ob + u2 - RB];
 		const d3 pv2 = lds_row_w<2, RROWS>(L, u2);
 		const d3 L2 = laplace_ell<RROWS>(r2, L, pv2, rs, more(r2, false));
-		bb2.x = L2.x - (o2.x * alpha + pv2.x * alpha1);
-		bb2.y = L2.y - (o2.y * alpha + pv2.y * alpha1);
-		bb2.z = L2.z - (o2.z * alpha + pv2.z * alpha1);
+		bb2.x = L2.x - ((double)o2.x * alpha + pv2.x * alpha1);
+		bb2.y = L2.y - ((double)o2.y * alpha + pv2.y * alpha1);
+		bb2.z = L2.z - ((double)o2.z * alpha + pv2.z * alpha1);
 	}
 	__syncthreads(); // every position row has been read
 	if (own || r1)
@@ -2109,12 +2126,24 @@ k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, co
 	pout[base + tid] = out;
 }
 
-// gather through a permutation: dst[i] = src[perm ? perm[i] : i]
-__global__ void k_hc_load(const d3 *__restrict__ src, const uint32_t *__restrict__ perm, uint32_t n, d3 *__restrict__ dst)
+// gather through a permutation: dst[i] = src[perm ? perm[i] : i].  dst32 (when
+// given): the same as floats, and *wide is raised if a coordinate is not one
+__global__ void k_hc_load(const d3 *__restrict__ src, const uint32_t *__restrict__ perm, uint32_t n,
+                          d3 *__restrict__ dst, f3 *__restrict__ dst32, uint32_t *__restrict__ wide)
 {
 	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n)
-		dst[i] = src[perm ? perm[i] : i];
+	bool w = false;
+	if (i < n) {
+		const d3 v = src[perm ? perm[i] : i];
+		dst[i] = v;
+		if (dst32) {
+			const f3 f = {(float)v.x, (float)v.y, (float)v.z};
+			dst32[i] = f;
+			w = !((double)f.x == v.x && (double)f.y == v.y && (double)f.z == v.z);
+		}
+	}
+	if (dst32 && __ballot(w) && lane_id() == 0 && !ld_agent(wide)) // most waves find it raised
+		atomicOr(wide, 1u);
 }
 
 // final HC positions (border vertices keep the original), scattered back
@@ -2549,7 +2578,7 @@ size_t ring_o_rows(uint32_t nv, int rb) { return ring_blocks(nv, rb) * ring_dims
 
 void launch_ring_build(const uint32_t *start, const int2 *pairs, uint32_t nv, const double *o, uint32_t *ring,
                        uint32_t *rcnt, uint32_t *deg, uint32_t *ell, uint32_t *rdeg, uint32_t *rslots, double *o1,
-                       uint32_t *overflow, int rbv, hipStream_t s)
+                       uint32_t *overflow, const uint32_t *wide, int rbv, hipStream_t s)
 {
 	if (!nv)
 		return;
@@ -2558,33 +2587,34 @@ void launch_ring_build(const uint32_t *start, const int2 *pairs, uint32_t nv, co
 	case rb:                                                                                                     \
 		hipLaunchKernelGGL(k_ring_build<rb>, dim3(ring_blocks(nv, rb)), dim3(RingCfg<rb>::T), 0, s, start, pairs,  \
 		                   nv, \
-		                   (const d3 *)o, ring, (uint2 *)rcnt, deg, ell, rdeg, rslots, (d3 *)o1, overflow);        \
+		                   (const d3 *)o, ring, (uint2 *)rcnt, deg, ell, rdeg, rslots, o1, overflow, wide);        \
 		break;
 		N2M_RING_RBS(X)
 #undef X
 	}
 }
 void launch_hc_ring(const uint32_t *deg, const uint32_t *ell, const uint32_t *rdeg, const uint32_t *rslots,
-                    const uint32_t *ring, const uint32_t *rcnt, const double *o, const double *o1, const double *p,
-                    double *pout, uint32_t nv, double alpha, double beta, int rbv, hipStream_t s)
+                    const uint32_t *ring, const uint32_t *rcnt, const void *o, const void *o1, bool f32,
+                    const double *p, double *pout, uint32_t nv, double alpha, double beta, int rbv, hipStream_t s)
 {
 	if (!nv)
 		return;
 	switch (rbv) {
 #define X(rb)                                                                                                      \
 	case rb:                                                                                                     \
-		hipLaunchKernelGGL(k_hc_ring<rb>, dim3(ring_blocks(nv, rb)), dim3(RingCfg<rb>::T), 0, s, deg, ell, rdeg, rslots, \
-		                   ring, (const uint2 *)rcnt, (const d3 *)o, (const d3 *)o1, (const d3 *)p, (d3 *)pout, nv, \
-		                   alpha, 1.0 - alpha, beta, 1.0 - beta);                                                  \
+		hipLaunchKernelGGL((f32 ? k_hc_ring<rb, true> : k_hc_ring<rb, false>), dim3(ring_blocks(nv, rb)),         \
+		                   dim3(RingCfg<rb>::T), 0, s, deg, ell, rdeg, rslots, ring, (const uint2 *)rcnt, o, o1,  \
+		                   (const d3 *)p, (d3 *)pout, nv, alpha, 1.0 - alpha, beta, 1.0 - beta);                  \
 		break;
 		N2M_RING_RBS(X)
 #undef X
 	}
 }
 
-void launch_hc_load(const double *src, const uint32_t *perm, uint32_t n, double *dst, hipStream_t s)
+void launch_hc_load(const double *src, const uint32_t *perm, uint32_t n, double *dst, hipStream_t s, float *dst32,
+                    uint32_t *wide)
 {
-	hipLaunchKernelGGL(k_hc_load, dim3(g1(n)), dim3(256), 0, s, (const d3 *)src, perm, n, (d3 *)dst);
+	hipLaunchKernelGGL(k_hc_load, dim3(g1(n)), dim3(256), 0, s, (const d3 *)src, perm, n, (d3 *)dst, (f3 *)dst32, wide);
 }
 void launch_hc_store(const double *p, const double *o, const uint8_t *border, const uint32_t *perm, uint32_t n,
                   double *dst, hipStream_t s)

@@ -301,7 +301,8 @@ void launch_laplace_halo(const uint32_t *start, const uint32_t *slots, const uin
 // (ring_words; counts as uint2 in rcnt, 2 words per block), the pairs of the
 // block and of ring 1 as 16-bit LDS row slots (ell: ring_ell_words, rslots:
 // ring_pair_words; degrees and list starts in deg, nv words, and rdeg,
-// ring_o_rows words), and ring 1's original positions (o1: ring_o_rows rows)
+// ring_o_rows words), and ring 1's original positions (o1: ring_o_rows rows, of
+// floats when *wide is 0).  f32: o and o1 hold floats
 int ring_rb(uint32_t nv); // vertices per block for a mesh of nv (N2M_HC_RB: 256, 512, 640, 768 or 896)
 uint32_t ring_blocks(uint32_t nv, int rb);
 size_t ring_words(uint32_t nv, int rb);
@@ -310,13 +311,16 @@ size_t ring_ell_words(uint32_t nv, int rb);
 size_t ring_o_rows(uint32_t nv, int rb); // ring 1's original positions
 void launch_ring_build(const uint32_t *start, const int2 *pairs, uint32_t nv, const double *o, uint32_t *ring,
                        uint32_t *rcnt, uint32_t *deg, uint32_t *ell, uint32_t *rdeg, uint32_t *rslots, double *o1,
-                       uint32_t *overflow, int rb, hipStream_t s);
+                       uint32_t *overflow, const uint32_t *wide, int rb, hipStream_t s);
 void launch_hc_ring(const uint32_t *deg, const uint32_t *ell, const uint32_t *rdeg, const uint32_t *rslots,
-                    const uint32_t *ring, const uint32_t *rcnt, const double *o, const double *o1, const double *p,
-                    double *pout, uint32_t nv, double alpha, double beta, int rb, hipStream_t s);
+                    const uint32_t *ring, const uint32_t *rcnt, const void *o, const void *o1, bool f32,
+                    const double *p, double *pout, uint32_t nv, double alpha, double beta, int rb, hipStream_t s);
 // smoothing state: 3 doubles per vertex, optionally gathered / scattered
 // through a vertex permutation
-void launch_hc_load(const double *src, const uint32_t *perm, uint32_t n, double *dst, hipStream_t s);
+// dst32 (when given) receives the positions as floats, and *wide is raised if
+// a coordinate is not one
+void launch_hc_load(const double *src, const uint32_t *perm, uint32_t n, double *dst, hipStream_t s,
+                    float *dst32 = nullptr, uint32_t *wide = nullptr);
 void launch_hc_store(const double *p, const double *o, const uint8_t *border, const uint32_t *perm, uint32_t n,
                   double *dst, hipStream_t s);
 void launch_pts_bbox(const double *pts, uint32_t n, uint32_t *bb, hipStream_t s);

@@ -349,6 +349,25 @@ def test_hc_sizes(gpu, oracle, nv, iters, shuffled):
     assert np.array_equal(p, q)
 
 
+@pytest.mark.parametrize('wide', [None, 0, 63, 64, -1])
+def test_hc_float_originals(gpu, oracle, wide):
+    """HC with originals that are all floats (kept as floats by the one-launch
+    form) and with one vertex that is not, at the ends and wave borders; a
+    NaN or infinite coordinate is kept as a double too."""
+    img = support.blobs((40, 44, 48), 3, noise=2.0)
+    rc, tris, pts = oracle.meshify(img, float(np.percentile(img, 60)), True, False, False, cubes=1)
+    assert rc == 0 and np.array_equal(pts, pts.astype(np.float32).astype(np.float64))
+    odd = [1e-9] if wide is None else [1e-9, np.inf, np.nan]
+    for d in odd:
+        a = pts.copy()
+        if wide is not None:
+            a[wide, 1] += d
+        b = a.copy()
+        gpu.lib().laplacian_smoothHC(a, tris, 0.1, 0.5, 7, False)
+        oracle.laplacian_smoothHC(b, tris, 0.1, 0.5, 7, False)
+        assert support.nan_eq(a, b)
+
+
 @pytest.mark.parametrize('threads,hc_in_worker', [('1', '1'), ('1', '0'), ('0', '0')])
 @pytest.mark.parametrize('cubes', [0, 1])
 def test_pipeline_isolevels(gpu, oracle, monkeypatch, threads, hc_in_worker, cubes):
