@@ -760,7 +760,7 @@ struct VolOut {
 	int lo[3], hi[3];
 	float vmin; // min of the final volume (Lewiner padding)
 	// the apply stage's Lewiner sign bits of the final volume (null when not
-	// written): lw_clamp(v - iso) > 0 / < 0, ceil(nx / 32) words per row
+	// written): lw_clamp(v - iso) > 0 / < 0, bit j <-> voxel j
 	const uint32_t *sgp = nullptr, *sgn = nullptr;
 };
 
@@ -858,7 +858,7 @@ bool volume_stages(n2m_ctx *C, float *vol, const int dim[3], const n2m_params &P
 	// apply + edge darken + bounding box, src/meshify.c:332-371
 	uint32_t *sgp = nullptr, *sgn = nullptr;
 	if (P.cubes == N2M_CUBES_LEWINER) { // the sign bits the classify pass reads
-		const size_t sw = (size_t)((NX + 31) / 32) * NY * NZ;
+		const size_t sw = (nvox + 31) / 32;
 		sgp = C->buf<uint32_t>(S_SIGNP, sw);
 		sgn = C->buf<uint32_t>(S_SIGNN, sw);
 	}

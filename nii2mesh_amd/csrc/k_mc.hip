@@ -556,7 +556,7 @@ k_lw_classify(const float *__restrict__ img, LwGeo g, uint8_t *__restrict__ pfla
 
 // The whole-volume pass from sign bits.  P / N hold the bits
 // lw_clamp(v - iso) > 0 and < 0 of every voxel in linear order (the apply
-// stage writes them; rows of whole 32-voxel words).  A wave takes a chunk of
+// stage writes them).  A wave takes a chunk of
 // 64 points of a row as 64-bit words: the three crossing masks
 // (c0 < 0 ? c1 > 0 : c1 < 0, NaN-exact with the two bits) and the mask of
 // cubes with corners on both sides come from a few word operations; only
@@ -564,7 +564,8 @@ k_lw_classify(const float *__restrict__ img, LwGeo g, uint8_t *__restrict__ pfla
 // depends on face or interior tests read the eight corner values.
 struct SignBits {
 	const uint32_t *P, *N;
-	size_t nwords;         // words of each array (nx * ny * nz / 32)
+	size_t nwords;         // words of each array
+	uint32_t tail;         // the bits of the last word that are voxels
 	uint32_t padP, padN;   // a padding word (the signs of mnv, lw_clamp applied)
 	int nx;
 	long long nxy;
@@ -576,8 +577,12 @@ struct SignBits {
 		const long long j = (long long)g.lo0 + x + (long long)(y + g.lo1) * nx + (long long)(z + g.lo2) * nxy;
 		const size_t w = (size_t)(j >> 5);
 		const int sh = (int)(j & 31);
-		const uint32_t w0 = w < nwords ? a[w] : pad, w1 = w + 1 < nwords ? a[w + 1] : pad,
-		               w2 = w + 2 < nwords ? a[w + 2] : pad;
+		uint32_t w0 = w < nwords ? a[w] : pad, w1 = w + 1 < nwords ? a[w + 1] : pad, w2 = w + 2 < nwords ? a[w + 2] : pad;
+		if (w + 3 >= nwords) { // the last word is among them
+			w0 = w + 1 == nwords ? (w0 & tail) | (pad & ~tail) : w0;
+			w1 = w + 2 == nwords ? (w1 & tail) | (pad & ~tail) : w1;
+			w2 = w + 3 == nwords ? (w2 & tail) | (pad & ~tail) : w2;
+		}
 		const unsigned long long lo = (unsigned long long)w0 | ((unsigned long long)w1 << 32);
 		b64 = (w2 >> sh) & 1u;
 		return sh ? (lo >> sh) | ((unsigned long long)w2 << (64 - sh)) : lo;
@@ -1200,7 +1205,9 @@ void launch_lw_classify_bits(const float *img, int nx, int ny, int nz, const int
 	SignBits sb;
 	sb.P = P;
 	sb.N = N;
-	sb.nwords = (size_t)nx * ny * nz / 32; // nx % 32 == 0
+	const size_t nvox = (size_t)nx * ny * nz;
+	sb.nwords = (nvox + 31) / 32;
+	sb.tail = nvox % 32 ? (1u << (nvox % 32)) - 1u : 0xffffffffu;
 	sb.nx = nx;
 	sb.nxy = (long long)nx * ny;
 	const float m = fabsf(mnv) < FLT_EPSILON ? FLT_EPSILON : mnv; // lw_clamp

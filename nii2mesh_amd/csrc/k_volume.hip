@@ -653,9 +653,9 @@ void launch_minmax(const float *img, size_t n, uint32_t *range, hipStream_t s)
 }
 
 // ---------------------------------------------------------------------------
-// Threshold mask bits: bit = (img >= iso) (or img != 0 when `nonzero`).
-// A workgroup walks whole rows (the row index is uniform, so no per-voxel
-// division); one wave covers 64 consecutive x of a row, padded to 64.
+// Threshold mask bits: bit = (img >= iso) (or img != 0 when `nonzero`), the
+// masks of all isolevels of `iso` in one read, mask k to bits + k * iso.nwords.
+// range / only_moved: see launch_mask_bits (one isolevel).
 // ---------------------------------------------------------------------------
 // the isolevel of a mask (launch_mask_bits); false: the mask stays
 __device__ __forceinline__ bool mask_iso(const uint32_t *range, int only_moved, float &iso)
@@ -667,32 +667,45 @@ __device__ __forceinline__ bool mask_iso(const uint32_t *range, int only_moved, 
 	return atlas_iso(iso, ord2f(range[0]), ord2f(range[1]), &iso, &edgeMax, &moved) && (moved || !only_moved);
 }
 
+// Any row length: a wave takes 64 consecutive voxels of a row (an item; the
+// items of a row are ceil(nx / 64)), MB_IN items in flight.  245 x 347 x 275,
+// three isolevels: 130 us in three passes of one workgroup per row, 49 so.
+constexpr int MB_IN = 4;
 __global__ void __launch_bounds__(256)
-k_mask_bits(const float *__restrict__ img, int nx, int ny, int nz, int W, int xpad, float iso,
-            int nonzero, uint32_t *__restrict__ bits, const uint32_t *__restrict__ range, int only_moved)
+k_mask_bits(const float *__restrict__ img, int nx, size_t rows, int W, IsoMasks iso, int nonzero,
+            uint32_t *__restrict__ bits, const uint32_t *__restrict__ range, int only_moved)
 {
-	if (!mask_iso(range, only_moved, iso))
+	float iso0 = iso.v[0]; // the others stay among the arguments
+	if (!mask_iso(range, only_moved, iso0))
 		return;
-	const size_t rows = (size_t)ny * nz;
-	for (size_t row = blockIdx.x; row < rows; row += gridDim.x) {
-		const float *src = img + row * nx;
-		uint32_t *dst = bits + (size_t)W * row;
-		for (int x0 = 0; x0 < xpad; x0 += blockDim.x) {
-			const int x = x0 + threadIdx.x;
-			if (x - (int)lane_id() >= xpad)
-				break; // whole waves past the padded row (xpad is a multiple of 64)
-			bool p = false;
-			if (x < nx) {
-				const float v = src[x];
-				p = nonzero ? (v != 0.0f) : (v >= iso);
+	const int lane = lane_id(), nch = (nx + N2M_WAVE - 1) / N2M_WAVE;
+	const size_t items = rows * nch, step = (size_t)gridDim.x * (256 / N2M_WAVE) * MB_IN;
+	for (size_t it = ((size_t)blockIdx.x * (256 / N2M_WAVE) + wave_id()) * MB_IN; it < items; it += step) {
+		size_t row = it / nch;
+		int ch = (int)(it - row * nch);
+		float v[MB_IN];
+		bool in[MB_IN];
+		size_t wi[MB_IN];
+		int w1[MB_IN]; // words of the item inside the row
+#pragma unroll
+		for (int k = 0; k < MB_IN; k++) {
+			const int x = ch * N2M_WAVE + lane;
+			in[k] = it + k < items && x < nx;
+			v[k] = in[k] ? img[row * nx + x] : 0.f;
+			wi[k] = row * W + 2 * ch;
+			w1[k] = it + k < items ? (2 * ch + 1 < W ? 2 : 1) : 0;
+			if (++ch == nch) {
+				ch = 0;
+				row++;
 			}
-			const unsigned long long m = __ballot(p);
-			const int wx = (x & ~63) / 32;
-			if ((x & 63) == 0)
-				dst[wx] = (uint32_t)m;
-			else if ((x & 63) == 32 && wx + 1 < W)
-				dst[wx + 1] = (uint32_t)(m >> 32);
 		}
+#pragma unroll
+		for (int k = 0; k < MB_IN; k++)
+			for (int q = 0; q < iso.n; q++) {
+				const unsigned long long m = __ballot(in[k] && (nonzero ? v[k] != 0.0f : v[k] >= (q ? iso.v[q] : iso0)));
+				if (lane < w1[k])
+					bits[q * iso.nwords + wi[k] + lane] = (uint32_t)(lane ? m >> 32 : m);
+			}
 	}
 }
 
@@ -701,43 +714,12 @@ k_mask_bits(const float *__restrict__ img, int nx, int ny, int nz, int W, int xp
 // rows per pass) or fill whole passes of it.  A lane tests 4 voxels; 8
 // neighbouring lanes OR their nibbles into a word.
 __global__ void __launch_bounds__(256)
-k_mask_bits4(const float *__restrict__ img, int nx, int ny, int nz, int W, float iso, int nonzero,
+k_mask_bits4(const float *__restrict__ img, int nx, size_t rows, int W, IsoMasks iso, int nonzero,
              uint32_t *__restrict__ bits, const uint32_t *__restrict__ range, int only_moved)
 {
-	if (!mask_iso(range, only_moved, iso))
+	float iso0 = iso.v[0]; // the others stay among the arguments
+	if (!mask_iso(range, only_moved, iso0))
 		return;
-	const size_t rows = (size_t)ny * nz;
-	const int lpr = nx >> 2, span = lpr < (int)blockDim.x ? lpr : (int)blockDim.x;
-	const int rpi = (int)blockDim.x / span, sub = threadIdx.x / span, q0 = threadIdx.x % span;
-	for (size_t row0 = (size_t)blockIdx.x * rpi; row0 < rows; row0 += (size_t)gridDim.x * rpi) {
-		const size_t row = row0 + sub;
-		const bool live = sub < rpi && row < rows;
-		for (int q = q0; q < lpr; q += span) { // the same trip count on every lane
-			uint32_t nib = 0;
-			if (live) {
-				const float4 v = reinterpret_cast<const float4 *>(img + row * nx)[q];
-				if (nonzero)
-					nib = (v.x != 0.0f) | (v.y != 0.0f) << 1 | (v.z != 0.0f) << 2 | (v.w != 0.0f) << 3;
-				else
-					nib = (v.x >= iso) | (v.y >= iso) << 1 | (v.z >= iso) << 2 | (v.w >= iso) << 3;
-			}
-			uint32_t wv = nib << (4 * (q & 7));
-			wv |= __shfl_xor(wv, 1, N2M_WAVE);
-			wv |= __shfl_xor(wv, 2, N2M_WAVE);
-			wv |= __shfl_xor(wv, 4, N2M_WAVE);
-			if (live && (q & 7) == 0)
-				bits[(size_t)W * row + (q >> 3)] = wv;
-		}
-	}
-}
-
-// The masks of several isolevels in one read of the volume (same layout
-// and conditions as k_mask_bits4): mask k to bits + k * iso.nwords.
-__global__ void __launch_bounds__(256)
-k_mask_bits4_multi(const float *__restrict__ img, int nx, int ny, int nz, int W, IsoMasks iso,
-                   uint32_t *__restrict__ bits)
-{
-	const size_t rows = (size_t)ny * nz;
 	const int lpr = nx >> 2, span = lpr < (int)blockDim.x ? lpr : (int)blockDim.x;
 	const int rpi = (int)blockDim.x / span, sub = threadIdx.x / span, q0 = threadIdx.x % span;
 	for (size_t row0 = (size_t)blockIdx.x * rpi; row0 < rows; row0 += (size_t)gridDim.x * rpi) {
@@ -748,9 +730,11 @@ k_mask_bits4_multi(const float *__restrict__ img, int nx, int ny, int nz, int W,
 			if (live)
 				v = reinterpret_cast<const float4 *>(img + row * nx)[q];
 			for (int k = 0; k < iso.n; k++) {
-				const float t = iso.v[k];
+				const float t = k ? iso.v[k] : iso0;
 				uint32_t nib = 0;
-				if (live)
+				if (live && nonzero)
+					nib = (v.x != 0.0f) | (v.y != 0.0f) << 1 | (v.z != 0.0f) << 2 | (v.w != 0.0f) << 3;
+				else if (live)
 					nib = (v.x >= t) | (v.y >= t) << 1 | (v.z >= t) << 2 | (v.w >= t) << 3;
 				uint32_t wv = nib << (4 * (q & 7));
 				wv |= __shfl_xor(wv, 1, N2M_WAVE);
@@ -765,40 +749,46 @@ k_mask_bits4_multi(const float *__restrict__ img, int nx, int ny, int nz, int W,
 
 static unsigned row_blocks(size_t rows) { return (unsigned)(rows < 8192 ? (rows ? rows : 1) : 8192); }
 
+static void mask_pass(const float *img, int nx, int ny, int nz, const IsoMasks &m, int nonzero, uint32_t *bits,
+                      const uint32_t *range, int only_moved, hipStream_t s)
+{
+	const int W = (nx + 31) / 32, lpr = nx / 4;
+	const size_t rows = (size_t)ny * nz;
+	// a pass that nearly always has nothing to do is launched small
+	const unsigned most = only_moved ? 512 : 4096;
+	if (nx % 32 == 0 && (reinterpret_cast<uintptr_t>(img) & 15u) == 0 && (lpr <= 256 || lpr % 256 == 0)) {
+		const size_t rpi = lpr < 256 ? 256 / lpr : 1;
+		const unsigned nb = row_blocks((rows + rpi - 1) / rpi);
+		hipLaunchKernelGGL(k_mask_bits4, dim3(only_moved && nb > most ? most : nb), dim3(256), 0, s, img, nx, rows, W, m,
+		                   nonzero, bits, range, only_moved);
+	} else {
+		const size_t items = rows * ((nx + N2M_WAVE - 1) / N2M_WAVE), per = 256 / N2M_WAVE * MB_IN;
+		const size_t nb = (items + per - 1) / per;
+		hipLaunchKernelGGL(k_mask_bits, dim3((unsigned)(nb < most ? (nb ? nb : 1) : most)), dim3(256), 0, s, img, nx,
+		                   rows, W, m, nonzero, bits, range, only_moved);
+	}
+}
+
 void launch_mask_bits_multi(const float *img, int nx, int ny, int nz, const float *isos, int n, uint32_t *bits,
                             hipStream_t s)
 {
-	const int W = (nx + 31) / 32, lpr = nx / 4;
-	const size_t nwords = (size_t)W * ny * nz;
-	if (n <= N2M_SMOOTH_MASKS && nx % 32 == 0 && (reinterpret_cast<uintptr_t>(img) & 15u) == 0 &&
-	    (lpr <= 256 || lpr % 256 == 0)) {
-		IsoMasks m{};
-		m.n = n;
-		for (int k = 0; k < n; k++)
-			m.v[k] = isos[k];
-		m.nwords = nwords;
-		const size_t rows = (size_t)ny * nz, rpi = lpr < 256 ? 256 / lpr : 1;
-		hipLaunchKernelGGL(k_mask_bits4_multi, dim3(row_blocks((rows + rpi - 1) / rpi)), dim3(256), 0, s, img, nx,
-		                   ny, nz, W, m, bits);
-		return;
+	IsoMasks m{};
+	m.nwords = (size_t)((nx + 31) / 32) * ny * nz;
+	for (int k0 = 0; k0 < n; k0 += N2M_SMOOTH_MASKS) {
+		m.n = n - k0 < N2M_SMOOTH_MASKS ? n - k0 : N2M_SMOOTH_MASKS;
+		for (int k = 0; k < m.n; k++)
+			m.v[k] = isos[k0 + k];
+		mask_pass(img, nx, ny, nz, m, 0, bits + k0 * m.nwords, nullptr, 0, s);
 	}
-	for (int k = 0; k < n; k++)
-		launch_mask_bits(img, nx, ny, nz, isos[k], 0, bits + k * nwords, s);
 }
 
 void launch_mask_bits(const float *img, int nx, int ny, int nz, float iso, int nonzero, uint32_t *bits,
                       hipStream_t s, const uint32_t *range, bool only_moved)
 {
-	int W = (nx + 31) / 32, xpad = (nx + 63) / 64 * 64;
-	const int lpr = nx / 4;
-	if (nx % 32 == 0 && (reinterpret_cast<uintptr_t>(img) & 15u) == 0 && (lpr <= 256 || lpr % 256 == 0)) {
-		const size_t rows = (size_t)ny * nz, rpi = lpr < 256 ? 256 / lpr : 1;
-		hipLaunchKernelGGL(k_mask_bits4, dim3(row_blocks((rows + rpi - 1) / rpi)), dim3(256), 0, s, img, nx, ny,
-		                   nz, W, iso, nonzero, bits, range, only_moved ? 1 : 0);
-		return;
-	}
-	hipLaunchKernelGGL(k_mask_bits, dim3(row_blocks((size_t)ny * nz)), dim3(256), 0, s, img, nx, ny, nz, W, xpad,
-	                   iso, nonzero, bits, range, only_moved ? 1 : 0);
+	IsoMasks m{};
+	m.n = 1;
+	m.v[0] = iso;
+	mask_pass(img, nx, ny, nz, m, nonzero, bits, range, only_moved ? 1 : 0, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -873,26 +863,38 @@ void launch_dilate_bits(const uint32_t *in, uint32_t *out, int nx, int ny, int n
 // 5.6 for the small launch, which takes the place of a copy.
 constexpr int AP_WORDS = 7, AP_MAXWG = 1024;
 
-__global__ void __launch_bounds__(256)
-k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, float iso, float mn,
-        float edgeMax, const uint32_t *__restrict__ keep, const uint32_t *__restrict__ dil, int fill,
-        const uint32_t *__restrict__ range, uint32_t *__restrict__ part, uint32_t *__restrict__ sgp,
-        uint32_t *__restrict__ sgn)
-{
-	__shared__ int s_red[6][4];
-	__shared__ uint32_t s_min[4];
-	if (range) {
-		bool moved;
-		mn = ord2f(range[0]);
-		if (!atlas_iso(iso, mn, ord2f(range[1]), &iso, &edgeMax, &moved))
-			return;
+// Division of 32-bit numbers by a fixed one (multiply and shift; the method of
+// Granlund and Montgomery, "Division by invariant integers using
+// multiplication", 1994)
+struct FixedDiv {
+	uint32_t m, s1, s2;
+	explicit FixedDiv(uint32_t d)
+	{
+		uint32_t l = 0;
+		while (l < 32 && (1ull << l) < d)
+			l++;
+		m = (uint32_t)(((1ull << 32) * ((1ull << l) - d)) / d + 1);
+		s1 = l < 1 ? l : 1;
+		s2 = l > 1 ? l - 1 : 0;
 	}
+	__device__ uint32_t operator()(uint32_t n) const
+	{
+		const uint32_t t = __umulhi(m, n);
+		return (t + ((n - t) >> s1)) >> s2;
+	}
+};
+
+// What the apply stage does to one voxel, and the box and minimum it keeps.
+// kw / dw: the keep / dilated-mask words that hold bit x & 31.
+struct ApplyVoxel {
+	float iso, mn, edgeMax;
+	int nx;
+	bool k_on, d_on;
 	float lmin = __builtin_inff();
 	int bmin[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff}, bmax[3] = {-1, -1, -1};
-	const size_t rows = (size_t)ny * nz;
-	// one voxel: kw / dw are the keep / dilated-mask words holding bit x & 31
-	auto voxel = [&](int x, int y, int z, bool face_row, float val, uint32_t kw, uint32_t dw, bool k_on,
-	                 bool d_on) -> float {
+
+	__device__ __forceinline__ float operator()(int x, int y, int z, bool face_row, float val, uint32_t kw, uint32_t dw)
+	{
 		if (k_on && ((kw >> (x & 31)) & 1u))
 			val = (float)fmax((double)val, (double)iso);
 		if (d_on && !((dw >> (x & 31)) & 1u))
@@ -909,11 +911,84 @@ k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, f
 			val = fminf(edgeMax, val);
 		lmin = fminf(lmin, val);
 		return val;
-	};
+	}
+
+	// the workgroup's box and minimum to its column of part
+	__device__ __forceinline__ void store(uint32_t *__restrict__ part)
+	{
+		__shared__ int s_red[6][4];
+		__shared__ uint32_t s_min[4];
+		for (int k = 0; k < 3; k++) {
+			bmin[k] = wave_min_i32(bmin[k]);
+			bmax[k] = wave_max_i32(bmax[k]);
+		}
+		const uint32_t om = wave_min_u32(f2ord(lmin));
+		if (lane_id() == 0) {
+			for (int k = 0; k < 3; k++) {
+				s_red[k][wave_id()] = bmin[k];
+				s_red[3 + k][wave_id()] = bmax[k];
+			}
+			s_min[wave_id()] = om;
+		}
+		__syncthreads();
+		if (threadIdx.x < 6) {
+			const int k = threadIdx.x;
+			int r = s_red[k][0];
+			for (int w = 1; w < 4; w++)
+				r = k < 3 ? min(r, s_red[k][w]) : max(r, s_red[k][w]);
+			part[k * AP_MAXWG + blockIdx.x] = (uint32_t)r;
+		}
+		if (threadIdx.x == 6)
+			part[6 * AP_MAXWG + blockIdx.x] = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
+	}
+};
+
+// the sign bits of 4 voxels of the Lewiner data lw_clamp(v - iso), whose 8
+// lanes (lane & 7 = part) together hold a word; lane 0 of them writes it
+__device__ __forceinline__ void apply_signs(const float (&vv)[4], int nlive, float iso, int part, size_t word, bool write,
+                                            uint32_t *__restrict__ sgp, uint32_t *__restrict__ sgn)
+{
+	uint32_t bp = 0, bn = 0;
+#pragma unroll
+	for (int u = 0; u < 4; u++) {
+		float d = vv[u] - iso;
+		d = fabsf(d) < FLT_EPSILON ? FLT_EPSILON : d;
+		bp |= (uint32_t)(u < nlive && d > 0.f) << u;
+		bn |= (uint32_t)(u < nlive && d < 0.f) << u;
+	}
+	bp <<= 4 * part;
+	bn <<= 4 * part;
+#pragma unroll
+	for (int m = 1; m < 8; m <<= 1) {
+		bp |= __shfl_xor(bp, m);
+		bn |= __shfl_xor(bn, m);
+	}
+	if (write && part == 0) {
+		sgp[word] = bp;
+		sgn[word] = bn;
+	}
+}
+
+// row by row; vec4: 16-byte loads and stores (rows of nx = 4 * lpr voxels).
+// sgp / sgn (vec4, nx % 32 == 0): the sign bits.
+__global__ void __launch_bounds__(256)
+k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, float iso, float mn,
+        float edgeMax, const uint32_t *__restrict__ keep, const uint32_t *__restrict__ dil, int fill,
+        const uint32_t *__restrict__ range, uint32_t *__restrict__ part, uint32_t *__restrict__ sgp,
+        uint32_t *__restrict__ sgn)
+{
+	if (range) {
+		bool moved;
+		mn = ord2f(range[0]);
+		if (!atlas_iso(iso, mn, ord2f(range[1]), &iso, &edgeMax, &moved))
+			return;
+	}
+	const size_t rows = (size_t)ny * nz;
 	const bool k_on = fill && keep, d_on = dil != nullptr;
+	ApplyVoxel voxel{iso, mn, edgeMax, nx, k_on, d_on};
 	if (vec4) {
-		// 16-byte loads and stores; rows of nx = 4 * lpr voxels, several rows
-		// per pass when a row has fewer 16-byte chunks than the workgroup
+		// several rows per pass when a row has fewer 16-byte chunks than the
+		// workgroup has threads
 		const int lpr = nx >> 2, span = lpr < (int)blockDim.x ? lpr : (int)blockDim.x;
 		const int rpi = (int)blockDim.x / span, sub = threadIdx.x / span, q0 = threadIdx.x % span;
 		for (size_t row0 = (size_t)blockIdx.x * rpi; row0 < rows; row0 += (size_t)gridDim.x * rpi) {
@@ -928,38 +1003,17 @@ k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, f
 				const int x = 4 * q;
 				const uint32_t kw = k_on ? keep[(size_t)W * row + (x >> 5)] : 0u;
 				const uint32_t dw = d_on ? dil[(size_t)W * row + (x >> 5)] : 0u;
-				float4 v = in[q];
-				v.x = voxel(x, y, z, face_row, v.x, kw, dw, k_on, d_on);
-				v.y = voxel(x + 1, y, z, face_row, v.y, kw, dw, k_on, d_on);
-				v.z = voxel(x + 2, y, z, face_row, v.z, kw, dw, k_on, d_on);
-				v.w = voxel(x + 3, y, z, face_row, v.w, kw, dw, k_on, d_on);
-				line[q] = v;
-				if (sgp) {
-					// sign bits of the Lewiner data lw_clamp(v - iso): the 8
-					// lanes of an aligned group hold one 32-voxel word of the
-					// row (nx % 32 == 0 and the span a multiple of 8, so the
-					// group shares its row and its trip count)
-					const float vv[4] = {v.x, v.y, v.z, v.w};
-					uint32_t bp = 0, bn = 0;
+				const float4 v = in[q];
+				float vv[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-					for (int u = 0; u < 4; u++) {
-						float d = vv[u] - iso;
-						d = fabsf(d) < FLT_EPSILON ? FLT_EPSILON : d;
-						bp |= (uint32_t)(d > 0.f) << u;
-						bn |= (uint32_t)(d < 0.f) << u;
-					}
-					bp <<= 4 * (q & 7);
-					bn <<= 4 * (q & 7);
-#pragma unroll
-					for (int m = 1; m < 8; m <<= 1) {
-						bp |= __shfl_xor(bp, m);
-						bn |= __shfl_xor(bn, m);
-					}
-					if ((q & 7) == 0) {
-						sgp[(size_t)W * row + (x >> 5)] = bp;
-						sgn[(size_t)W * row + (x >> 5)] = bn;
-					}
-				}
+				for (int u = 0; u < 4; u++)
+					vv[u] = voxel(x + u, y, z, face_row, vv[u], kw, dw);
+				line[q] = make_float4(vv[0], vv[1], vv[2], vv[3]);
+				// the 8 lanes of an aligned group hold one 32-voxel word of the
+				// row (nx % 32 == 0 and the span a multiple of 8, so the group
+				// shares its row and its trip count)
+				if (sgp)
+					apply_signs(vv, 4, iso, q & 7, (size_t)W * row + (x >> 5), true, sgp, sgn);
 			}
 		}
 	} else {
@@ -972,32 +1026,77 @@ k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, f
 			for (int x = threadIdx.x; x < nx; x += blockDim.x) {
 				const uint32_t kw = k_on ? keep[(size_t)W * row + (x >> 5)] : 0u;
 				const uint32_t dw = d_on ? dil[(size_t)W * row + (x >> 5)] : 0u;
-				line[x] = voxel(x, y, z, face_row, in[x], kw, dw, k_on, d_on);
+				line[x] = voxel(x, y, z, face_row, in[x], kw, dw);
 			}
 		}
 	}
-	for (int k = 0; k < 3; k++) {
-		bmin[k] = wave_min_i32(bmin[k]);
-		bmax[k] = wave_max_i32(bmax[k]);
+	voxel.store(part);
+}
+
+// The same in linear voxel order, for rows of any length: 16-byte loads and
+// stores, 4 voxels per thread wherever its rows begin, so that the sign bits
+// come out as the classify pass reads them (bit j of the arrays <-> voxel j)
+// and rows of odd length need no other classify.  142 x 178 x 142: apply 24 ->
+// 15 us, classify (from the values before) 35 -> 20.
+__global__ void __launch_bounds__(256)
+k_apply_linear(const float *src, float *img, int nx, int ny, int nz, uint32_t nvox, FixedDiv by_nx, FixedDiv by_ny, int W,
+               float iso, float mn, float edgeMax, const uint32_t *__restrict__ keep,
+               const uint32_t *__restrict__ dil, int fill, const uint32_t *__restrict__ range,
+               uint32_t *__restrict__ part, uint32_t *__restrict__ sgp, uint32_t *__restrict__ sgn)
+{
+	if (range) {
+		bool moved;
+		mn = ord2f(range[0]);
+		if (!atlas_iso(iso, mn, ord2f(range[1]), &iso, &edgeMax, &moved))
+			return;
 	}
-	uint32_t om = wave_min_u32(f2ord(lmin));
-	if (lane_id() == 0) {
-		for (int k = 0; k < 3; k++) {
-			s_red[k][wave_id()] = bmin[k];
-			s_red[3 + k][wave_id()] = bmax[k];
+	const bool k_on = fill && keep, d_on = dil != nullptr;
+	ApplyVoxel voxel{iso, mn, edgeMax, nx, k_on, d_on};
+	const uint32_t nq = (uint32_t)(((unsigned long long)nvox + 31) / 32 * 8); // whole groups of 8 lanes
+	for (uint32_t q = blockIdx.x * 256 + threadIdx.x; q < nq; q += gridDim.x * 256) {
+		const uint32_t v0 = 4 * q;
+		const int nlive = v0 >= nvox ? 0 : (nvox - v0 < 4 ? (int)(nvox - v0) : 4);
+		float vv[4] = {0.f, 0.f, 0.f, 0.f};
+		if (nlive == 4) {
+			const float4 f = reinterpret_cast<const float4 *>(src)[q];
+			vv[0] = f.x;
+			vv[1] = f.y;
+			vv[2] = f.z;
+			vv[3] = f.w;
+		} else {
+			for (int u = 0; u < nlive; u++)
+				vv[u] = src[v0 + u];
 		}
-		s_min[wave_id()] = om;
+		uint32_t row = by_nx(v0);
+		int x = (int)(v0 - row * (uint32_t)nx), z = (int)by_ny(row), y = (int)(row - (uint32_t)z * (uint32_t)ny);
+		uint32_t kw = 0, dw = 0;
+#pragma unroll
+		for (int u = 0; u < 4; u++) {
+			if (u < nlive) {
+				if (u == 0 || (x & 31) == 0) {
+					kw = k_on ? keep[(size_t)W * row + (x >> 5)] : 0u;
+					dw = d_on ? dil[(size_t)W * row + (x >> 5)] : 0u;
+				}
+				vv[u] = voxel(x, y, z, y == 0 || z == 0 || y == ny - 1 || z == nz - 1, vv[u], kw, dw);
+				if (++x == nx) {
+					x = 0;
+					row++;
+					if (++y == ny) {
+						y = 0;
+						z++;
+					}
+				}
+			}
+		}
+		if (nlive == 4)
+			reinterpret_cast<float4 *>(img)[q] = make_float4(vv[0], vv[1], vv[2], vv[3]);
+		else
+			for (int u = 0; u < nlive; u++)
+				img[v0 + u] = vv[u];
+		if (sgp)
+			apply_signs(vv, nlive, iso, q & 7, q >> 3, true, sgp, sgn);
 	}
-	__syncthreads();
-	if (threadIdx.x < 6) {
-		int k = threadIdx.x;
-		int r = s_red[k][0];
-		for (int w = 1; w < 4; w++)
-			r = k < 3 ? min(r, s_red[k][w]) : max(r, s_red[k][w]);
-		part[k * AP_MAXWG + blockIdx.x] = (uint32_t)r;
-	}
-	if (threadIdx.x == 6)
-		part[6 * AP_MAXWG + blockIdx.x] = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
+	voxel.store(part);
 }
 
 // the workgroups' partial boxes and minima to host[0..6], the range to
@@ -1037,27 +1136,31 @@ k_apply_box(const uint32_t *__restrict__ part, int nwg, int nx, int ny, int nz, 
 
 size_t apply_part_words() { return (size_t)AP_WORDS * AP_MAXWG; }
 
-bool apply_sign_bits_ok(const float *src, const float *img, int nx)
-{
-	const float *in = src ? src : img;
-	return nx % 32 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(img)) & 15u) == 0;
-}
-
 bool launch_apply(const float *src, float *img, int nx, int ny, int nz, float iso, float mn, float edgeMax,
                   const uint32_t *keep, const uint32_t *dil, int fill, const uint32_t *range, uint32_t *part,
                   uint32_t *host, hipStream_t s, uint32_t *sgp, uint32_t *sgn)
 {
 	const int W = (nx + 31) / 32;
 	const float *in = src ? src : img;
-	const bool vec4 = nx % 4 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(img)) & 15u) == 0;
-	if (!sgp || !sgn || !apply_sign_bits_ok(src, img, nx))
+	const size_t rows = (size_t)ny * nz, nvox = rows * nx;
+	const bool aligned = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(img)) & 15u) == 0;
+	// by rows where that gives whole words and vectors (or no sign bits are
+	// asked for), in linear order otherwise, by single voxels where the
+	// volumes are not aligned or have 2^32 voxels
+	const bool vec4 = aligned && nx % 4 == 0 && (!sgp || nx % 32 == 0);
+	const bool linear = aligned && !vec4 && nvox < 0xffffffe0ull;
+	if (!vec4 && !linear)
 		sgp = sgn = nullptr;
-	const size_t rows = (size_t)ny * nz;
 	const size_t rpi = vec4 && nx / 4 < 256 ? 256 / (nx / 4) : 1;
-	const size_t items = (rows + rpi - 1) / rpi;
+	const size_t items = linear ? (nvox + 1023) / 1024 : (rows + rpi - 1) / rpi;
 	const unsigned nwg = (unsigned)(items < (size_t)AP_MAXWG ? (items ? items : 1) : (size_t)AP_MAXWG);
-	hipLaunchKernelGGL(k_apply, dim3(nwg), dim3(256), 0, s, in, img, nx, ny, nz, W, vec4 ? 1 : 0, iso, mn, edgeMax,
-	                   keep, dil, fill, range, part, sgp, sgn);
+	if (linear)
+		hipLaunchKernelGGL(k_apply_linear, dim3(nwg), dim3(256), 0, s, in, img, nx, ny, nz, (uint32_t)nvox,
+		                   FixedDiv((uint32_t)nx), FixedDiv((uint32_t)ny), W, iso, mn, edgeMax, keep, dil, fill, range,
+		                   part, sgp, sgn);
+	else
+		hipLaunchKernelGGL(k_apply, dim3(nwg), dim3(256), 0, s, in, img, nx, ny, nz, W, vec4 ? 1 : 0, iso, mn, edgeMax,
+		                   keep, dil, fill, range, part, sgp, sgn);
 	hipLaunchKernelGGL(k_apply_box, dim3(1), dim3(AP_MAXWG), 0, s, (const uint32_t *)part, (int)nwg, nx, ny, nz,
 	                   range, host);
 	return sgp != nullptr;

@@ -102,9 +102,9 @@ void launch_dilate_bits(const uint32_t *in, uint32_t *out, int nx, int ny, int n
 // (atlas_iso); without variability nothing is written at all.  part: apply_part_words()
 // words of scratch.  host: 9 words the device can write (pinned): box, ordered
 // minimum of the result, and the range words (when given).
-// sgp / sgn (when given and nx % 32 == 0 with 16-byte aligned volumes):
-// the Lewiner sign bits of the result, lw_clamp(v - iso) > 0 / < 0, ceil(nx
-// / 32) words per row; returns whether they were written
+// sgp / sgn (when given, and the volumes are 16-byte aligned and of fewer than
+// some 2^32 voxels): the Lewiner sign bits of the result, lw_clamp(v - iso) >
+// 0 / < 0, bit j <-> voxel j; returns whether they were written
 bool launch_apply(const float *src, float *img, int nx, int ny, int nz, float iso, float mn, float edgeMax,
                   const uint32_t *keep, const uint32_t *dil, int fill, const uint32_t *range, uint32_t *part,
                   uint32_t *host, hipStream_t s, uint32_t *sgp = nullptr, uint32_t *sgn = nullptr);
@@ -173,7 +173,7 @@ size_t lw_nseg_total(int nx, int ny, int nz, const int lo[3], const int hi[3]);
 // each), or, when fmask is given, to per-axis bit masks (lw_fmask_words
 // words); tiling rows to crow, segment counts to segcnt
 // launch_lw_classify (fmask form) from the sign bits the apply stage wrote
-// (P: lw_clamp(v - iso) > 0, N: < 0; per volume row, ceil(nx / 32) words)
+// (P: lw_clamp(v - iso) > 0, N: < 0; bit j <-> voxel j)
 void launch_lw_classify_bits(const float *img, int nx, int ny, int nz, const int lo[3], const int hi[3], float iso,
                              float mnv, int originalMC, const uint32_t *P, const uint32_t *N, uint16_t *crow,
                              uint32_t *segcnt, unsigned long long *fmask, hipStream_t s);

@@ -520,14 +520,16 @@ def _sign_bits_volume(kind, shape, seed):
     return img, float(np.float32(np.nanpercentile(img, 60)))
 
 
-@pytest.mark.parametrize('shape', [(9, 11, 32), (20, 23, 64), (14, 18, 96)])
+@pytest.mark.parametrize('shape', [(9, 11, 32), (20, 23, 64), (14, 18, 96), (8, 9, 31), (9, 11, 33), (10, 9, 36),
+                                   (20, 23, 45), (5, 7, 130), (30, 33, 127)])
 @pytest.mark.parametrize('kind', ['blobs', 'face', 'ties', 'nan'])
 @pytest.mark.parametrize('flags', [(True, True, True), (False, False, False), (True, False, True)])
 @pytest.mark.parametrize('o1', [0, 1])
 def test_meshify_lewiner_sign_bits(gpu, oracle, shape, kind, flags, o1):
-    """Lewiner meshify on volumes whose rows are whole 32-voxel words, where
-    the classify pass reads the apply stage's sign bits instead of the
-    values: the same meshes and mutated volume as the oracle."""
+    """Lewiner meshify, whose classify pass reads the apply stage's sign bits
+    instead of the values, on volumes whose rows are whole 32-voxel words and
+    on rows of other lengths (written in linear order; the last word is
+    partly padding): the same meshes and mutated volume as the oracle."""
     img, iso = _sign_bits_volume(kind, shape, 30 + shape[2])
     if iso is None:
         iso = float(np.float32(np.percentile(img, 62)))
