@@ -1773,21 +1773,25 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 		nfl += (size_t)t.nx * t.ny * t.nz;
 	}
 	float *crops = C->buf<float>(S_AT_CROPS, nfl);
-	std::vector<uint32_t> bmap;
+	// first workgroup of every task in a launch, and the launch's block map
+	// (filled on the device)
+	size_t nmap = 0;
 	auto plan = [&](auto blocks_of) {
-		bmap.clear();
+		nmap = 0;
 		for (size_t k = 0; k < T.size(); k++) {
-			T[k].first_block = (int)bmap.size();
-			bmap.insert(bmap.end(), (size_t)blocks_of(T[k]), (uint32_t)k);
+			T[k].first_block = (int)nmap;
+			nmap += (size_t)blocks_of(T[k]);
+			if (nmap >= ((size_t)1 << 31))
+				fail("atlas launch of %zu workgroups", nmap);
 		}
-		if (bmap.size() >= ((size_t)1 << 31))
-			fail("atlas launch of %zu workgroups", bmap.size());
-		upload(C, C->buf<AtlasTask>(S_AT_TASKS, T.size()), T);
-		upload(C, C->buf<uint32_t>(S_AT_BMAP, bmap.size()), bmap);
-		return (unsigned)bmap.size();
+		AtlasTask *d = C->buf<AtlasTask>(S_AT_TASKS, T.size());
+		upload(C, d, T);
+		launch_atlas_bmap(d, (int)T.size(), (uint32_t)nmap, C->buf<uint32_t>(S_AT_BMAP, nmap), s);
+		C->check();
+		return (unsigned)nmap;
 	};
 	auto dT = [&] { return C->buf<AtlasTask>(S_AT_TASKS, T.size()); };
-	auto dmap = [&] { return C->buf<uint32_t>(S_AT_BMAP, bmap.size()); };
+	auto dmap = [&] { return C->buf<uint32_t>(S_AT_BMAP, nmap); };
 
 	// 1. binarise + pre-smooth every crop, per-task range (src/meshify.c:299-311)
 	uint32_t *red = C->buf<uint32_t>(S_AT_RED, (size_t)9 * T.size());

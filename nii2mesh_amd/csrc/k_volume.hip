@@ -445,7 +445,11 @@ void launch_atlas_smooth(const float *labels, int gnx, int gny, int gnz, const A
 }
 
 // darken the voxels on the volume's faces, bounding box of >= iso and the
-// minimum of the result, per task (src/meshify.c:347-371)
+// minimum of the result, per task (src/meshify.c:347-371).  Bound by its reads
+// once a workgroup takes enough voxels: with 4 per thread, a division for
+// each and the workgroups' box atomics four times as many, 370 crops with
+// 20.3 M voxels took 198 us, 16 per thread 58.
+constexpr int AA_VPT = 16;
 __device__ __forceinline__ void atlas_apply_item(float *__restrict__ crops, int gnx, int gny, int gnz,
                                                  const AtlasTask *__restrict__ tasks,
                                                  const uint32_t *__restrict__ blockTask, unsigned b,
@@ -460,26 +464,51 @@ __device__ __forceinline__ void atlas_apply_item(float *__restrict__ crops, int 
 	float lmin = __builtin_inff();
 	int bmin[3] = {0x7fffffff, 0x7fffffff, 0x7fffffff}, bmax[3] = {-1, -1, -1};
 	float *img = crops + t.off;
-	for (int k = 0; k < 4; k++) {
-		size_t v = ((size_t)local * 4 + k) * 256 + threadIdx.x;
-		if (v >= n)
-			break;
-		const int x = (int)(v % t.nx), y = (int)((v / t.nx) % t.ny), z = (int)(v / ((size_t)t.nx * t.ny));
-		float val = img[v];
-		if (val >= t.iso) {
-			bmin[0] = min(bmin[0], x);
-			bmax[0] = max(bmax[0], x);
-			bmin[1] = min(bmin[1], y);
-			bmax[1] = max(bmax[1], y);
-			bmin[2] = min(bmin[2], z);
-			bmax[2] = max(bmax[2], z);
+	// AA_VPT voxels per thread, the workgroup's threads side by side; the
+	// coordinates are divided out once and stepped from there
+	const size_t v0 = (size_t)local * AA_VPT * 256 + threadIdx.x;
+	const int dx = 256 % t.nx, sy = 256 / t.nx, dy = sy % t.ny, dz = sy / t.ny;
+	const size_t r0 = v0 / t.nx;
+	int x = (int)(v0 - r0 * t.nx), y = (int)(r0 % t.ny), z = (int)(r0 / t.ny);
+	for (int k0 = 0; k0 < AA_VPT; k0 += 8) {
+		float in[8];
+#pragma unroll
+		for (int k = 0; k < 8; k++) {
+			const size_t v = v0 + (size_t)(k0 + k) * 256;
+			in[k] = v < n ? img[v] : 0.f;
 		}
-		const int gx = t.ox + x, gy = t.oy + y, gz = t.oz + z;
-		if (gx == 0 || gy == 0 || gz == 0 || gx == gnx - 1 || gy == gny - 1 || gz == gnz - 1) {
-			val = fminf(t.edgeMax, val);
-			img[v] = val;
+#pragma unroll
+		for (int k = 0; k < 8; k++) {
+			const size_t v = v0 + (size_t)(k0 + k) * 256;
+			if (v < n) {
+				float val = in[k];
+				if (val >= t.iso) {
+					bmin[0] = min(bmin[0], x);
+					bmax[0] = max(bmax[0], x);
+					bmin[1] = min(bmin[1], y);
+					bmax[1] = max(bmax[1], y);
+					bmin[2] = min(bmin[2], z);
+					bmax[2] = max(bmax[2], z);
+				}
+				const int gx = t.ox + x, gy = t.oy + y, gz = t.oz + z;
+				if (gx == 0 || gy == 0 || gz == 0 || gx == gnx - 1 || gy == gny - 1 || gz == gnz - 1) {
+					val = fminf(t.edgeMax, val);
+					img[v] = val;
+				}
+				lmin = fminf(lmin, val);
+			}
+			x += dx;
+			y += dy;
+			z += dz;
+			if (x >= t.nx) {
+				x -= t.nx;
+				y++;
+			}
+			if (y >= t.ny) {
+				y -= t.ny;
+				z++;
+			}
 		}
-		lmin = fminf(lmin, val);
 	}
 	for (int k = 0; k < 3; k++) {
 		bmin[k] = wave_min_i32(bmin[k]);
@@ -607,20 +636,22 @@ void launch_put(uint32_t *dst, const PutWords &w, int n, hipStream_t s)
 // ---------------------------------------------------------------------------
 // Intensity range without smoothing (src/meshify.c:306-311).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
+constexpr int MM_BS = 1024, MM_WGS = 256;
+__global__ void __launch_bounds__(MM_BS)
 k_minmax(const float *__restrict__ img, size_t n, int vec4, uint32_t *range)
 {
-	__shared__ uint32_t s_red[2][4];
+	constexpr int NW = MM_BS / N2M_WAVE;
+	__shared__ uint32_t s_red[2][NW];
 	float lmin = __builtin_inff(), lmax = -__builtin_inff();
-	size_t n4 = vec4 ? n / 4 : 0;
+	const size_t n4 = vec4 ? n / 4 : 0, tid = blockIdx.x * (size_t)MM_BS + threadIdx.x, step = (size_t)gridDim.x * MM_BS;
 	const float4 *v4 = reinterpret_cast<const float4 *>(img);
-	for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n4; i += (size_t)gridDim.x * blockDim.x) {
-		float4 v = v4[i];
+#pragma unroll 4
+	for (size_t i = tid; i < n4; i += step) {
+		const float4 v = v4[i];
 		lmin = fminf(fminf(lmin, v.x), fminf(v.y, fminf(v.z, v.w)));
 		lmax = fmaxf(fmaxf(lmax, v.x), fmaxf(v.y, fmaxf(v.z, v.w)));
 	}
-	for (size_t i = n4 * 4 + blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
-	     i += (size_t)gridDim.x * blockDim.x) {
+	for (size_t i = n4 * 4 + tid; i < n; i += step) {
 		lmin = fminf(lmin, img[i]);
 		lmax = fmaxf(lmax, img[i]);
 	}
@@ -631,7 +662,7 @@ k_minmax(const float *__restrict__ img, size_t n, int vec4, uint32_t *range)
 	}
 	__syncthreads();
 	if (threadIdx.x == 0) {
-		for (int w = 1; w < 4; w++) {
+		for (int w = 1; w < NW; w++) {
 			omin = min(omin, s_red[0][w]);
 			omax = max(omax, s_red[1][w]);
 		}
@@ -644,12 +675,31 @@ k_minmax(const float *__restrict__ img, size_t n, int vec4, uint32_t *range)
 	}
 }
 
+// one workgroup of 1024 per CU at most, few atomics (256^3: 29 us with 2048 of
+// 256, 20 so)
 void launch_minmax(const float *img, size_t n, uint32_t *range, hipStream_t s)
 {
-	size_t blocks = (n / 4 + 255) / 256;
-	blocks = blocks < 1 ? 1 : (blocks > 2048 ? 2048 : blocks);
+	size_t blocks = (n / 4 + MM_BS - 1) / MM_BS;
+	blocks = blocks < 1 ? 1 : (blocks > (size_t)MM_WGS ? (size_t)MM_WGS : blocks);
 	int vec4 = ((uintptr_t)img & 15) == 0; // float4 loads need 16-byte alignment
-	hipLaunchKernelGGL(k_minmax, dim3((unsigned)blocks), dim3(256), 0, s, img, n, vec4, range);
+	hipLaunchKernelGGL(k_minmax, dim3((unsigned)blocks), dim3(MM_BS), 0, s, img, n, vec4, range);
+}
+
+// the block map of a launch over all tasks: task k's workgroups
+// [tasks[k].first_block, + count[k]) name it
+__global__ void k_atlas_bmap(const AtlasTask *__restrict__ tasks, int ntasks, uint32_t nblocks, uint32_t *__restrict__ bmap)
+{
+	const int k = blockIdx.x;
+	const uint32_t b0 = (uint32_t)tasks[k].first_block,
+	               b1 = k + 1 < ntasks ? (uint32_t)tasks[k + 1].first_block : nblocks;
+	for (uint32_t b = b0 + threadIdx.x; b < b1; b += blockDim.x)
+		bmap[b] = (uint32_t)k;
+}
+
+void launch_atlas_bmap(const AtlasTask *tasks, int ntasks, uint32_t nblocks, uint32_t *bmap, hipStream_t s)
+{
+	if (ntasks)
+		hipLaunchKernelGGL(k_atlas_bmap, dim3(ntasks), dim3(256), 0, s, tasks, ntasks, nblocks, bmap);
 }
 
 // ---------------------------------------------------------------------------
@@ -1297,7 +1347,10 @@ unsigned atlas_smooth_blocks(int nx, int ny, int nz, int smooth, int tile)
 	}
 	return (unsigned)(((size_t)nx * ny * nz + SM_BS - 1) / SM_BS);
 }
-unsigned atlas_apply_blocks(int nx, int ny, int nz) { return (unsigned)(((size_t)nx * ny * nz + 1023) / 1024); }
+unsigned atlas_apply_blocks(int nx, int ny, int nz)
+{
+	return (unsigned)(((size_t)nx * ny * nz + 256 * AA_VPT - 1) / (256 * AA_VPT));
+}
 
 // one label of the per-label loop: out = (lo < v < hi), count of ones
 // (src/nii2mesh.c:553-563)

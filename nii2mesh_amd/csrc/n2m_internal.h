@@ -138,6 +138,8 @@ void launch_atlas_apply(float *crops, int gnx, int gny, int gnz, const AtlasTask
 // iso, mn, edgeMax of every task from its range (ranges[2t], ord min/max),
 // as atlas_iso; a task without variability gets a NaN iso
 void launch_atlas_iso(AtlasTask *tasks, int ntasks, const uint32_t *ranges, float req, hipStream_t s);
+// bmap[b] = the task whose workgroups (from its first_block on) hold b
+void launch_atlas_bmap(const AtlasTask *tasks, int ntasks, uint32_t nblocks, uint32_t *bmap, hipStream_t s);
 unsigned atlas_smooth_blocks(int nx, int ny, int nz, int smooth, int tile);
 unsigned atlas_apply_blocks(int nx, int ny, int nz);
 void launch_binarize(const float *labels, size_t n, float lo, float hi, float *out, uint32_t *count, hipStream_t s);

@@ -243,3 +243,19 @@ def test_atlas_host_entry(gpu, oracle, cubes):
     assert rc == 0
     compare([(s, t, p) for _, s, t, p in res], want)
     assert [lab for lab, _, _, _ in res] == list(range(1, len(want) + 1))
+
+
+# crops at the edges of the darkening stage's 4096-voxel share of a workgroup
+# (x, y and z steps that carry, rows longer than the 256 threads, one voxel
+# over, one short), equal to the oracle bit for bit
+@pytest.mark.parametrize('shape', [(3, 3, 700), (700, 3, 3), (3, 700, 3), (16, 16, 16), (7, 45, 13), (17, 241, 2),
+                                   (15, 273, 3), (9, 5, 300)])
+def test_atlas_crop_shapes(gpu, oracle, shape):
+    nz, ny, nx = shape
+    rng = np.random.default_rng(nx * 1000 + ny)
+    vol = np.ones(shape, np.float32)
+    vol[rng.random(shape) < 0.3] = 2
+    vol[rng.random(shape) < 0.2] = 0
+    for loop in (False, True):
+        got = run_gpu(gpu, vol, 0, 0, True, False, 0, None, loop)
+        compare(got, expect(oracle, vol, 0, 0, True, False, 0, None))
