@@ -162,7 +162,6 @@ enum Slot {
 	S_K1,
 	S_V1,
 	S_RCOUNT,
-	S_FLAGS,
 	S_SEGID,
 	S_STARTS,
 	S_LCLS,
@@ -730,24 +729,23 @@ uint32_t *scan_scratch(n2m_ctx *C, size_t n)
 // round trip for the three totals
 void scan3(n2m_ctx *C, const uint32_t *in, uint32_t *out, size_t n, uint32_t tot[3])
 {
-	uint32_t *scr = scan_scratch(C, n);
-	for (int k = 0; k < 3; k++)
-		scan_excl_u32(in + k * n, out + k * n, n, C->d_small + SM_TOTAL + k, scr, C->stream);
+	const uint32_t *t = C->h_small + SM_TOTAL; // written by the scan itself
+	scan_excl_rows_u32(in, out, n, n, n, 3, C->h_small + SM_TOTAL, scan_scratch(C, n), C->stream);
 	C->check();
-	const uint32_t *t = C->fetch(SM_TOTAL, 3);
+	C->sync();
 	for (int k = 0; k < 3; k++)
 		tot[k] = t[k];
 }
 
 uint32_t scan(n2m_ctx *C, const uint32_t *in, uint32_t *out, size_t n, bool want_total)
 {
-	uint32_t *scr = scan_scratch(C, n);
-	uint32_t *tot = C->d_small + SM_TOTAL;
-	scan_excl_u32(in, out, n, want_total ? tot : nullptr, scr, C->stream);
+	uint32_t *tot = C->h_small + SM_TOTAL;
+	scan_excl_u32(in, out, n, want_total ? tot : nullptr, scan_scratch(C, n), C->stream);
 	C->check();
 	if (!want_total)
 		return 0;
-	return C->fetch(SM_TOTAL, 1)[0];
+	C->sync();
+	return *tot;
 }
 
 // ------------------------------------------------------------------------
@@ -992,17 +990,17 @@ uint32_t weld(n2m_ctx *C, const double *pts, uint32_t npt, const int *tris_in /*
 	bool in1 = radix_sort_u32(k0, v0, k1, v1, npt, 32, rc, scr, s);
 	C->tend();
 	uint32_t *keys = in1 ? k1 : k0, *vals = in1 ? v1 : v0;
-	uint32_t *flags = C->buf<uint32_t>(S_FLAGS, npt), *segid = C->buf<uint32_t>(S_SEGID, npt);
-	C->tbegin("weld_segments", 8.0 * npt);
-	launch_weld_segflags(keys, npt, flags, s);
+	uint32_t *segid = C->buf<uint32_t>(S_SEGID, npt), *starts = C->buf<uint32_t>(S_STARTS, npt);
+	C->tbegin("weld_segments", 12.0 * npt);
+	launch_weld_segments(keys, nullptr, npt, segid, starts, C->h_small + SM_WNSEG, scan_scratch(C, npt), s);
 	C->tend();
-	uint32_t nseg = scan(C, flags, segid, npt, true);
-	uint32_t *starts = C->buf<uint32_t>(S_STARTS, nseg);
+	C->check();
+	C->sync();
+	const uint32_t nseg = C->h_small[SM_WNSEG];
 	int *lcls = C->buf<int>(S_LCLS, npt);
 	uint32_t *seeds = C->buf<uint32_t>(S_SEEDS, nseg), *seedbase = C->buf<uint32_t>(S_SEEDBASE, nseg);
 	uint32_t *lrep = C->buf<uint32_t>(S_LREP, npt);
 	C->tbegin("weld_greedy", 4.0 * npt + 4.0 * npt + 24.0 * npt + 8.0 * npt);
-	launch_weld_segstarts(flags, segid, npt, starts, s);
 	launch_weld_greedy(starts, nseg, npt, keys, vals, pts, lcls, seeds, lrep, s);
 	C->tend();
 	uint32_t nnew = scan(C, seeds, seedbase, nseg, true);
@@ -1020,14 +1018,13 @@ uint32_t weld(n2m_ctx *C, const double *pts, uint32_t npt, const int *tris_in /*
 	}
 	int *cls = C->buf<int>(S_CLS, npt), *rep = C->buf<int>(S_REP, nnew);
 	C->tbegin("weld_assign", 4.0 * npt * 5 + 4.0 * npt + 4.0 * nnew);
-	launch_weld_assign(vals, lcls, flags, segid, seedbase, lrep, npt, cls, rep, s);
+	launch_weld_assign(vals, lcls, segid, seedbase, lrep, npt, cls, rep, s);
 	C->tend();
 	pts_out = C->buf<double>(S_PTS1, (size_t)3 * nnew);
 	if (wpos) {
 		double *wp = C->buf<double>(S_WPOS, (size_t)3 * npt);
-		C->tbegin("weld_gather", 28.0 * nnew + 24.0 * nnew + 8.0 * npt + 24.0 * npt + 24.0 * npt);
-		launch_gather_pts(pts, rep, nnew, pts_out, s);
-		launch_weld_wpos(pts, cls, rep, npt, wp, s);
+		C->tbegin("weld_gather", 24.0 * nnew + 8.0 * npt + 24.0 * npt + 24.0 * npt);
+		launch_weld_wpos(pts, cls, rep, npt, wp, pts_out, s);
 		C->tend();
 		*wpos = wp;
 	} else {
@@ -1105,8 +1102,8 @@ uint32_t remove_degenerate_welded(n2m_ctx *C, const int *tris_in, uint32_t npt, 
 // (npt vertices, nt triangles), the launches cover them and read the counts
 // from the device, and a weld that merges nothing numbers each vertex as
 // itself (the reference's unchanged output).  pts_out / tris_out receive the
-// result arrays; the vertex and triangle counts are left in SM_WNNEW and
-// SM_DEGK, for one copy to the host.  The same kernels and order of
+// result arrays; the last launch leaves the vertex and triangle counts in
+// h_small (SM_WNNEW and SM_DEGK), valid after a sync.  The same kernels and order of
 // operations as weld() and remove_degenerate_welded().
 void weld_clean_deferred(n2m_ctx *C, const double *pts, uint32_t npt, const int *tris_in, uint32_t nt,
                          double *&pts_out, int *&tris_out)
@@ -1123,40 +1120,36 @@ void weld_clean_deferred(n2m_ctx *C, const double *pts, uint32_t npt, const int 
 	bool in1 = radix_sort_u32(k0, v0, k1, v1, npt, 32, rc, scr, s);
 	C->tend();
 	uint32_t *keys = in1 ? k1 : k0, *vals = in1 ? v1 : v0;
-	uint32_t *flags = C->buf<uint32_t>(S_FLAGS, npt), *segid = C->buf<uint32_t>(S_SEGID, npt);
-	uint32_t *d_nseg = C->d_small + SM_WNSEG, *d_nnew = C->d_small + SM_WNNEW, *d_k = C->d_small + SM_DEGK;
-	C->tbegin("weld_segments", 8.0 * npt);
-	launch_weld_segflags(keys, npt, flags, s);
-	scan_excl_u32(flags, segid, npt, d_nseg, scr, s);
+	uint32_t *segid = C->buf<uint32_t>(S_SEGID, npt), *starts = C->buf<uint32_t>(S_STARTS, npt);
+	uint32_t *d_nseg = C->d_small + SM_WNSEG, *d_nnew = C->d_small + SM_WNNEW;
+	C->tbegin("weld_segments", 12.0 * npt);
+	launch_weld_segments(keys, nullptr, npt, segid, starts, d_nseg, scr, s);
 	C->tend();
-	uint32_t *starts = C->buf<uint32_t>(S_STARTS, npt);
 	int *lcls = C->buf<int>(S_LCLS, npt);
 	uint32_t *seeds = C->buf<uint32_t>(S_SEEDS, npt), *seedbase = C->buf<uint32_t>(S_SEEDBASE, npt);
 	uint32_t *lrep = C->buf<uint32_t>(S_LREP, npt);
 	C->tbegin("weld_greedy", 4.0 * npt + 4.0 * npt + 24.0 * npt + 8.0 * npt);
-	launch_weld_segstarts(flags, segid, npt, starts, s);
 	launch_weld_greedy(starts, npt, npt, keys, vals, pts, lcls, seeds, lrep, s, d_nseg);
 	scan_excl_u32(seeds, seedbase, npt, d_nnew, scr, s);
 	C->tend();
 	int *cls = C->buf<int>(S_CLS, npt), *rep = C->buf<int>(S_REP, npt);
 	C->tbegin("weld_assign", 4.0 * npt * 5 + 4.0 * npt + 4.0 * npt);
-	launch_weld_assign(vals, lcls, flags, segid, seedbase, lrep, npt, cls, rep, s, d_nnew);
+	launch_weld_assign(vals, lcls, segid, seedbase, lrep, npt, cls, rep, s, d_nnew);
 	C->tend();
 	pts_out = C->buf<double>(S_PTS1, (size_t)3 * npt);
 	double *wpos = C->buf<double>(S_WPOS, (size_t)3 * npt);
-	C->tbegin("weld_gather", 28.0 * npt + 24.0 * npt + 8.0 * npt + 24.0 * npt + 24.0 * npt);
-	launch_gather_pts(pts, rep, npt, pts_out, s, d_nnew);
-	launch_weld_wpos(pts, cls, rep, npt, wpos, s);
+	C->tbegin("weld_gather", 24.0 * npt + 8.0 * npt + 24.0 * npt + 24.0 * npt);
+	launch_weld_wpos(pts, cls, rep, npt, wpos, pts_out, s);
 	C->tend();
 	int *t1 = C->buf<int>(S_TRIS1, (size_t)3 * (nt ? nt : 1));
 	uint32_t *keep = C->buf<uint32_t>(S_KEEP, nt), *pos = C->buf<uint32_t>(S_KEEPPOS, nt);
 	C->tbegin("degenerate", 12.0 * nt + 12.0 * nt + 72.0 * nt + 4.0 * nt);
 	launch_remap_degen(tris_in, cls, npt, wpos, nt, t1, keep, s);
-	scan_excl_u32(keep, pos, nt, d_k, scan_scratch(C, nt), s);
+	scan_excl_u32(keep, pos, nt, nullptr, scan_scratch(C, nt), s);
 	C->tend();
 	int *out = C->buf<int>(S_TRIS0, (size_t)3 * (nt ? nt : 1));
 	C->tbegin("compact_tris", 12.0 * nt + 12.0 * nt);
-	launch_compact_tris(t1, keep, pos, nt, out, s);
+	launch_compact_tris(t1, keep, pos, nt, out, s, d_nnew, C->h_small + SM_WNNEW);
 	C->tend();
 	tris_out = out;
 }
@@ -1193,7 +1186,9 @@ bool surface_stages(n2m_ctx *C, const float *vol, const int dim[3], const VolOut
 	int *tris = nullptr;
 	if (!P.verbose) { // the counts come back once, at the end
 		weld_clean_deferred(C, pts0, mc.npt, tris0, mc.ntri, pts, tris);
-		const uint32_t *cnt = C->fetch(SM_WNNEW, 2);
+		C->check();
+		C->sync();
+		const uint32_t *cnt = C->h_small + SM_WNNEW;
 		const uint32_t np = cnt[0], nt = cnt[1];
 		if (np < 3) // src/meshify.c:380
 			return false;
@@ -1225,6 +1220,7 @@ bool meshify_device(n2m_ctx *C, const float *src, float *vol, const int dim[3], 
 	hipStream_t s = C->stream;
 	bool have_range = false;
 	uint32_t *spec = nullptr;
+	const float *smoothed = nullptr; // the voxels, where vol does not hold them yet
 	if (P.preSmooth && NX >= 5 && NY >= 5 && NZ >= 5) { // src/meshify.c:299-304
 		double t0 = now_ms();
 		C->put_volume();
@@ -1237,7 +1233,7 @@ bool meshify_device(n2m_ctx *C, const float *src, float *vol, const int dim[3], 
 		launch_smooth(src, out, NX, NY, NZ, C->d_small + SM_RANGE, &P.isolevel, 1, spec, s);
 		C->tend();
 		if (out != vol)
-			HIPX(hipMemcpyAsync(vol, out, 4 * nvox, hipMemcpyDeviceToDevice, s));
+			smoothed = out;
 		have_range = true;
 		if (P.verbose) {
 			C->sync();
@@ -1247,8 +1243,13 @@ bool meshify_device(n2m_ctx *C, const float *src, float *vol, const int dim[3], 
 		HIPX(hipMemcpyAsync(vol, src, 4 * nvox, hipMemcpyDeviceToDevice, s));
 	}
 	VolOut vo;
-	if (!volume_stages(C, vol, dim, P, have_range, spec, vo))
+	if (!volume_stages(C, vol, dim, P, have_range, spec, vo, smoothed)) {
+		if (smoothed) { // vol is left smoothed, whichever stage gave up
+			HIPX(hipMemcpyAsync(vol, smoothed, 4 * nvox, hipMemcpyDeviceToDevice, s));
+			C->sync();
+		}
 		return false;
+	}
 	return surface_stages(C, vol, dim, vo, P, m);
 }
 
@@ -1921,7 +1922,6 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 		});
 		uint8_t *cfg = C->buf<uint8_t>(S_CFG, cubes);
 		uint32_t *bs = C->buf<uint32_t>(S_BLOCK, (size_t)nb + 1), *bo = C->buf<uint32_t>(S_BLOCKOFF, (size_t)nb + 1);
-		HIPX(hipMemsetAsync(bs + nb, 0, 4, s));
 		auto count_with = [&](int k) {
 			launch_atlas_classic_count(crops, dT(), dmap(), nb, atlas_grid(C, nb, k), cfg, bs, s);
 			C->check();
@@ -1930,7 +1930,8 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 		C->tbegin("atlas_mc_classic_count", 4.0 * cubes + cubes);
 		count_with(ccfg);
 		C->tend();
-		scan_excl_u32(bs, bo, (size_t)nb + 1, nullptr, scan_scratch(C, (size_t)nb + 1), s);
+		// nb sums, and the total behind them
+		scan_excl_rows_u32(bs, bo, (size_t)nb + 1, nb, 0, 1, nullptr, scan_scratch(C, (size_t)nb + 1), s);
 		C->check();
 		std::vector<uint32_t> idx(nt_ + 1);
 		for (size_t k = 0; k < nt_; k++)
@@ -1971,8 +1972,6 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 		uint8_t *pf = C->buf<uint8_t>(S_PFLAGS, npts);
 		uint16_t *cr = C->buf<uint16_t>(S_CROW, npts);
 		uint32_t *cnt = C->buf<uint32_t>(S_SEGCNT, 3 * stride), *base = C->buf<uint32_t>(S_SEGBASE, 3 * stride);
-		for (int j = 0; j < 3; j++)
-			HIPX(hipMemsetAsync(cnt + j * stride + nb, 0, 4, s));
 		auto classify_with = [&](int k) {
 			launch_atlas_lw_classify(crops, dT(), dmap(), nb, atlas_grid(C, nb, k), P.originalMC, pf, cr, cnt, stride,
 			                         s);
@@ -1982,8 +1981,7 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 		C->tbegin("atlas_mc_lewiner_classify", 7.0 * npts);
 		classify_with(lcfg);
 		C->tend();
-		for (int j = 0; j < 3; j++)
-			scan_excl_u32(cnt + j * stride, base + j * stride, stride, nullptr, scan_scratch(C, stride), s);
+		scan_excl_rows_u32(cnt, base, stride, nb, stride, 3, nullptr, scan_scratch(C, stride), s);
 		C->check();
 		std::vector<uint32_t> idx(3 * (nt_ + 1));
 		for (int j = 0; j < 3; j++) {
@@ -2039,20 +2037,17 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 	uint32_t *keys = in1 ? k1 : k0, *vals = in1 ? v1 : v0;
 	const uint32_t *TK = vtask;
 	C->tend();
-	uint32_t *flags = C->buf<uint32_t>(S_FLAGS, Vtot), *segid = C->buf<uint32_t>(S_SEGID, Vtot);
-	C->tbegin("atlas_weld_segments", 12.0 * Vtot);
-	launch_atlas_weld_segflags(keys, TK, Vtot, flags, s);
-	C->tend();
 	// The counts stay on the device until one copy at the end: the launches
 	// cover their upper bound Vtot.
 	uint32_t *d_nseg = C->d_small + SM_WNSEG, *d_nnew = C->d_small + SM_WNNEW;
-	scan_excl_u32(flags, segid, Vtot, d_nseg, scr, s);
-	uint32_t *starts = C->buf<uint32_t>(S_STARTS, Vtot);
+	uint32_t *segid = C->buf<uint32_t>(S_SEGID, Vtot), *starts = C->buf<uint32_t>(S_STARTS, Vtot);
+	C->tbegin("atlas_weld_segments", 16.0 * Vtot);
+	launch_weld_segments(keys, TK, Vtot, segid, starts, d_nseg, scr, s);
+	C->tend();
 	int *lcls = C->buf<int>(S_LCLS, Vtot);
 	uint32_t *seeds = C->buf<uint32_t>(S_SEEDS, Vtot), *seedbase = C->buf<uint32_t>(S_SEEDBASE, Vtot);
 	uint32_t *lrep = C->buf<uint32_t>(S_LREP, Vtot);
 	C->tbegin("atlas_weld_greedy", 4.0 * Vtot + 4.0 * Vtot + 24.0 * Vtot + 8.0 * Vtot);
-	launch_weld_segstarts(flags, segid, Vtot, starts, s);
 	launch_weld_greedy(starts, Vtot, Vtot, keys, vals, pts0, lcls, seeds, lrep, s, d_nseg);
 	C->tend();
 	scan_excl_u32(seeds, seedbase, Vtot, d_nnew, scr, s);
@@ -2073,7 +2068,7 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 	int *cls = C->buf<int>(S_CLS, Vtot), *rep = C->buf<int>(S_REP, Vtot);
 	C->tbegin("atlas_weld_assign", 4.0 * Vtot * 6 + 4.0 * Vtot + 4.0 * Vtot);
 	launch_atlas_class_base(TK, segid, seedbase, Vtot, dcb, s);
-	launch_weld_assign(vals, lcls, flags, segid, seedbase, lrep, Vtot, cls, rep, s);
+	launch_weld_assign(vals, lcls, segid, seedbase, lrep, Vtot, cls, rep, s);
 	launch_atlas_weld_tasks(dcb, dvb, dnext, (int)nt_, d_nnew, dncls, di, s);
 	launch_atlas_weld_identity(Vtot, vtask, dvb, dcb, di, cls, rep, s);
 	C->tend();
@@ -2088,12 +2083,11 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 	// 5. degenerate triangles (src/meshify.c:113-168); every class number is
 	// below the class count, so Vtot bounds the vertex ids as well
 	uint32_t *keep = C->buf<uint32_t>(S_KEEP, (size_t)Ttot + 1), *kpos = C->buf<uint32_t>(S_KEEPPOS, (size_t)Ttot + 1);
-	HIPX(hipMemsetAsync(keep + Ttot, 0, 4, s));
 	C->tbegin("atlas_degenerate", 12.0 * Ttot + 72.0 * Ttot + 4.0 * Ttot);
 	if (Ttot)
 		launch_degen_flags(pts1, tris1, Ttot, Vtot, keep, s);
 	C->tend();
-	scan_excl_u32(keep, kpos, (size_t)Ttot + 1, nullptr, scan_scratch(C, (size_t)Ttot + 1), s);
+	scan_excl_rows_u32(keep, kpos, (size_t)Ttot + 1, Ttot, 0, 1, nullptr, scan_scratch(C, (size_t)Ttot + 1), s);
 	uint32_t *dtb = C->buf<uint32_t>(S_AT_IDX, nt_ + 1);
 	upload(C, dtb, tbase);
 	launch_gather_u32(kpos, dtb, (uint32_t)(nt_ + 1), res, s);

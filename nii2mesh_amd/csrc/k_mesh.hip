@@ -19,7 +19,52 @@ namespace n2m {
 // ---------------------------------------------------------------------------
 constexpr int SC_BS = 256, SC_IPT = 8, SC_TILE = SC_BS * SC_IPT;
 
-__global__ void __launch_bounds__(SC_BS) k_scan_reduce(const uint32_t *__restrict__ in, size_t n, uint32_t *sums)
+// What a scan reads (the value at i) and writes (i, the sum before it, the
+// value), so that a pass that only makes or consumes the words runs inside
+// it.  Row r of a batch starts r * stride words on.
+struct ScanWords {
+	const uint32_t *in; // may equal out: a tile is read before it is written
+	uint32_t *out;
+	size_t nin, stride; // values past nin count as 0
+	__device__ uint32_t get(size_t i, uint32_t row) const { return i < nin ? in[row * stride + i] : 0u; }
+	__device__ void put(size_t i, uint32_t row, uint32_t sum, uint32_t) const { out[row * stride + i] = sum; }
+};
+
+// in: a thread's SC_IPT neighbouring values, so that the loads go out together
+template <class OP>
+__device__ __forceinline__ uint32_t scan_load(const OP &op, size_t base, size_t n, uint32_t row, uint32_t *v)
+{
+	uint32_t sum = 0;
+	if (base + SC_IPT <= n) {
+#pragma unroll
+		for (int k = 0; k < SC_IPT; k++)
+			v[k] = op.get(base + k, row);
+	} else {
+#pragma unroll
+		for (int k = 0; k < SC_IPT; k++)
+			v[k] = base + k < n ? op.get(base + k, row) : 0u;
+	}
+#pragma unroll
+	for (int k = 0; k < SC_IPT; k++)
+		sum += v[k];
+	return sum;
+}
+
+template <class OP>
+__device__ __forceinline__ uint32_t scan_store(const OP &op, size_t base, size_t n, uint32_t row, const uint32_t *v,
+                                               uint32_t run)
+{
+#pragma unroll
+	for (int k = 0; k < SC_IPT; k++) {
+		if (base + k < n)
+			op.put(base + k, row, run, v[k]);
+		run += v[k];
+	}
+	return run;
+}
+
+template <class OP>
+__global__ void __launch_bounds__(SC_BS) k_scan_reduce(OP op, size_t n, uint32_t *sums)
 {
 	__shared__ uint32_t scratch[SC_BS / N2M_WAVE + 1];
 	size_t base = blockIdx.x * (size_t)SC_TILE;
@@ -27,49 +72,39 @@ __global__ void __launch_bounds__(SC_BS) k_scan_reduce(const uint32_t *__restric
 	for (int k = 0; k < SC_IPT; k++) {
 		size_t i = base + k * SC_BS + threadIdx.x;
 		if (i < n)
-			s += in[i];
+			s += op.get(i, blockIdx.y);
 	}
 	s = block_sum_u32<SC_BS>(s, scratch);
 	if (threadIdx.x == 0)
-		sums[blockIdx.x] = s;
+		sums[blockIdx.y * (size_t)gridDim.x + blockIdx.x] = s;
 }
 
-__global__ void __launch_bounds__(SC_BS)
-k_scan_apply(const uint32_t *__restrict__ in, uint32_t *__restrict__ out, size_t n, const uint32_t *offs,
-             uint32_t *total)
+// offs: each row's tile sums, scanned (null for one tile); total: a word per row
+template <class OP>
+__global__ void __launch_bounds__(SC_BS) k_scan_apply(OP op, size_t n, const uint32_t *offs, uint32_t *total)
 {
 	__shared__ uint32_t scratch[SC_BS / N2M_WAVE + 1];
-	size_t base = blockIdx.x * (size_t)SC_TILE + (size_t)threadIdx.x * SC_IPT;
-	uint32_t v[SC_IPT], s = 0;
-#pragma unroll
-	for (int k = 0; k < SC_IPT; k++) {
-		size_t i = base + k;
-		v[k] = i < n ? in[i] : 0u;
-		s += v[k];
-	}
-	uint32_t tot;
-	uint32_t run = block_excl_scan<SC_BS>(s, scratch, &tot) + (offs ? offs[blockIdx.x] : 0u);
-#pragma unroll
-	for (int k = 0; k < SC_IPT; k++) {
-		size_t i = base + k;
-		if (i < n)
-			out[i] = run;
-		run += v[k];
-	}
+	const size_t base = blockIdx.x * (size_t)SC_TILE + (size_t)threadIdx.x * SC_IPT;
+	uint32_t v[SC_IPT], tot;
+	uint32_t run = block_excl_scan<SC_BS>(scan_load(op, base, n, blockIdx.y, v), scratch, &tot);
+	run += offs ? offs[blockIdx.y * (size_t)gridDim.x + blockIdx.x] : 0u;
+	run = scan_store(op, base, n, blockIdx.y, v, run);
 	if (total && blockIdx.x == gridDim.x - 1 && threadIdx.x == SC_BS - 1)
-		*total = run;
+		total[blockIdx.y] = run;
 }
 
 // Scans of up to SP_MAX_TILES tiles run in one pass (k_scan_1p); longer ones
 // reduce, scan the partial sums and apply (three launches: there the serial
-// chain of look-backs costs more than the two extra launches).  The first
-// SP_WORDS words of the scratch belong to the single-pass scan: two counters
-// (tickets handed out, workgroups finished), then one 64-bit word per tile
-// (status << 32 | sum).  They are zero between scans: the caller zeroes them
+// chain of look-backs costs more than the two extra launches).  A batch of
+// up to SC_ROWS equally long scans takes the launches of one.  The first
+// SC_ROWS * SP_WORDS words of the scratch belong to the single-pass scan: for
+// each row two counters (tickets handed out, workgroups finished), then one
+// 64-bit word per tile (status << 32 | sum).  They are zero between scans: the caller zeroes them
 // once when the scratch is allocated, and the last workgroup of every
 // single-pass scan clears what that scan used.  The partial sums of the
 // multi-level form follow them.
 constexpr int SP_MAX_TILES = 128, SP_WORDS = 320; // SP_WORDS >= 2 + 2 * SP_MAX_TILES
+constexpr int SC_ROWS = 3;
 static_assert(SP_WORDS >= 2 + 2 * SP_MAX_TILES, "single-pass scan scratch");
 
 size_t scan_scratch_words(size_t n)
@@ -79,9 +114,9 @@ size_t scan_scratch_words(size_t n)
 		n = (n + SC_TILE - 1) / SC_TILE;
 		w += n;
 	}
-	return SP_WORDS + w + 1;
+	return SC_ROWS * (SP_WORDS + w) + 1;
 }
-size_t scan_scratch_zero_words() { return SP_WORDS; }
+size_t scan_scratch_zero_words() { return SC_ROWS * SP_WORDS; }
 
 constexpr uint32_t SP_AGG = 1u, SP_INC = 2u; // tile status: own sum / inclusive prefix
 constexpr uint32_t SP_SPIN_MAX = 1u << 20;   // bound on the polls of one predecessor
@@ -92,11 +127,13 @@ constexpr uint32_t SP_SPIN_MAX = 1u << 20;   // bound on the polls of one predec
 // sums (or the inclusive prefix, where published) of the tiles before it,
 // and publishes its inclusive prefix.  A predecessor's sum is published
 // before that workgroup waits for anything, so every wait ends.
-__global__ void __launch_bounds__(SC_BS)
-k_scan_1p(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t *scr, uint32_t ntiles)
+template <class OP>
+__global__ void __launch_bounds__(SC_BS) k_scan_1p(OP op, size_t n, uint32_t *total, uint32_t *scr, uint32_t ntiles)
 {
 	__shared__ uint32_t scratch[SC_BS / N2M_WAVE + 1];
 	__shared__ uint32_t s_tile, s_prefix, s_last;
+	const uint32_t row = blockIdx.y;
+	scr += row * SP_WORDS;
 	uint32_t *ctr = scr;
 	unsigned long long *flags = reinterpret_cast<unsigned long long *>(scr + 2);
 	if (threadIdx.x == 0)
@@ -104,15 +141,8 @@ k_scan_1p(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t
 	__syncthreads();
 	const uint32_t tile = s_tile;
 	const size_t base = tile * (size_t)SC_TILE + (size_t)threadIdx.x * SC_IPT;
-	uint32_t v[SC_IPT], sum = 0;
-#pragma unroll
-	for (int k = 0; k < SC_IPT; k++) {
-		const size_t i = base + k;
-		v[k] = i < n ? in[i] : 0u;
-		sum += v[k];
-	}
-	uint32_t agg;
-	uint32_t run = block_excl_scan<SC_BS>(sum, scratch, &agg);
+	uint32_t v[SC_IPT], agg;
+	uint32_t run = block_excl_scan<SC_BS>(scan_load(op, base, n, row, v), scratch, &agg);
 	// the look-back, by the first wave: lane l reads the word of tile
 	// j0 - l, so one round trip covers 64 predecessors; it stops at the
 	// nearest tile with an inclusive prefix (tile 0 always has one)
@@ -147,16 +177,9 @@ k_scan_1p(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t
 		}
 	}
 	__syncthreads();
-	run += s_prefix;
-#pragma unroll
-	for (int k = 0; k < SC_IPT; k++) {
-		const size_t i = base + k;
-		if (i < n)
-			out[i] = run;
-		run += v[k];
-	}
+	run = scan_store(op, base, n, row, v, run + s_prefix);
 	if (total && tile == ntiles - 1 && threadIdx.x == SC_BS - 1)
-		*total = run;
+		total[row] = run;
 	// the last workgroup to finish clears the counters and the tile words:
 	// every other one has finished its look-back by then
 	if (threadIdx.x == 0)
@@ -172,7 +195,7 @@ k_scan_1p(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t
 	}
 }
 
-__global__ void k_zero_u32(uint32_t *p) { *p = 0u; }
+__global__ void k_zero_u32(uint32_t *p) { p[threadIdx.x] = 0u; }
 
 // In-place exclusive scan of up to SC_SMALL words by one workgroup: the
 // partial sums level of a scan of up to SC_TILE * SC_SMALL words, in one
@@ -182,6 +205,7 @@ constexpr int SC_SBS = 1024, SC_SIPT = 16, SC_SMALL = SC_SBS * SC_SIPT;
 __global__ void __launch_bounds__(SC_SBS) k_scan_sums(uint32_t *__restrict__ a, uint32_t n)
 {
 	__shared__ uint32_t scratch[SC_SBS / N2M_WAVE + 1];
+	a += blockIdx.x * (size_t)n; // a row per workgroup
 	const uint32_t base = threadIdx.x * SC_SIPT;
 	uint32_t v[SC_SIPT], s = 0;
 #pragma unroll
@@ -199,37 +223,50 @@ __global__ void __launch_bounds__(SC_SBS) k_scan_sums(uint32_t *__restrict__ a, 
 	}
 }
 
-// the multi-level form; sums: scan_scratch_words(n) - SP_WORDS words
-static void scan_levels(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t *sums, hipStream_t s)
+// the multi-level form; sums: the scratch words past the single-pass scan's
+template <class OP>
+static void scan_levels(const OP &op, size_t n, unsigned rows, uint32_t *total, uint32_t *sums, hipStream_t s)
 {
 	const size_t nb = (n + SC_TILE - 1) / SC_TILE;
 	if (nb == 1) {
-		hipLaunchKernelGGL(k_scan_apply, dim3(1), dim3(SC_BS), 0, s, in, out, n, (const uint32_t *)nullptr, total);
+		hipLaunchKernelGGL(k_scan_apply<OP>, dim3(1, rows), dim3(SC_BS), 0, s, op, n, (const uint32_t *)nullptr, total);
 		return;
 	}
-	hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SC_BS), 0, s, in, n, sums);
+	hipLaunchKernelGGL(k_scan_reduce<OP>, dim3((unsigned)nb, rows), dim3(SC_BS), 0, s, op, n, sums);
 	if (nb <= (size_t)SC_SMALL)
-		hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SC_SBS), 0, s, sums, (uint32_t)nb);
+		hipLaunchKernelGGL(k_scan_sums, dim3(rows), dim3(SC_SBS), 0, s, sums, (uint32_t)nb);
 	else
-		scan_levels(sums, sums, nb, nullptr, sums + nb, s);
-	hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SC_BS), 0, s, in, out, n, (const uint32_t *)sums,
+		scan_levels(ScanWords{sums, sums, nb, nb}, nb, rows, nullptr, sums + rows * nb, s);
+	hipLaunchKernelGGL(k_scan_apply<OP>, dim3((unsigned)nb, rows), dim3(SC_BS), 0, s, op, n, (const uint32_t *)sums,
 	                   total);
+}
+
+template <class OP>
+static void scan_run(const OP &op, size_t n, unsigned rows, uint32_t *total, uint32_t *scratch, hipStream_t s)
+{
+	if (n == 0) {
+		if (total) // a kernel, not a memset: launch errors reach the caller's stream check
+			hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(rows), 0, s, total);
+		return;
+	}
+	const size_t nb = (n + SC_TILE - 1) / SC_TILE;
+	if (nb > 1 && nb <= (size_t)SP_MAX_TILES)
+		hipLaunchKernelGGL(k_scan_1p<OP>, dim3((unsigned)nb, rows), dim3(SC_BS), 0, s, op, n, total, scratch,
+		                   (uint32_t)nb);
+	else
+		scan_levels(op, n, rows, total, scratch + SC_ROWS * SP_WORDS, s);
 }
 
 void scan_excl_u32(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t *scratch,
                    hipStream_t s)
 {
-	if (n == 0) {
-		if (total) // a kernel, not a memset: launch errors reach the caller's stream check
-			hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, s, total);
-		return;
-	}
-	const size_t nb = (n + SC_TILE - 1) / SC_TILE;
-	if (nb > 1 && nb <= (size_t)SP_MAX_TILES)
-		hipLaunchKernelGGL(k_scan_1p, dim3((unsigned)nb), dim3(SC_BS), 0, s, in, out, n, total, scratch,
-		                   (uint32_t)nb);
-	else
-		scan_levels(in, out, n, total, scratch + SP_WORDS, s);
+	scan_run(ScanWords{in, out, n, n}, n, 1, total, scratch, s);
+}
+
+void scan_excl_rows_u32(const uint32_t *in, uint32_t *out, size_t n, size_t nin, size_t stride, int rows,
+                        uint32_t *total, uint32_t *scratch, hipStream_t s)
+{
+	scan_run(ScanWords{in, out, nin, stride}, n, (unsigned)rows, total, scratch, s);
 }
 
 // ---------------------------------------------------------------------------
@@ -616,25 +653,40 @@ __global__ void k_weld_keys(const double *__restrict__ pts, uint32_t n, uint32_t
 	vals[i] = i;
 }
 
-__global__ void k_weld_segflags(const uint32_t *__restrict__ keys, uint32_t n, uint32_t *flags)
-{
-	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	const float tol = 0.00001f;
-	uint32_t f = 1;
-	if (i > 0)
-		f = (ord2f(keys[i]) - ord2f(keys[i - 1])) >= tol;
-	flags[i] = f;
-}
+// The segments in one scan: the value at sorted position i is whether a
+// segment starts there (always at the first position of a task, tk, when
+// given); written are i's segment and, at a start, the segment's first
+// position.  The flags as a pass and an array of their own, and the starts as
+// another pass, took two launches more (4 us each at 30 k vertices), and at 6.1 M
+// 54 us where this takes 45.
+template <bool TASKS>
+struct WeldSegments {
+	const uint32_t *keys, *tk;
+	uint32_t *seg, *starts;
+	// no load depends on another's value, so a thread's loads go out together
+	__device__ uint32_t get(size_t i, uint32_t) const
+	{
+		const float tol = 0.00001f;
+		const size_t h = i ? i - 1 : 0;
+		const uint32_t a = keys[h], b = keys[i];
+		const uint32_t ta = TASKS ? tk[h] : 0u, tb = TASKS ? tk[i] : 0u;
+		return (uint32_t)(i == 0) | (uint32_t)(ta != tb) | (uint32_t)((ord2f(b) - ord2f(a)) >= tol);
+	}
+	__device__ void put(size_t i, uint32_t, uint32_t sum, uint32_t v) const
+	{
+		seg[i] = sum + v - 1u;
+		if (v)
+			starts[sum] = (uint32_t)i;
+	}
+};
 
-// segment starts from the exclusive scan of the flags
-__global__ void k_weld_segstarts(const uint32_t *__restrict__ flags, const uint32_t *__restrict__ segid,
-                                 uint32_t n, uint32_t *starts)
+void launch_weld_segments(const uint32_t *keys, const uint32_t *tk, uint32_t n, uint32_t *seg, uint32_t *starts,
+                          uint32_t *total, uint32_t *scratch, hipStream_t s)
 {
-	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n && flags[i])
-		starts[segid[i]] = i;
+	if (tk)
+		scan_run(WeldSegments<true>{keys, tk, seg, starts}, n, 1, total, scratch, s);
+	else
+		scan_run(WeldSegments<false>{keys, tk, seg, starts}, n, 1, total, scratch, s);
 }
 
 // d_nseg (when given) holds the segment count on the device: the launch
@@ -876,7 +928,7 @@ __global__ void k_weld_greedy(const uint32_t *__restrict__ starts, uint32_t nseg
 // the position): from lrep at the seeds when given, else by atomics on a rep
 // array the caller filled with -1.
 __global__ void k_weld_assign(const uint32_t *__restrict__ vals, const int *__restrict__ lcls,
-                              const uint32_t *__restrict__ flags, const uint32_t *__restrict__ segid,
+                              const uint32_t *__restrict__ seg,
                               const uint32_t *__restrict__ seedbase, uint32_t n, int *__restrict__ cls,
                               int *__restrict__ rep, const uint32_t *__restrict__ d_nnew,
                               const uint32_t *__restrict__ lrep)
@@ -884,10 +936,9 @@ __global__ void k_weld_assign(const uint32_t *__restrict__ vals, const int *__re
 	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
 	if (i >= n)
 		return;
-	uint32_t sg = segid[i] + flags[i] - 1; // inclusive segment index
 	uint32_t v = vals[i];
 	const bool ident = d_nnew && *d_nnew == n;
-	const int c = ident ? (int)v : (int)seedbase[sg] + lcls[i];
+	const int c = ident ? (int)v : (int)seedbase[seg[i]] + lcls[i];
 	cls[v] = c;
 	if (!lrep)
 		atomicMax(&rep[c], (int)v);
@@ -942,15 +993,6 @@ void launch_weld_keys(const double *pts, uint32_t n, uint32_t *keys, uint32_t *v
 {
 	hipLaunchKernelGGL(k_weld_keys, dim3(g1(n)), dim3(256), 0, s, pts, n, keys, vals);
 }
-void launch_weld_segflags(const uint32_t *keys, uint32_t n, uint32_t *flags, hipStream_t s)
-{
-	hipLaunchKernelGGL(k_weld_segflags, dim3(g1(n)), dim3(256), 0, s, keys, n, flags);
-}
-void launch_weld_segstarts(const uint32_t *flags, const uint32_t *segid, uint32_t n, uint32_t *starts,
-                           hipStream_t s)
-{
-	hipLaunchKernelGGL(k_weld_segstarts, dim3(g1(n)), dim3(256), 0, s, flags, segid, n, starts);
-}
 void launch_weld_greedy(const uint32_t *starts, uint32_t nseg, uint32_t n, const uint32_t *keys,
                         const uint32_t *vals, const double *pts, int *lcls, uint32_t *seeds, uint32_t *lrep,
                         hipStream_t s, const uint32_t *d_nseg)
@@ -958,12 +1000,12 @@ void launch_weld_greedy(const uint32_t *starts, uint32_t nseg, uint32_t n, const
 	hipLaunchKernelGGL(k_weld_greedy, dim3(g1(nseg)), dim3(256), 0, s, starts, nseg, n, keys, vals, pts, lcls,
 	                   seeds, d_nseg, lrep);
 }
-void launch_weld_assign(const uint32_t *vals, const int *lcls, const uint32_t *flags, const uint32_t *segid,
-                        const uint32_t *seedbase, const uint32_t *lrep, uint32_t n, int *cls, int *rep,
-                        hipStream_t s, const uint32_t *d_nnew)
+void launch_weld_assign(const uint32_t *vals, const int *lcls, const uint32_t *seg, const uint32_t *seedbase,
+                        const uint32_t *lrep, uint32_t n, int *cls, int *rep, hipStream_t s,
+                        const uint32_t *d_nnew)
 {
-	hipLaunchKernelGGL(k_weld_assign, dim3(g1(n)), dim3(256), 0, s, vals, lcls, flags, segid, seedbase, n, cls,
-	                   rep, d_nnew, lrep);
+	hipLaunchKernelGGL(k_weld_assign, dim3(g1(n)), dim3(256), 0, s, vals, lcls, seg, seedbase, n, cls, rep,
+	                   d_nnew, lrep);
 }
 void launch_gather_pts(const double *pts, const int *rep, uint32_t n, double *out, hipStream_t s,
                        const uint32_t *d_n)
@@ -1008,17 +1050,26 @@ __global__ void k_degen_flags(const double *__restrict__ pts, const int *__restr
 
 // The welded position of every vertex in its own (pre-weld) order, wpos[v] =
 // pts[rep[cls[v]]] (the weld's output position of v's class), so that
-// triangles can read positions in emit order.  rep[c] is mostly v itself.
+// triangles can read positions in emit order.  rep[c] is mostly v itself;
+// that vertex writes the weld's output position of c (out) as well, which
+// spares the output a gather of its own (a launch, and the positions again).
 __global__ void k_weld_wpos(const double *__restrict__ pts, const int *__restrict__ cls,
-                            const int *__restrict__ rep, uint32_t npt, double *__restrict__ wpos)
+                            const int *__restrict__ rep, uint32_t npt, double *__restrict__ wpos,
+                            double *__restrict__ out)
 {
 	uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
 	if (v >= npt)
 		return;
-	const size_t r = (size_t)(uint32_t)rep[cls[v]];
-	wpos[(size_t)v * 3] = pts[r * 3];
-	wpos[(size_t)v * 3 + 1] = pts[r * 3 + 1];
-	wpos[(size_t)v * 3 + 2] = pts[r * 3 + 2];
+	const size_t c = (size_t)(uint32_t)cls[v], r = (size_t)(uint32_t)rep[c];
+	const double x = pts[r * 3], y = pts[r * 3 + 1], z = pts[r * 3 + 2];
+	wpos[(size_t)v * 3] = x;
+	wpos[(size_t)v * 3 + 1] = y;
+	wpos[(size_t)v * 3 + 2] = z;
+	if (r == v) {
+		out[c * 3] = x;
+		out[c * 3 + 1] = y;
+		out[c * 3 + 2] = z;
+	}
 }
 
 // k_remap_tris and k_degen_flags in one pass: the welded ids of a
@@ -1061,9 +1112,10 @@ __global__ void k_remap_degen(const int *__restrict__ tris_in, const int *__rest
 	keep[i] = k;
 }
 
-void launch_weld_wpos(const double *pts, const int *cls, const int *rep, uint32_t npt, double *wpos, hipStream_t s)
+void launch_weld_wpos(const double *pts, const int *cls, const int *rep, uint32_t npt, double *wpos, double *out,
+                      hipStream_t s)
 {
-	hipLaunchKernelGGL(k_weld_wpos, dim3(g1(npt)), dim3(256), 0, s, pts, cls, rep, npt, wpos);
+	hipLaunchKernelGGL(k_weld_wpos, dim3(g1(npt)), dim3(256), 0, s, pts, cls, rep, npt, wpos, out);
 }
 
 void launch_remap_degen(const int *tris_in, const int *cls, uint32_t npt, const double *wpos, uint32_t nt,
@@ -1072,10 +1124,16 @@ void launch_remap_degen(const int *tris_in, const int *cls, uint32_t npt, const 
 	hipLaunchKernelGGL(k_remap_degen, dim3(g1(nt)), dim3(256), 0, s, tris_in, cls, npt, wpos, nt, tris_out, keep);
 }
 
+// counts (when given): the class count *d_np and the kept triangles, for the host
 __global__ void k_compact_tris(const int *__restrict__ tris, const uint32_t *__restrict__ keep,
-                               const uint32_t *__restrict__ pos, uint32_t nt, int *__restrict__ out)
+                               const uint32_t *__restrict__ pos, uint32_t nt, int *__restrict__ out,
+                               const uint32_t *__restrict__ d_np, uint32_t *counts)
 {
 	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (counts && i == 0) {
+		counts[0] = *d_np;
+		counts[1] = nt ? pos[nt - 1] + keep[nt - 1] : 0u;
+	}
 	if (i >= nt || !keep[i])
 		return;
 	uint32_t o = pos[i];
@@ -1090,9 +1148,9 @@ void launch_degen_flags(const double *pts, const int *tris, uint32_t nt, uint32_
 	hipLaunchKernelGGL(k_degen_flags, dim3(g1(nt)), dim3(256), 0, s, pts, tris, nt, np, keep);
 }
 void launch_compact_tris(const int *tris, const uint32_t *keep, const uint32_t *pos, uint32_t nt, int *out,
-                         hipStream_t s)
+                         hipStream_t s, const uint32_t *d_np, uint32_t *counts)
 {
-	hipLaunchKernelGGL(k_compact_tris, dim3(g1(nt)), dim3(256), 0, s, tris, keep, pos, nt, out);
+	hipLaunchKernelGGL(k_compact_tris, dim3(g1(nt)), dim3(256), 0, s, tris, keep, pos, nt, out, d_np, counts);
 }
 
 // ---------------------------------------------------------------------------
@@ -2856,19 +2914,6 @@ __global__ void k_atlas_weld_keys(const double *__restrict__ pts, uint32_t n, co
 	vtask[i] = (uint32_t)t;
 }
 
-__global__ void k_atlas_weld_segflags(const uint32_t *__restrict__ keys, const uint32_t *__restrict__ tk, uint32_t n,
-                                      uint32_t *flags)
-{
-	uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= n)
-		return;
-	const float tol = 0.00001f;
-	uint32_t f = 1;
-	if (i > 0 && tk[i] == tk[i - 1])
-		f = (ord2f(keys[i]) - ord2f(keys[i - 1])) >= tol;
-	flags[i] = f;
-}
-
 // first class of each task (the seed at its first sorted position)
 __global__ void k_atlas_class_base(const uint32_t *__restrict__ tk, const uint32_t *__restrict__ segid,
                                    const uint32_t *__restrict__ seedbase, uint32_t n, uint32_t *cbase)
@@ -2944,12 +2989,6 @@ void launch_atlas_weld_keys(const double *pts, uint32_t n, const uint32_t *vbase
 	if (n)
 		hipLaunchKernelGGL(k_atlas_weld_keys, dim3(g1(n)), dim3(256), 0, s, pts, n, vbase, ntasks, keys, vals,
 		                   vtask);
-}
-void launch_atlas_weld_segflags(const uint32_t *keys, const uint32_t *tk, uint32_t n, uint32_t *flags,
-                                hipStream_t s)
-{
-	if (n)
-		hipLaunchKernelGGL(k_atlas_weld_segflags, dim3(g1(n)), dim3(256), 0, s, keys, tk, n, flags);
 }
 void launch_atlas_class_base(const uint32_t *tk, const uint32_t *segid, const uint32_t *seedbase, uint32_t n,
                              uint32_t *cbase, hipStream_t s)

@@ -222,8 +222,13 @@ int lw_seg_len();
 // k_mesh.hip
 size_t scan_scratch_words(size_t n);
 size_t scan_scratch_zero_words(); // leading words kept zero between scans
+// total (may be host memory the device writes): the sum, when given
 void scan_excl_u32(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t *scratch,
                    hipStream_t s);
+// up to 3 scans in the launches of one: row r at in + r * stride -> out + r *
+// stride, n words of which those past nin count as 0; a total per row
+void scan_excl_rows_u32(const uint32_t *in, uint32_t *out, size_t n, size_t nin, size_t stride, int rows,
+                        uint32_t *total, uint32_t *scratch, hipStream_t s);
 size_t radix_counts_words(size_t n);
 bool radix_sort_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, size_t n, int bits,
                     uint32_t *counts, uint32_t *scan_scratch, hipStream_t s);
@@ -239,9 +244,10 @@ bool radix_sort_seg_u32(uint32_t *k0, uint32_t *v0, uint32_t *k1, uint32_t *v1, 
                         const RsTile *desc, size_t ntiles, uint32_t *counts, uint32_t *scan_scratch,
                         hipStream_t s);
 void launch_weld_keys(const double *pts, uint32_t n, uint32_t *keys, uint32_t *vals, hipStream_t s);
-void launch_weld_segflags(const uint32_t *keys, uint32_t n, uint32_t *flags, hipStream_t s);
-void launch_weld_segstarts(const uint32_t *flags, const uint32_t *segid, uint32_t n, uint32_t *starts,
-                           hipStream_t s);
+// the sorted keys' segments (never across two tasks of tk, when given): seg[i],
+// the segment of position i, starts[k] its first position, and the count
+void launch_weld_segments(const uint32_t *keys, const uint32_t *tk, uint32_t n, uint32_t *seg, uint32_t *starts,
+                          uint32_t *total, uint32_t *scratch, hipStream_t s);
 // d_nseg / d_nnew / d_n: counts left on the device (no host round trip);
 // the launches then cover the upper bound n
 // lrep: n words written by the greedy pass (each seed's representative), from
@@ -249,13 +255,15 @@ void launch_weld_segstarts(const uint32_t *flags, const uint32_t *segid, uint32_
 void launch_weld_greedy(const uint32_t *starts, uint32_t nseg, uint32_t n, const uint32_t *keys,
                         const uint32_t *vals, const double *pts, int *lcls, uint32_t *seeds, uint32_t *lrep,
                         hipStream_t s, const uint32_t *d_nseg = nullptr);
-void launch_weld_assign(const uint32_t *vals, const int *lcls, const uint32_t *flags, const uint32_t *segid,
-                        const uint32_t *seedbase, const uint32_t *lrep, uint32_t n, int *cls, int *rep,
-                        hipStream_t s, const uint32_t *d_nnew = nullptr);
+void launch_weld_assign(const uint32_t *vals, const int *lcls, const uint32_t *seg, const uint32_t *seedbase,
+                        const uint32_t *lrep, uint32_t n, int *cls, int *rep, hipStream_t s,
+                        const uint32_t *d_nnew = nullptr);
 void launch_gather_pts(const double *pts, const int *rep, uint32_t n, double *out, hipStream_t s,
                        const uint32_t *d_n = nullptr);
-// wpos[v] = pts[rep[cls[v]]]: the welded position of every pre-weld vertex v
-void launch_weld_wpos(const double *pts, const int *cls, const int *rep, uint32_t npt, double *wpos, hipStream_t s);
+// wpos[v] = pts[rep[cls[v]]]: the welded position of every pre-weld vertex v,
+// and out[c] = pts[rep[c]], that of every class
+void launch_weld_wpos(const double *pts, const int *cls, const int *rep, uint32_t npt, double *wpos, double *out,
+                      hipStream_t s);
 // remap (tris_in null: implicit 3t+k) and degenerate flags in one pass
 void launch_remap_degen(const int *tris_in, const int *cls, uint32_t npt, const double *wpos, uint32_t nt,
                         int *tris_out, uint32_t *keep, hipStream_t s);
@@ -265,7 +273,7 @@ void launch_remap_tris(const int *tris_in, const int *cls, uint32_t nt, uint32_t
 void launch_degen_flags(const double *pts, const int *tris, uint32_t nt, uint32_t np, uint32_t *keep,
                         hipStream_t s);
 void launch_compact_tris(const int *tris, const uint32_t *keep, const uint32_t *pos, uint32_t nt, int *out,
-                         hipStream_t s);
+                         hipStream_t s, const uint32_t *d_np = nullptr, uint32_t *counts = nullptr);
 // CSR of the references: count (with each corner's arrival rank), scan,
 // fill at start + rank, then sort each vertex's list and expand to pairs
 // inv given: counts the references of inv[tris[i]] and writes those ids to
@@ -345,8 +353,6 @@ size_t long_huge_words(size_t nt);
 // batched atlas weld (k_mesh.hip)
 void launch_atlas_weld_keys(const double *pts, uint32_t n, const uint32_t *vbase, int ntasks, uint32_t *keys,
                             uint32_t *vals, uint32_t *vtask, hipStream_t s);
-void launch_atlas_weld_segflags(const uint32_t *keys, const uint32_t *tk, uint32_t n, uint32_t *flags,
-                                hipStream_t s);
 void launch_atlas_class_base(const uint32_t *tk, const uint32_t *segid, const uint32_t *seedbase, uint32_t n,
                              uint32_t *cbase, hipStream_t s);
 void launch_atlas_weld_tasks(uint32_t *cbase, const uint32_t *vbase, const uint32_t *nextne, int ntasks,

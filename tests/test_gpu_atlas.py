@@ -257,5 +257,5 @@ def test_atlas_crop_shapes(gpu, oracle, shape):
     vol[rng.random(shape) < 0.3] = 2
     vol[rng.random(shape) < 0.2] = 0
     for loop in (False, True):
-        got = run_gpu(gpu, vol, 0, 0, True, False, 0, None, loop)
+        _, got = run_gpu(gpu, vol, 0, 0, True, False, 0, None, loop)
         compare(got, expect(oracle, vol, 0, 0, True, False, 0, None))
