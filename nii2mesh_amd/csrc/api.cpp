@@ -286,7 +286,6 @@ struct n2m_ctx {
 	DevBuf bufs[S_COUNT];
 	std::vector<Mesh> meshes;
 	Mesh atlas_mesh;                    // union of the label meshes of the last atlas run
-	Mesh host_mesh;                     // the host-memory meshify()'s result, buffers kept between calls
 	std::vector<n2m_atlas_entry> atlas; // one entry per label 1..n
 	struct {                            // last differentiable forward
 		bool valid = false;
@@ -537,7 +536,6 @@ void ctx_free(n2m_ctx *c)
 		if (b.p)
 			(void)hipFree(b.p);
 	c->meshes.push_back(c->atlas_mesh);
-	c->meshes.push_back(c->host_mesh);
 	for (auto &m : c->meshes) {
 		if (m.tris.p)
 			(void)hipFree(m.tris.p);
@@ -3361,7 +3359,17 @@ int meshify(float *img, short dim[3], int originalMC, float isolevel, vec3i **t,
 		float *src = C->buf<float>(S_VOL, nvox);
 		xfer_big(C, src, img, 4 * nvox, false);
 		n2m_params P{cubes_flavour(), originalMC, isolevel, preSmooth, onlyLargest, fillBubbles, verbose};
-		Mesh &m = C->host_mesh; // its buffers trade places with the scratch's (adopt)
+		Mesh m;
+		struct Free {
+			Mesh &m;
+			~Free()
+			{
+				if (m.tris.p)
+					(void)hipFree(m.tris.p);
+				if (m.pts.p)
+					(void)hipFree(m.pts.p);
+			}
+		} fr{m};
 		bool ok = meshify_device(C, src, src, d, P, m);
 		// the reference leaves img smoothed, filled and darkened
 		xfer_big(C, img, src, 4 * nvox, true);
