@@ -353,7 +353,11 @@ def main():
     atlas_vol = None
     if not args.no_atlas:
         out['atlas'], atlas_vol = atlas_leg(torch, n2m, synth)
-    if not args.no_cpu:
+    if not args.no_cpu and not os.path.exists(os.path.join(REF_DIR, 'nii2mesh_lewiner')):
+        # the line is printed all the same, without the reference's times
+        log('cpu baseline skipped: no reference build in %s (make -C oracle ref)' % REF_DIR)
+        out['cpu_baseline'] = None
+    elif not args.no_cpu:
         log('cpu baseline ...')
         out['cpu_baseline'] = cpu_baseline(vol, isos)
         log('cpu baseline %.6f GVoxel/s, stages %s' % (out['cpu_baseline']['value'], out['cpu_baseline']['stages_ms']))

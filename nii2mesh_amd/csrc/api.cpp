@@ -261,7 +261,7 @@ enum Small {
 	SM_RING = 45,  // 1 word: a smoothing block overflowed its two rings
 	SM_WNSEG = 48, // 1 word: weld segment count (left on the device)
 	SM_WNNEW = 49, // 1 word: welded vertex count (left on the device)
-	SM_DEGK = 50,  // 1 word: triangles kept by the degenerate test (follows SM_WNNEW)
+	SM_DEGK = 50,  // 1 word, host only: triangles kept by the degenerate test (follows SM_WNNEW)
 	SM_WORDS = 64
 };
 

@@ -62,13 +62,6 @@ __device__ __forceinline__ const NbrRow *nbr_rows(int conn, int *n)
 
 __device__ __forceinline__ uint32_t run_starts(uint32_t w) { return w & ~(w << 1); }
 
-// first bit of the run of w (starts = run_starts(w)) that contains bit b
-__device__ __forceinline__ int run_of(uint32_t starts, int b)
-{
-	uint32_t m = b == 31 ? starts : (starts & ((2u << b) - 1u));
-	return 31 - __clz(m);
-}
-
 // length of the run of w starting at bit s
 __device__ __forceinline__ int run_len(uint32_t w, int s)
 {

@@ -1052,7 +1052,8 @@ __global__ void k_degen_flags(const double *__restrict__ pts, const int *__restr
 // pts[rep[cls[v]]] (the weld's output position of v's class), so that
 // triangles can read positions in emit order.  rep[c] is mostly v itself;
 // that vertex writes the weld's output position of c (out) as well, which
-// spares the output a gather of its own (a launch, and the positions again).
+// spares small meshes a gather's launch (4 us; three meshes of 13 M vertices
+// take 0.45 ms either way).
 __global__ void k_weld_wpos(const double *__restrict__ pts, const int *__restrict__ cls,
                             const int *__restrict__ rep, uint32_t npt, double *__restrict__ wpos,
                             double *__restrict__ out)
@@ -1772,8 +1773,8 @@ k_laplace_h(const uint32_t *__restrict__ start, const uint32_t *__restrict__ slo
 // and finishes the block's vertices (the hc_b step).  Only the new positions
 // go to memory: no pn / b arrays.  Ring-1 vertices are computed by every block
 // that borders them, with the same terms in the same order, so the values are
-// those of the two-launch form.  Ring-1 pair lists are kept per block as LDS
-// slots (roff: 16-bit offsets, rslots: slot pairs).
+// those of the two-launch form.  The pair lists of block and ring 1 are kept per
+// block as pairs of LDS rows (see k_ring_build).
 // ---------------------------------------------------------------------------
 constexpr int HE = 6; // a vertex's pairs kept pair by pair, see k_ring_build
 // RB (vertices per block) is a template parameter: 512 to 896 with 1024
