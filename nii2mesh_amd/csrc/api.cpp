@@ -710,9 +710,9 @@ void set_mesh_count(n2m_ctx *c, int n)
 
 // scratch of the device scans: sized for 2^31 elements up front, so a later
 // scan never reallocates a buffer that queued kernels still read
-uint32_t *scan_scratch(n2m_ctx *C, size_t n)
+uint32_t *scan_scratch(n2m_ctx *C, size_t n, int rows = 1)
 {
-	size_t w = scan_scratch_words(n) + 16;
+	size_t w = scan_scratch_words(n, rows) + 16;
 	uint32_t *p = C->buf<uint32_t>(S_SCAN, w > ((size_t)1 << 21) ? w : ((size_t)1 << 21));
 	// the single-pass scan keeps the scratch's leading words zero between
 	// scans: zero them once per allocation, stream-ordered before the scans
@@ -730,7 +730,7 @@ uint32_t *scan_scratch(n2m_ctx *C, size_t n)
 void scan3(n2m_ctx *C, const uint32_t *in, uint32_t *out, size_t n, uint32_t tot[3])
 {
 	const uint32_t *t = C->h_small + SM_TOTAL; // written by the scan itself
-	scan_excl_rows_u32(in, out, n, n, n, 3, C->h_small + SM_TOTAL, scan_scratch(C, n), C->stream);
+	scan_excl_rows_u32(in, out, n, n, n, 3, C->h_small + SM_TOTAL, scan_scratch(C, n, 3), C->stream);
 	C->check();
 	C->sync();
 	for (int k = 0; k < 3; k++)
@@ -1981,7 +1981,7 @@ void atlas_chunk(n2m_ctx *C, const float *labels, const int dim[3], const n2m_pa
 		C->tbegin("atlas_mc_lewiner_classify", 7.0 * npts);
 		classify_with(lcfg);
 		C->tend();
-		scan_excl_rows_u32(cnt, base, stride, nb, stride, 3, nullptr, scan_scratch(C, stride), s);
+		scan_excl_rows_u32(cnt, base, stride, nb, stride, 3, nullptr, scan_scratch(C, stride, 3), s);
 		C->check();
 		std::vector<uint32_t> idx(3 * (nt_ + 1));
 		for (int j = 0; j < 3; j++) {

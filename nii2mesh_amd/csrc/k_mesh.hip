@@ -107,14 +107,14 @@ constexpr int SP_MAX_TILES = 128, SP_WORDS = 320; // SP_WORDS >= 2 + 2 * SP_MAX_
 constexpr int SC_ROWS = 3;
 static_assert(SP_WORDS >= 2 + 2 * SP_MAX_TILES, "single-pass scan scratch");
 
-size_t scan_scratch_words(size_t n)
+size_t scan_scratch_words(size_t n, int rows)
 {
 	size_t w = 0;
 	while (n > SC_TILE) {
 		n = (n + SC_TILE - 1) / SC_TILE;
 		w += n;
 	}
-	return SC_ROWS * (SP_WORDS + w) + 1;
+	return SC_ROWS * SP_WORDS + rows * w + 1;
 }
 size_t scan_scratch_zero_words() { return SC_ROWS * SP_WORDS; }
 

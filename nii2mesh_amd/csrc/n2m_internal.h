@@ -220,7 +220,7 @@ void launch_atlas_lw_emit(const float *crops, const AtlasTask *tasks, int ntasks
 int lw_seg_len();
 
 // k_mesh.hip
-size_t scan_scratch_words(size_t n);
+size_t scan_scratch_words(size_t n, int rows = 1);
 size_t scan_scratch_zero_words(); // leading words kept zero between scans
 // total (may be host memory the device writes): the sum, when given
 void scan_excl_u32(const uint32_t *in, uint32_t *out, size_t n, uint32_t *total, uint32_t *scratch,
