@@ -19,6 +19,9 @@
 //
 // Predicate: bit of `bits` (packed rows, see k_volume.hip), or its complement
 // inside the volume when `invert` (background labelling for bubble fill).
+// The bits past a row's end must be 0, as every pass that writes a mask leaves
+// them: then there is at most one run per voxel, which is what the label
+// arrays and the root list are sized for.
 #include "n2m_device.cuh"
 #include "n2m_internal.h"
 

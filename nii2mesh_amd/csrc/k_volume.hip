@@ -707,14 +707,18 @@ void launch_atlas_bmap(const AtlasTask *tasks, int ntasks, uint32_t nblocks, uin
 // masks of all isolevels of `iso` in one read, mask k to bits + k * iso.nwords.
 // range / only_moved: see launch_mask_bits (one isolevel).
 // ---------------------------------------------------------------------------
-// the isolevel of a mask (launch_mask_bits); false: the mask stays
+// the isolevel of a mask (launch_mask_bits); false: the mask stays.  Without
+// variability no voxel passes: the labelling is queued before the host knows
+// the range, and the mask it reads has to have been written.
 __device__ __forceinline__ bool mask_iso(const uint32_t *range, int only_moved, float &iso)
 {
 	if (!range)
 		return true;
 	float edgeMax;
 	bool moved = false;
-	return atlas_iso(iso, ord2f(range[0]), ord2f(range[1]), &iso, &edgeMax, &moved) && (moved || !only_moved);
+	if (!atlas_iso(iso, ord2f(range[0]), ord2f(range[1]), &iso, &edgeMax, &moved))
+		iso = __builtin_nanf("");
+	return moved || !only_moved;
 }
 
 // Any row length: a wave takes 64 consecutive voxels of a row (an item; the

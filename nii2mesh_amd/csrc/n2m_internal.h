@@ -91,8 +91,9 @@ void launch_smooth(const float *in, float *out, int nx, int ny, int nz, uint32_t
                    int nmask, uint32_t *bits, hipStream_t s);
 void launch_minmax(const float *img, size_t n, uint32_t *range, hipStream_t s);
 // range (when given): the ordered min / max words of img on the device; the
-// isolevel is then what meshify() takes for `iso` in that range, and with
-// only_moved the mask is written only when that is another value
+// isolevel is then what meshify() takes for `iso` in that range (the mask is
+// empty where that has no variability), and with only_moved the mask is
+// written only when that is another value
 void launch_mask_bits(const float *img, int nx, int ny, int nz, float iso, int nonzero, uint32_t *bits,
                       hipStream_t s, const uint32_t *range = nullptr, bool only_moved = false);
 void launch_dilate_bits(const uint32_t *in, uint32_t *out, int nx, int ny, int nz, hipStream_t s);

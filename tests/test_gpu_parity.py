@@ -621,6 +621,41 @@ def test_meshify_iso_fallback_and_failures(gpu, oracle):
     assert gpu.lib(0).meshify(c.copy(), 1.0)[0] == 1
 
 
+@pytest.mark.parametrize('smooth', [False, True])
+@pytest.mark.parametrize('largest,fill', [(True, False), (False, True), (True, True)])
+@pytest.mark.parametrize('shape', [(40, 36, 2), (33, 31, 7), (20, 18, 33), (16, 17, 65), (6, 7, 96), (4, 50, 64)])
+def test_meshify_constant_unsmoothed(gpu, oracle, shape, largest, fill, smooth):
+    """A constant volume that no smoothing pass wrote a mask of (smoothing off,
+    or a side below 5) fails and stays as it is, with the largest cluster and
+    the bubble fill on, after a noisy volume of the same size through the same
+    context; the noisy volume's mesh is the same before and after."""
+    import torch
+    if smooth and min(shape) >= 5:
+        shape = shape[:2] + (4,)
+    rng = np.random.default_rng(shape[2])
+    noisy = (rng.standard_normal(shape) * 20 + 100).astype(np.float32)
+    flat = np.full(shape, 3.0, np.float32)
+    flags = (smooth, largest, fill)
+    for cubes in (0, 1):
+        lib = gpu.lib(cubes)
+        for img in (noisy, flat, noisy):
+            a, b = img.copy(), img.copy()
+            ra, rb = lib.meshify(a, 95.0, *flags), oracle.meshify(b, 95.0, *flags, cubes=cubes)
+            assert ra[0] == rb[0] == (1 if img is flat else 0)
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+            if img is not flat:
+                assert _eq(ra[1], rb[1]) and _eq(ra[2], rb[2])
+            else:
+                assert np.array_equal(a, flat)
+        with gpu.DeviceContext() as ctx:  # each isolevel on a context of its own
+            prm = ctx.params(0.0, cubes=cubes, preSmooth=smooth, onlyLargest=largest, fillBubbles=fill)
+            for img in (noisy, flat, noisy):
+                d = torch.from_numpy(img).cuda()
+                torch.cuda.synchronize()
+                assert ctx.pipeline(d.data_ptr(), shape[::-1], prm, [95.0, 105.0], hc_iters=2) == (1 if img is flat else 0)
+                assert np.array_equal(d.cpu().numpy(), img)
+
+
 @pytest.mark.parametrize('flavour,flags', [('classic', (True, True, False)), ('lewiner', (True, True, True))])
 def test_meshify_plain_u8_128(gpu, oracle, flavour, flags):
     """The 128^3 uint8 workload at isolevel 128."""
