@@ -1318,17 +1318,22 @@ void check_tris(const int *tris, int ntri, int nvert)
 }
 
 // Meshes of fewer than kRelabelAlways vertices are renumbered for kRelabelIters
-// iterations and more: it takes about 45 us there, and an iteration of 19
-// thousand vertices 5.1 us instead of 7.6 (in marching-cubes order its blocks'
-// rings do not fit the small blocks).  The keys have 5 bits per axis (two
-// radix passes) up to kRelabelFine vertices, 8 bits beyond.
-constexpr uint32_t kRelabelAlways = 32768, kRelabelMin = 4096, kRelabelFine = 131072;
+// iterations and more, from `least` vertices on.  HC: it takes about 45 us
+// there, and an iteration of 19 thousand vertices 5.1 us instead of 7.6 (in
+// marching-cubes order its blocks' rings do not fit the small blocks).
+// Laplacian (halo form, less to gain; host call with 24 / 100 iterations, us,
+// in marching-cubes order and renumbered): 5.2 k vertices 290 / 757 and
+// 307 / 780, 9.1 k 336 / 836 and 332 / 818, 16.9 k 380 / 907 and 370 / 864.
+// The keys have 5 bits per axis (two radix passes) up to kRelabelFine vertices,
+// 8 bits beyond.
+constexpr uint32_t kRelabelAlways = 32768, kRelabelHc = 4096, kRelabelLaplace = 8192, kRelabelFine = 131072;
 constexpr int kRelabelIters = 24;
 
-Relabel morton_relabel(n2m_ctx *C, const double *pts, const int *tris, uint32_t nv, uint32_t nt, int iter)
+Relabel morton_relabel(n2m_ctx *C, const double *pts, const int *tris, uint32_t nv, uint32_t nt, int iter,
+                       uint32_t least)
 {
 	Relabel r;
-	if (nv < kRelabelMin || (nv < kRelabelAlways && iter < kRelabelIters))
+	if (nv < least || (nv < kRelabelAlways && iter < kRelabelIters))
 		return r;
 	hipStream_t s = C->stream;
 	C->tbegin("hc_relabel", 24.0 * nv * 2 + 16.0 * 4 * nv);
@@ -1434,7 +1439,7 @@ void smooth_hc_device(n2m_ctx *C, double *pts, const int *tris, uint32_t nv, uin
 	if (nv == 0)
 		return;
 	hipStream_t s = C->stream;
-	Relabel R = morton_relabel(C, pts, tris, nv, nt, iter);
+	Relabel R = morton_relabel(C, pts, tris, nv, nt, iter, kRelabelHc);
 	const int *T = R.on ? R.tris : tris;
 	Csr c = build_csr(C, T, nv, nt, false, &R);
 	// one launch per iteration (two-ring form) where every block's rings fit,
@@ -1519,7 +1524,7 @@ void laplace_device(n2m_ctx *C, double *pts, const int *tris, uint32_t nv, uint3
 	if (nv == 0 || iter <= 0)
 		return;
 	hipStream_t s = C->stream;
-	Relabel R = morton_relabel(C, pts, tris, nv, nt, iter);
+	Relabel R = morton_relabel(C, pts, tris, nv, nt, iter, kRelabelLaplace);
 	Csr c = build_csr(C, R.on ? R.tris : tris, nv, nt, false, &R);
 	const Halo H = build_halo(C, c, nv, nt);
 	const size_t n3 = 3 * (size_t)nv;

@@ -319,14 +319,14 @@ def test_hc_ring_block_sizes(gpu, oracle, monkeypatch, rb, lock):
     assert 'hc_ring' in stats and 'hc_a' not in stats
 
 
-@pytest.mark.parametrize('nv', [4095, 4096, 32767, 32768, 120000, 120001, 163841])
+@pytest.mark.parametrize('nv', [4095, 4096, 8191, 8192, 32767, 32768, 120000, 120001, 163841])
 @pytest.mark.parametrize('iters', [2, 24])
 @pytest.mark.parametrize('shuffled', [False, True])
 def test_hc_sizes(gpu, oracle, nv, iters, shuffled):
-    """HC smoothing around the sizes where the renumbering starts (with many
-    and with few iterations) and where the small blocks end, on a torus strip
-    with vertices of degree 3 to 12; shuffled, its blocks' rings overflow
-    wherever it is not renumbered, and the larger forms take over."""
+    """HC and Laplacian smoothing around the sizes where the renumbering starts
+    (with many and with few iterations) and where the small blocks end, on a
+    torus strip with vertices of degree 3 to 12; shuffled, its blocks' rings
+    overflow wherever it is not renumbered, and the larger forms take over."""
     rng = np.random.default_rng(nv + iters)
     w = 61
     h = nv // w
@@ -344,9 +344,13 @@ def test_hc_sizes(gpu, oracle, nv, iters, shuffled):
         perm = rng.permutation(nv)
         pts, tris = pts[np.argsort(perm)], perm[tris].astype(np.int32)
     p, q = np.ascontiguousarray(pts), np.ascontiguousarray(pts).copy()
+    l, m = p.copy(), p.copy()
     gpu.lib().laplacian_smoothHC(p, tris, 0.1, 0.5, iters, True)
     oracle.laplacian_smoothHC(q, np.ascontiguousarray(tris), 0.1, 0.5, iters, True)
     assert np.array_equal(p, q)
+    gpu.load().n2m_laplacian_smooth(l, np.ascontiguousarray(tris), nv, len(tris), iters)
+    oracle.laplacian_smooth(m, np.ascontiguousarray(tris), iters)
+    assert np.array_equal(l, m)
 
 
 @pytest.mark.parametrize('wide', [None, 0, 63, 64, -1])
