@@ -2594,17 +2594,23 @@ void launch_laplace_halo(const uint32_t *start, const uint32_t *slots, const uin
 		                   (const d3 *)p, (d3 *)pout, nv);
 }
 // Vertices per two-ring block: N2M_HC_RB (256, 512, 640, 768 or 896), read by
-// each smoothing call, or by the mesh's size.  One iteration, us:
+// each smoothing call, or by the mesh's size.  One iteration, us, on smooth
+// meshes (above) and on noisy ones:
 //
-//   vertices    3.5 k   58 k   92 k  151 k  181 k  369 k  606 k
-//   256          4.9    5.4    7.2    9.0    9.3   15.5   22.5
-//   640          6.7    7.4    7.7    8.5   11.8   17.9   23.3
+//   vertices   51 k   74 k  101 k  127 k  144 k  162 k  181 k  447 k  625 k  889 k  1.01 M  1.13 M  1.48 M
+//   256         5.4    7.0    7.4    7.7    9.2    9.3    9.2   17.0   21.7   27.6    31.0    33.9    42.5
+//   640         7.3    7.4    7.8    8.1    8.2    8.5   11.9   18.6   22.5   29.2
+//   896         8.2    8.3    8.8    8.9    9.2    9.3    9.5   16.9   22.1   27.9    31.6    33.3    41.9
 //
-// A block of 640 on its own CU is the better one as long as the chip takes all
-// of them at once (256 CUs); small blocks pack it more evenly up to some
-// 700 k; beyond, larger blocks read less ring: the 512^3 pipeline, whose
-// largest mesh has 9.6 M vertices, took 52.9 ms with 256, 49.9 with 640, 49.1
-// with 768 and 48.7 with 896.
+//   vertices  119 k  188 k  272 k  413 k  525 k  745 k  1.00 M  1.21 M  1.39 M  1.91 M  4.37 M  9.38 M
+//   256         9.0   10.9   15.1   20.1   22.8   29.6    36.7    43.1    47.7    68.0   158     337
+//   640         9.5   14.1   14.9   20.7   24.7   30.9            45.0
+//   896        10.6   11.9   17.1   19.9   24.8   30.8    37.8    43.1    47.6    63.1   150     312
+//
+// Small blocks pack the chip more evenly; a block of 640 is the better one
+// where the small ones are more than two per CU (256 CUs) and the chip takes
+// all of the 640s at once.  From some 1.1 M on larger blocks, which read less
+// ring, are as fast and then faster, and their build is (9.4 M: 4.2 ms for 5.0).
 int ring_rb(uint32_t nv)
 {
 	const char *e = getenv("N2M_HC_RB");
@@ -2612,9 +2618,9 @@ int ring_rb(uint32_t nv)
 	for (int rb : {256, 512, 640, 768, 896})
 		if (v == rb)
 			return rb;
-	if (nv > 650000)
+	if (nv > 1100000)
 		return 896;
-	return nv > 120000 && nv <= 256 * 640 ? 640 : 256;
+	return nv > 2 * 256 * 256 && nv <= 256 * 640 ? 640 : 256;
 }
 #define N2M_RING_RBS(X) X(256) X(512) X(640) X(768) X(896)
 struct RingDims {

@@ -319,7 +319,7 @@ def test_hc_ring_block_sizes(gpu, oracle, monkeypatch, rb, lock):
     assert 'hc_ring' in stats and 'hc_a' not in stats
 
 
-@pytest.mark.parametrize('nv', [4095, 4096, 8191, 8192, 32767, 32768, 120000, 120001, 163841])
+@pytest.mark.parametrize('nv', [4095, 4096, 8191, 8192, 32767, 32768, 120000, 131072, 131073, 163840, 163841])
 @pytest.mark.parametrize('iters', [2, 24])
 @pytest.mark.parametrize('shuffled', [False, True])
 def test_hc_sizes(gpu, oracle, nv, iters, shuffled):
