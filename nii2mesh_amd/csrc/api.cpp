@@ -1452,7 +1452,8 @@ void smooth_hc_device(n2m_ctx *C, double *pts, const int *tris, uint32_t nv, uin
 	launch_hc_load(pts, R.on ? R.perm : nullptr, nv, o, s, o32, C->d_small + SM_WIDE);
 	// the rings and whether a triangle repeats a vertex (for the border flags)
 	// come back in one round trip; rings that overflowed at another size are
-	// built again with 640 vertices per block, which leaves them the most room
+	// built again with 512 vertices per block, which leaves them the most room
+	// (2304 rows less the block's own; a small block has 1152 in all)
 	const char *er = getenv("N2M_HC_RING");
 	const bool want_ring = iter > 0 && !(er && *er == '0');
 	Ring G;
@@ -1466,9 +1467,9 @@ void smooth_hc_device(n2m_ctx *C, double *pts, const int *tris, uint32_t nv, uin
 		repeats = f[0] != 0;
 		f32 = f[SM_WIDE - SM_FLAG] == 0;
 		G.on = want_ring && f[SM_RING - SM_FLAG] == 0;
-		if (want_ring && !G.on && G.rb != 640) {
+		if (want_ring && !G.on && G.rb != 512) {
 			C->put(SM_RING, {0u});
-			G = build_ring(C, c, nv, nt, o, 640);
+			G = build_ring(C, c, nv, nt, o, 512);
 			G.on = C->fetch(SM_RING, 1)[0] == 0;
 		}
 	}

@@ -319,6 +319,35 @@ def test_hc_ring_block_sizes(gpu, oracle, monkeypatch, rb, lock):
     assert 'hc_ring' in stats and 'hc_a' not in stats
 
 
+@pytest.mark.parametrize('rb,smooth,builds,form', [('', True, 2, 'hc_ring'), ('640', True, 2, 'hc_ring'),
+                                                    ('896', True, 2, 'hc_ring'), ('512', True, 1, 'hc_ring'),
+                                                    ('512', False, 1, 'hc_a'), ('896', False, 2, 'hc_a')])
+def test_hc_ring_overflow_retry(gpu, oracle, monkeypatch, rb, smooth, builds, form):
+    """Rings that overflow are built again with 512 vertices per block, the
+    size with the most room.  In marching-cubes order (few iterations) the
+    smoothed surface's rings overflow at 256, 640 and 896 vertices per block
+    (12, 9 and 25 of its blocks) but not at 512; the other's at every size."""
+    import torch
+    monkeypatch.setenv('N2M_HC_RB', rb)
+    shape, seed, noise = ((60, 64, 68), 8, 8.0) if smooth else ((30, 32, 34), 4, 12.0)
+    img = support.blobs(shape, seed, noise=noise)
+    iso = float(np.float32(np.percentile(img, 50)))
+    rc, to, po = oracle.meshify(img.copy(), iso, smooth, False, False, cubes=1)
+    assert rc == 0 and len(po) == (28202 if smooth else 28195)
+    with gpu.DeviceContext() as ctx:
+        d = torch.from_numpy(img).cuda()
+        torch.cuda.synchronize()
+        prm = ctx.params(iso, cubes=1, preSmooth=smooth, onlyLargest=False, fillBubbles=False)
+        assert ctx.meshify(d.data_ptr(), shape[::-1], prm) == 0
+        ctx.timing(True)
+        assert ctx.smooth_hc(0, 0.1, 0.5, 5, True) == 0
+        t, p = ctx.mesh(0)
+        stats = ctx.kernel_stats()
+    oracle.laplacian_smoothHC(po, to, 0.1, 0.5, 5, True)
+    assert _eq(t, to) and np.array_equal(p, po)
+    assert stats['hc_rings'][1] == builds and form in stats
+
+
 @pytest.mark.parametrize('nv', [4095, 4096, 8191, 8192, 32767, 32768, 120000, 131072, 131073, 163840, 163841])
 @pytest.mark.parametrize('iters', [2, 24])
 @pytest.mark.parametrize('shuffled', [False, True])
