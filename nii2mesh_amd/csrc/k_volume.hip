@@ -1641,7 +1641,9 @@ k_thr_range(ThrRecord *__restrict__ r, const uint32_t *__restrict__ rows, int nr
 				s_lo = 0;
 				s_hi = kBins - 1;
 			}
-			unsigned long long upto = c; // 64-bit: volumes of 2^32 voxels and more
+			// 64-bit sums; the bins and the NaN count themselves have 32 bits, so
+			// none of them may reach 2^32 voxels
+			unsigned long long upto = c;
 #pragma unroll
 			for (int d = 1; d < N2M_WAVE; d <<= 1) {
 				const unsigned long long o = __shfl_up(upto, d);
