@@ -259,7 +259,7 @@ enum Small {
 	SM_WIDE = 41,  // 1 word: a smoothed coordinate is not a float
 	SM_HALO = 44,  // 1 word: a smoothing block overflowed its halo
 	SM_RING = 45,  // 1 word: a smoothing block overflowed its two rings
-	SM_WNSEG = 48, // 1 word: weld segment count (left on the device)
+	SM_WNSEG = 48, // 1 word: weld segment count (on the host in weld(), else left on the device)
 	SM_WNNEW = 49, // 1 word: welded vertex count (left on the device)
 	SM_DEGK = 50,  // 1 word, host only: triangles kept by the degenerate test (follows SM_WNNEW)
 	SM_WORDS = 64

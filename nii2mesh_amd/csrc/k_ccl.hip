@@ -7,10 +7,10 @@
 // order and the largest-cluster tie rule (lowest label wins,
 // src/bwlabel.c:463) is "smallest root wins".
 //
-//  1. k_ccl_local: a workgroup labels the runs of a tile of 256 words (128x8x8
-//     voxels) in LDS and writes each run's tile-local root to
-//     L; it also clears AUX at every tile-local root (every global root is
-//     one of them).
+//  1. k_ccl_local: a workgroup labels the runs of a tile of CC_BS words (its
+//     shape follows the row length, see launch_ccl) in LDS and writes each
+//     run's tile-local root to L; it also clears AUX at every tile-local root
+//     (every global root is one of them).
 //  2. k_ccl_merge: tile-boundary voxels union with their backward neighbours
 //     in other tiles through global atomics.
 //  3. k_ccl_flatten: L[v] = root(v); per-root voxel counts (wave-aggregated

@@ -704,9 +704,9 @@ __device__ __forceinline__ double dist3v(double ax, double ay, double az, double
 // instead of one dependent load chain per comparison.
 constexpr int WG_REG = 8;
 
-// lrep (when given): at each seed's sorted position the largest vertex id
-// whose final class is the seed's (the member whose position the reference
-// keeps, src/meshify.c:100-101), WG_NOSEED elsewhere, so that the class
+// lrep: at each seed's sorted position the largest vertex id whose final class
+// is the seed's (the member whose position the reference keeps,
+// src/meshify.c:100-101), WG_NOSEED elsewhere, so that the class
 // representatives need no atomics.  A seed can claim a vertex an earlier
 // seed claimed; a segment where that happened takes the maxima again over
 // the final classes.
@@ -759,17 +759,15 @@ __device__ __forceinline__ void weld_segment_regs(uint32_t s, uint32_t b, uint32
 	for (int q = 0; q < WG_REG; q++)
 		if ((uint32_t)q < len) {
 			lcls[b + q] = cl[q];
-			if (lrep) {
-				uint32_t hi = WG_NOSEED;
-				if ((seedmask >> q) & 1u) { // members follow their seed
-					hi = v[q];
+			uint32_t hi = WG_NOSEED;
+			if ((seedmask >> q) & 1u) { // members follow their seed
+				hi = v[q];
 #pragma unroll
-					for (int j = q + 1; j < WG_REG; j++)
-						if ((uint32_t)j < len && cl[j] == cl[q])
-							hi = max(hi, v[j]);
-				}
-				lrep[b + q] = hi;
+				for (int j = q + 1; j < WG_REG; j++)
+					if ((uint32_t)j < len && cl[j] == cl[q])
+						hi = max(hi, v[j]);
 			}
+			lrep[b + q] = hi;
 		}
 	seeds[s] = (uint32_t)ns;
 }
@@ -783,35 +781,32 @@ __device__ __forceinline__ void weld_segment_serial(uint32_t s, uint32_t b, uint
 {
 	const float tol = 0.00001f;
 	for (uint32_t i = b; i < e; i++)
-	lcls[i] = -1;
+		lcls[i] = -1;
 	int ns = 0;
 	bool stolen = false;
 	for (uint32_t i = b; i < e; i++) {
-	if (lcls[i] >= 0) {
-		if (lrep)
+		if (lcls[i] >= 0) {
 			lrep[i] = WG_NOSEED;
-		continue;
-	}
-	const float k0 = ord2f(keys[i]);
-	const double *seed = pts + (size_t)vals[i] * 3;
-	// the seed is always in its own class: for a finite position its
-	// distance to itself is 0 < tol anyway; a NaN position matches
-	// nothing, and the reference would then leave it unassigned
-	// (old2new -1, src/meshify.c:66-79)
-	lcls[i] = ns;
-	uint32_t hi = vals[i];
-	for (uint32_t j = i + 1; j < e && (ord2f(keys[j]) - k0) < tol; j++)
-		if (dist3(seed, pts + (size_t)vals[j] * 3) < (double)tol) {
-			stolen |= lcls[j] >= 0;
-			lcls[j] = ns;
-			hi = max(hi, vals[j]);
+			continue;
 		}
-	if (lrep)
+		const float k0 = ord2f(keys[i]);
+		const double *seed = pts + (size_t)vals[i] * 3;
+		// the seed is always in its own class: for a finite position its
+		// distance to itself is 0 < tol anyway; a NaN position matches
+		// nothing, and the reference would then leave it unassigned
+		// (old2new -1, src/meshify.c:66-79)
+		lcls[i] = ns;
+		uint32_t hi = vals[i];
+		for (uint32_t j = i + 1; j < e && (ord2f(keys[j]) - k0) < tol; j++)
+			if (dist3(seed, pts + (size_t)vals[j] * 3) < (double)tol) {
+				stolen |= lcls[j] >= 0;
+				lcls[j] = ns;
+				hi = max(hi, vals[j]);
+			}
 		lrep[i] = hi;
-	ns++;
+		ns++;
 	}
-	if (lrep && stolen) // members follow their seed, within its key window
-	for (uint32_t i = b; i < e; i++) {
+	for (uint32_t i = b; stolen && i < e; i++) { // members follow their seed, within its key window
 		if (lrep[i] == WG_NOSEED)
 			continue;
 		const int c = lcls[i];
@@ -873,20 +868,14 @@ __device__ __forceinline__ void weld_segment_wave(uint32_t s, uint32_t b, uint32
 	}
 	if (in) {
 		lcls[b + j] = cl;
-		if (lrep)
-			lrep[b + j] = hi;
+		lrep[b + j] = hi;
 	}
 	if (j == 0)
 		seeds[s] = (uint32_t)ns;
 }
 
-// lrep (when given): at each seed's sorted position the largest vertex id
-// whose final class is the seed's (the member whose position the reference
-// keeps, src/meshify.c:100-101), WG_NOSEED elsewhere, so that the class
-// representatives need no atomics.  A seed can claim a vertex an earlier
-// seed claimed; a segment where that happened takes the maxima again over
-// the final classes.  One lane per segment; segments longer than WG_REG
-// (and at most a wave) are taken by the lane's whole wave in turn.
+// One lane per segment; segments longer than WG_REG (and at most a wave) are
+// taken by the lane's whole wave in turn.
 __global__ void k_weld_greedy(const uint32_t *__restrict__ starts, uint32_t nseg, uint32_t n,
                               const uint32_t *__restrict__ keys, const uint32_t *__restrict__ vals,
                               const double *__restrict__ pts, int *__restrict__ lcls, uint32_t *__restrict__ seeds,
@@ -906,8 +895,7 @@ __global__ void k_weld_greedy(const uint32_t *__restrict__ starts, uint32_t nseg
 		len = (s + 1 < nseg ? starts[s + 1] : n) - b;
 		if (len == 1) { // a vertex alone in its key window is its own class
 			lcls[b] = 0;
-			if (lrep)
-				lrep[b] = vals[b];
+			lrep[b] = vals[b];
 			seeds[s] = 1u;
 		} else if (len <= (uint32_t)WG_REG)
 			weld_segment_regs(s, b, len, keys, vals, pts, lcls, seeds, lrep);
@@ -925,8 +913,7 @@ __global__ void k_weld_greedy(const uint32_t *__restrict__ starts, uint32_t nseg
 // vertex was merged and, as the reference then keeps its input unchanged
 // (src/meshify.c:82-87), every vertex keeps its own number
 // The representative of each class (the last member in index order provides
-// the position): from lrep at the seeds when given, else by atomics on a rep
-// array the caller filled with -1.
+// the position) comes from lrep at the seeds.
 __global__ void k_weld_assign(const uint32_t *__restrict__ vals, const int *__restrict__ lcls,
                               const uint32_t *__restrict__ seg,
                               const uint32_t *__restrict__ seedbase, uint32_t n, int *__restrict__ cls,
@@ -940,9 +927,7 @@ __global__ void k_weld_assign(const uint32_t *__restrict__ vals, const int *__re
 	const bool ident = d_nnew && *d_nnew == n;
 	const int c = ident ? (int)v : (int)seedbase[seg[i]] + lcls[i];
 	cls[v] = c;
-	if (!lrep)
-		atomicMax(&rep[c], (int)v);
-	else if (ident)
+	if (ident)
 		rep[c] = (int)v;
 	else if (lrep[i] != WG_NOSEED)
 		rep[c] = (int)lrep[i];
@@ -2016,12 +2001,6 @@ k_ring_build(const uint32_t *__restrict__ start, const int2 *__restrict__ pairs,
 		rs[HE * S1 + poff + (k - HE)] = slot(pairs[hb + k]);
 }
 
-// The originals o and o1 of the iteration are doubles, or, when every coordinate
-// is a float (F32, see k_hc_load), floats.  Marching cubes computes Lewiner
-// vertices in floats, so their meshes take the second form as long as no
-// transform came between: 17 of some 153 bytes per vertex less for an
-// iteration that runs at the rate of a copy (9.6 M vertices:
-// 322 -> 311 us).
 // A vertex's list in the two-ring form: its first HK pairs, its degree | first
 // pair beyond HE << 16.
 struct EllRefs {
@@ -2060,6 +2039,11 @@ __device__ __forceinline__ d3 laplace_ell(const EllRefs &r, const lds_double *L,
 
 // one HC iteration (hc_a then hc_b) in two-ring form; pout != p.  LDS rows
 // in split form (an (x, y) array and a z array, read as 16 + 8 bytes).
+// The originals o and o1 are doubles, or, when every coordinate is a float
+// (F32, see k_hc_load), floats.  Marching cubes computes Lewiner vertices in
+// floats, so their meshes take the second form as long as no transform came
+// between: 17 of some 153 bytes per vertex less for an iteration that runs at
+// the rate of a copy (9.6 M vertices: 322 -> 311 us).
 template <int RB, bool F32>
 __global__ void __launch_bounds__(RingCfg<RB>::T, RingCfg<RB>::LARGE ? 8 : 4)
 k_hc_ring(const uint32_t *__restrict__ deg, const uint32_t *__restrict__ ell, const uint32_t *__restrict__ rdeg,
@@ -2629,7 +2613,9 @@ struct RingDims {
 static RingDims ring_dims(int rb)
 {
 	switch (rb) {
-#define X(n)                                                                                                       	case n:                                                                                                        		return {(size_t)RingCfg<n>::CAP, (size_t)RingCfg<n>::PCAP, (size_t)RingCfg<n>::R1CAP};
+#define X(n)                                                                                                      \
+	case n:                                                                                                      \
+		return {(size_t)RingCfg<n>::CAP, (size_t)RingCfg<n>::PCAP, (size_t)RingCfg<n>::R1CAP};
 		N2M_RING_RBS(X)
 #undef X
 	}

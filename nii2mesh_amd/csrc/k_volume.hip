@@ -999,7 +999,7 @@ struct ApplyVoxel {
 
 // the sign bits of 4 voxels of the Lewiner data lw_clamp(v - iso), whose 8
 // lanes (lane & 7 = part) together hold a word; lane 0 of them writes it
-__device__ __forceinline__ void apply_signs(const float (&vv)[4], int nlive, float iso, int part, size_t word, bool write,
+__device__ __forceinline__ void apply_signs(const float (&vv)[4], int nlive, float iso, int part, size_t word,
                                             uint32_t *__restrict__ sgp, uint32_t *__restrict__ sgn)
 {
 	uint32_t bp = 0, bn = 0;
@@ -1017,7 +1017,7 @@ __device__ __forceinline__ void apply_signs(const float (&vv)[4], int nlive, flo
 		bp |= __shfl_xor(bp, m);
 		bn |= __shfl_xor(bn, m);
 	}
-	if (write && part == 0) {
+	if (part == 0) {
 		sgp[word] = bp;
 		sgn[word] = bn;
 	}
@@ -1067,7 +1067,7 @@ k_apply(const float *src, float *img, int nx, int ny, int nz, int W, int vec4, f
 				// row (nx % 32 == 0 and the span a multiple of 8, so the group
 				// shares its row and its trip count)
 				if (sgp)
-					apply_signs(vv, 4, iso, q & 7, (size_t)W * row + (x >> 5), true, sgp, sgn);
+					apply_signs(vv, 4, iso, q & 7, (size_t)W * row + (x >> 5), sgp, sgn);
 			}
 		}
 	} else {
@@ -1148,7 +1148,7 @@ k_apply_linear(const float *src, float *img, int nx, int ny, int nz, uint32_t nv
 			for (int u = 0; u < nlive; u++)
 				img[v0 + u] = vv[u];
 		if (sgp)
-			apply_signs(vv, nlive, iso, q & 7, q >> 3, true, sgp, sgn);
+			apply_signs(vv, nlive, iso, q & 7, q >> 3, sgp, sgn);
 	}
 	voxel.store(part);
 }
